@@ -176,6 +176,28 @@ bool k_ok(int K, int gs) {
   return nb <= QMV_IT * lanes_for_blocks(nb);
 }
 
+// Workspace of a batch GEMM's activations in limb form (none at MAX_TOKENS tokens or fewer).
+size_t xl_ws(int M, int K) { return M > MAX_TOKENS ? al(xl_bytes(M, K)) : 0; }
+
+XlBatch xl_take(Ctx* c, int M, int K) { return xl_carve(ws_take<char>(c, xl_bytes(M, K)), M, K); }
+
+// y [M, N] = x [M, K] . W^T: the batch GEMM on x where it takes the matrix, else the GEMV paths on the
+// prepared blocks xp.  Workspace: xl_ws(M, K), free again on return.
+int dense_enqueue(Ctx* c, const char* name, const mtpx_q4& w, int N, int K, int gs, const uint16_t* x,
+                  const uint32_t* xp, int M, uint16_t* y, float* yf = nullptr) {
+  if (gemm_ok(w.w, w.s, w.b, N, K, gs, M)) {
+    const size_t mark = c->ws_used;
+    const XlBatch xl = xl_take(c, M, K);
+    LAUNCH(c, "xlimb", launch_xlimb(x, M, K, xl, c->stream));
+    LAUNCH(c, name, launch_gemm_pair(w.w, w.s, w.b, N, y, yf, nullptr, nullptr, nullptr, 0, nullptr, K, gs, xl, M,
+                                     c->stream));
+    c->ws_used = mark;
+    return MTPX_OK;
+  }
+  LAUNCH(c, name, launch_qmv(w.w, w.s, w.b, w.sb, N, K, gs, xp, M, y, yf, c->stream));
+  return MTPX_OK;
+}
+
 struct Kv {
   Ctx* ctx;
   int heads, dim;
@@ -215,7 +237,7 @@ size_t moe_ws_bytes(const mtpx_moe_weights* w, int M, int nwin = 1) {
   return al(4 * T * E) + al(4 * T) + al(4 * T * K) * 2 + al(sizeof(MoeDispatch) * (size_t)nwin) +
          al(4 * T * (H / 32) * XP_DW) + al(2 * slots * F) + al(2 * slots * H) +
          (nwin > 1 ? al(4 * slots) + al(8 * (size_t)moe_max_chunks((int)T, E, K)) + al(4) +
-                         al(4 * slots * (F / 32) * XP_DW)
+                         al(xl_bytes((int)T, H)) + al(xl_bytes((int)slots, F))
                    : 0) +
          4096;
 }
@@ -282,12 +304,20 @@ int moe_enqueue(Ctx* c, const mtpx_moe_weights* w, const uint16_t* x, int M, uin
       a.chunks = ws_take<int32_t>(c, 2 * (size_t)moe_max_chunks((int)T, a.E, a.K));
       a.chunk_n = ws_take<int32_t>(c, 1);
       a.max_chunks = moe_max_chunks((int)T, a.E, a.K);
-      a.xp_act = ws_take<uint32_t>(c, slots * (a.F / 32) * XP_DW);
       LAUNCH(c, "moe_sort", launch_moe_sort(a, c->stream));
-      if (moe_qmm_supported(a)) {  // down over the experts' chunks on the matrix cores
-        LAUNCH(c, "moe_gate_up", launch_moe_gate_up_dd(a, c->stream));
-        LAUNCH(c, "moe_act_prep", launch_xprep(reinterpret_cast<const bf16*>(a.act), (int)slots, a.F, a.xp_act, c->stream));
-        LAUNCH(c, "moe_down", launch_moe_qmm_down(a, c->stream));
+      if (moe_gemm_ok(a)) {  // the experts over their chunks on the matrix cores
+        // gate|up: a chunk costs 16 tokens whatever it holds, so below about 2.7 slots per expert the walk of
+        // one slot per workgroup is faster (whole prefill of four layers, 128 / 160 tokens of 512 experts
+        // top-10: 3515 / 3804 us by chunks, 3487 / 3959 by slots; 75 tokens: 2900 / 2650; 512: 7000 / 9700)
+        const XlBatch xt = xl_take(c, (int)T, a.H), xs = xl_take(c, (int)slots, a.F);
+        if (T * a.K * 3 >= (size_t)a.E * 8) {
+          LAUNCH(c, "xlimb", launch_xlimb(a.x, (int)T, a.H, xt, c->stream));
+          LAUNCH(c, "moe_gate_up", launch_moe_gemm_gate_up(a, xt, c->stream));
+        } else {
+          LAUNCH(c, "moe_gate_up", launch_moe_gate_up_dd(a, c->stream));
+        }
+        LAUNCH(c, "xlimb", launch_xlimb(a.act, (int)slots, a.F, xs, c->stream));
+        LAUNCH(c, "moe_down", launch_moe_gemm_down(a, xs, c->stream));
         LAUNCH(c, "moe_combine", launch_moe_combine(a, c->stream));
         return MTPX_OK;
       }
@@ -498,11 +528,11 @@ int layer_create(Ctx* c, const mtpx_layer_config* cfg, uint64_t seed, Layer** ou
   return MTPX_OK;
 }
 
-// Attention sublayer for M tokens whose prepared input blocks are in xp:
+// Attention sublayer for M tokens x whose prepared input blocks are in xp:
 // qkv GEMV, q/k norm + RoPE + KV append, verify attention with the output gate,
 // o_proj GEMV -> o [M, H].  xp is reused for the gated attention output, so it
 // holds max(H, HQ*D)/32 blocks per token.  Workspace already reserved.
-int attn_enqueue(Ctx* c, const Layer* L, Kv* kv, uint32_t* xp, int M, uint16_t* o) {
+int attn_enqueue(Ctx* c, const Layer* L, Kv* kv, const uint16_t* x, uint32_t* xp, int M, uint16_t* o) {
   const mtpx_layer_config& g = L->cfg;
   const int H = g.hidden, HQ = g.heads, HK = g.kv_heads, D = g.head_dim, QW = L->QW, gs = g.group_size;
   const int T = (int)(kv->offset + M);
@@ -511,7 +541,8 @@ int attn_enqueue(Ctx* c, const Layer* L, Kv* kv, uint32_t* xp, int M, uint16_t* 
   uint16_t* att = ws_take<uint16_t>(c, (size_t)M * HQ * D);
   float* part = ws_take<float>(c, attn_partial_floats(M, HQ, D, T));
   hipStream_t st = c->stream;
-  LAUNCH(c, "qmv_qkv", launch_qmv(L->w.qkv_w, L->w.qkv_s, L->w.qkv_b, L->w.qkv_sb, QW, H, gs, xp, M, qkv, nullptr, st));
+  int rc = dense_enqueue(c, "qmv_qkv", {L->w.qkv_w, L->w.qkv_s, L->w.qkv_b, L->w.qkv_sb}, QW, H, gs, x, xp, M, qkv);
+  if (rc) return rc;
   if (attn_prep_fused_ok(M, HQ, HK, D, QW)) {  // a verify window: the prep inside the partial launch
     LAUNCH(c, "attn_partial", launch_attn_partial_prep(qkv, QW, M, HQ, HK, D, g.rot_dims, L->w.q_norm, L->w.k_norm,
                                                        g.eps, L->w.rope_cos, L->w.rope_sin, kv->k, kv->v, kv->tmax, T,
@@ -524,14 +555,14 @@ int attn_enqueue(Ctx* c, const Layer* L, Kv* kv, uint32_t* xp, int M, uint16_t* 
                                                   1.0f / std::sqrt((float)D), part, st));
   }
   LAUNCH(c, "attn_combine", launch_attn_combine(M, HQ, HK, D, T, part, qkv, QW, HQ * D, nullptr, att, xp, st));
-  LAUNCH(c, "qmv_o", launch_qmv(L->w.o_w, L->w.o_s, L->w.o_b, L->w.o_sb, H, HQ * D, gs, xp, M, o, nullptr, st));
-  return MTPX_OK;
+  return dense_enqueue(c, "qmv_o", {L->w.o_w, L->w.o_s, L->w.o_b, L->w.o_sb}, H, HQ * D, gs, att, xp, M, o);
 }
 
 size_t attn_ws_bytes(const Layer* L, int M, int T) {
   const mtpx_layer_config& g = L->cfg;
   const int HQ = g.heads, D = g.head_dim;
-  return al(2 * (size_t)M * L->QW) + al(2 * (size_t)M * HQ * D) * 2 + al(4 * attn_partial_floats(M, HQ, D, T));
+  return al(2 * (size_t)M * L->QW) + al(2 * (size_t)M * HQ * D) * 2 + al(4 * attn_partial_floats(M, HQ, D, T)) +
+         xl_ws(M, g.hidden > HQ * D ? g.hidden : HQ * D);
 }
 
 // ---------------------------------------------------------------------------
@@ -576,12 +607,12 @@ size_t head_ws_bytes(const Head* hd, int S, int T) {
   const int XB = (H > HQ * D ? H : HQ * D) / 32;
   // per mixer call (three per step): lo, act [S, LW]; inj [S, hc]; xpL; w [S, W]
   const size_t mix = al(2 * (size_t)S * LW) * 2 + al(2 * (size_t)S * g.hc) + al(4 * (size_t)S * (LW / 32) * XP_DW) +
-                     al(2 * (size_t)S * W) + (S > MAX_TOKENS ? al(4 * (size_t)S * (W / 32) * XMB_DW) : 0);
+                     al(2 * (size_t)S * W) + xl_ws(S, W);
   const size_t moe = S > MAX_TOKENS ? moe_windows_ws_bytes(&hd->w.layer.moe, S) : moe_ws_bytes(&hd->w.layer.moe, S);
   return moe + attn_ws_bytes(hd->layer, S, T) + 3 * mix + al(2 * (size_t)S * H) * 6 +
          al(2 * (size_t)S * W) * 5 + al(2 * (size_t)S * g.hc) + al(4 * (size_t)S * XB * XP_DW) +
          al(4 * (size_t)S * (W / 32) * XP_DW) + al(2 * (size_t)hd->w.shortlist_rows) +
-         al(4 * argmax_work_items(1, hd->w.shortlist_rows)) * 2 + 8192;
+         al(4 * argmax_work_items(1, hd->w.shortlist_rows)) * 2 + xl_ws(S * g.hc, H) + 8192;
 }
 
 // One hyper-connection mixer over the normed rows (prepared blocks in xpW):
@@ -619,17 +650,23 @@ int hc_mix_enqueue(Ctx* c, const HcGeom& g, const mtpx_hc_weights* hw, const uin
   uint16_t* inj = ws_take<uint16_t>(c, (size_t)S * g.hc);
   uint32_t* xpL = ws_take<uint32_t>(c, (size_t)S * (LW / 32) * XP_DW);
   uint16_t* wm = ws_take<uint16_t>(c, (size_t)S * W);
-  if (qmv_pair_ok(hw->down.sb, hw->inject.w, hw->inject.sb, W, S)) {  // a batch: down and inject rows in one launch
-    uint32_t* xmb = ws_take<uint32_t>(c, (size_t)S * (W / 32) * XMB_DW);
-    LAUNCH(c, "hc_down_inject", launch_qmv_pair(hw->down.w, hw->down.sb, LW, reinterpret_cast<bf16*>(lo), hw->inject.w,
-                                                hw->inject.sb, g.hc, reinterpret_cast<bf16*>(inj), W, gs, xpW, xmb, S, st));
+  const bool inj_on = hw->inject.w != nullptr;
+  int rc;
+  if (gemm_ok(hw->down.w, hw->down.s, hw->down.b, LW, W, gs, S) &&
+      (!inj_on || gemm_ok(hw->inject.w, hw->inject.s, hw->inject.b, g.hc, W, gs, S))) {  // a batch: both in one launch
+    const size_t mark = c->ws_used;
+    const XlBatch xl = xl_take(c, S, W);
+    LAUNCH(c, "xlimb", launch_xlimb(reinterpret_cast<const bf16*>(normed), S, W, xl, st));
+    LAUNCH(c, "hc_down_inject",
+           launch_gemm_pair(hw->down.w, hw->down.s, hw->down.b, LW, reinterpret_cast<bf16*>(lo), nullptr, hw->inject.w,
+                            hw->inject.s, hw->inject.b, inj_on ? g.hc : 0, reinterpret_cast<bf16*>(inj), W, gs, xl, S, st));
+    c->ws_used = mark;
   } else {
-    LAUNCH(c, "hc_down", launch_qmv(hw->down.w, hw->down.s, hw->down.b, hw->down.sb, LW, W, gs, xpW, S, lo, nullptr, st));
-    if (hw->inject.w)
-      LAUNCH(c, "hc_inject", launch_qmv(hw->inject.w, hw->inject.s, hw->inject.b, hw->inject.sb, g.hc, W, gs, xpW, S, inj, nullptr, st));
+    if ((rc = dense_enqueue(c, "hc_down", hw->down, LW, W, gs, normed, xpW, S, lo))) return rc;
+    if (inj_on && (rc = dense_enqueue(c, "hc_inject", hw->inject, g.hc, W, gs, normed, xpW, S, inj))) return rc;
   }
   LAUNCH(c, "hc_silu", launch_silu_xprep(lo, S, LW, act, xpL, st));
-  LAUNCH(c, "hc_up", launch_qmv(hw->up.w, hw->up.s, hw->up.b, hw->up.sb, W, LW, gs, xpL, S, wm, nullptr, st));
+  if ((rc = dense_enqueue(c, "hc_up", hw->up, W, LW, gs, act, xpL, S, wm))) return rc;
   LAUNCH(c, "hc_mix", launch_hc_mix(wm, normed, hw->inject.w ? inj : nullptr, S, g.hc, H, x, j, xpH, st));
   return MTPX_OK;
 }
@@ -1521,13 +1558,16 @@ int mtpx_qmv(mtpx_ctx h, const uint32_t* wq, const uint16_t* s, const uint16_t* 
   ARG(gs_ok(gs) && k_ok(K, gs), "K=%d gs=%d unsupported", K, gs);
   if (set_device(c)) return MTPX_ERR_HIP;
   const size_t xpn = (size_t)M * (K / 32) * XP_DW;
-  int rc = ws_reserve(c, al(xpn * 4) + 256);
+  const bool batch = gemm_ok(wq, s, b, N, K, gs, M);
+  int rc = ws_reserve(c, (batch ? xl_ws(M, K) : al(xpn * 4)) + 256);
   if (rc) return rc;
   ws_begin(c);
-  uint32_t* xp = ws_take<uint32_t>(c, xpn);
-  LAUNCH(c, "xprep", launch_xprep(x, M, K, xp, c->stream));
-  LAUNCH(c, "qmv", launch_qmv(wq, s, b, sb, N, K, gs, xp, M, y, yf, c->stream));
-  return MTPX_OK;
+  uint32_t* xp = nullptr;
+  if (!batch) {
+    xp = ws_take<uint32_t>(c, xpn);
+    LAUNCH(c, "xprep", launch_xprep(x, M, K, xp, c->stream));
+  }
+  return dense_enqueue(c, "qmv", {wq, s, b, sb}, N, K, gs, x, xp, M, y, yf);
 }
 
 int mtpx_moe_forward(mtpx_ctx h, const mtpx_moe_weights* w, const uint16_t* x, int M, uint16_t* y, int32_t* idx,
@@ -1866,7 +1906,7 @@ int mtpx_layer_forward(mtpx_ctx h, mtpx_layer lh, mtpx_kv kvh, const uint16_t* x
   uint32_t* xp2 = ws_take<uint32_t>(c, (size_t)M * (H / 32) * XP_DW);
   hipStream_t st = c->stream;
   LAUNCH(c, "rmsnorm", launch_rmsnorm(x, nullptr, M, H, L->w.attn_norm, g.eps, nullptr, h1, xp, st));
-  if ((rc = attn_enqueue(c, L, kv, xp, M, o))) return rc;
+  if ((rc = attn_enqueue(c, L, kv, h1, xp, M, o))) return rc;
   LAUNCH(c, "rmsnorm", launch_rmsnorm(x, o, M, H, L->w.post_norm, g.eps, s, h2, xp2, st));
   if ((rc = moe_enqueue(c, &L->w.moe, h2, M, h1, nullptr, nullptr, nullptr, s, y, xp2))) return rc;
   kv->offset += M;
@@ -2677,7 +2717,7 @@ int target_verify_enqueue(Ctx* c, Target* t, TargetState* s, const int32_t* ids,
   const int T = (int)s->offset + S;
   const size_t mix = al(2 * (size_t)S * g.lowrank) * 2 + al(2 * (size_t)S * hc) +
                      al(4 * (size_t)S * (g.lowrank / 32) * XP_DW) + al(2 * (size_t)S * W) +
-                     (S > MAX_TOKENS ? al(4 * (size_t)S * (W / 32) * XMB_DW) : 0);
+                     xl_ws(S, W);
   const Layer* any_attn = nullptr;
   for (const TargetLayer& L : t->layers)
     if (L.attn) any_attn = L.attn;
@@ -2691,7 +2731,8 @@ int target_verify_enqueue(Ctx* c, Target* t, TargetState* s, const int32_t* ids,
                                     t->ple ? ple_ws_bytes(t->ple->cfg, SW) + al(2 * (size_t)S * W) : 0) + 4096;
   const size_t fixed = al(2 * (size_t)S * H) * 5 + al(2 * (size_t)S * W) * 4 + al(2 * (size_t)S * hc) * 2 +
                        al(4 * (size_t)S * (W / 32) * XP_DW) + al(4 * (size_t)S * XB * XP_DW) +
-                       al(4 * (size_t)S * (VD / 32) * XP_DW) + al(2 * (size_t)S * gg.pw) + 4096;
+                       al(4 * (size_t)S * (VD / 32) * XP_DW) + al(2 * (size_t)S * gg.pw) +
+                       (prefill ? al(2 * (size_t)S * VD) : 0) + xl_ws(S, std::max(H, VD)) + 4096;
   int rc = ws_reserve(c, fixed + per_layer);
   if (rc) return rc;
   ws_begin(c);
@@ -2710,6 +2751,7 @@ int target_verify_enqueue(Ctx* c, Target* t, TargetState* s, const int32_t* ids,
   uint32_t* xpH = ws_take<uint32_t>(c, (size_t)S * XB * XP_DW);
   uint32_t* xpG = ws_take<uint32_t>(c, (size_t)S * (VD / 32) * XP_DW);
   uint16_t* proj = ws_take<uint16_t>(c, (size_t)S * gg.pw);
+  uint16_t* gated = prefill ? ws_take<uint16_t>(c, (size_t)S * VD) : nullptr;
   const size_t mark = c->ws_used;
   hipStream_t st = c->stream;
   *launched = true;
@@ -2743,17 +2785,17 @@ int target_verify_enqueue(Ctx* c, Target* t, TargetState* s, const int32_t* ids,
     if (L.kind == MTPX_LAYER_GDN) {
       const mtpx_q4& ip = L.gdn->w.in_proj;
       const mtpx_q4& op = L.gdn->w.out_proj;
-      LAUNCH(c, "qmv_gdn_in", launch_qmv(ip.w, ip.s, ip.b, ip.sb, gg.pw, H, gs, xpH, S, proj, nullptr, st));
+      if ((rc = dense_enqueue(c, "qmv_gdn_in", ip, gg.pw, H, gs, x, xpH, S, proj))) return rc;
       if (prefill) {  // the batch in one launch, committed
         const size_t mark3 = c->ws_used;
-        if ((rc = gdn_enqueue_batch(c, L.gdn, s->gdn[i], proj, S, nullptr, xpG))) return rc;
+        if ((rc = gdn_enqueue_batch(c, L.gdn, s->gdn[i], proj, S, gated, xpG))) return rc;
         c->ws_used = mark3;
       } else if ((rc = gdn_enqueue(c, L.gdn, s->gdn[i], proj, S, nullptr, xpG))) {
         return rc;
       }
-      LAUNCH(c, "qmv_gdn_out", launch_qmv(op.w, op.s, op.b, op.sb, H, VD, gs, xpG, S, ao, nullptr, st));
+      if ((rc = dense_enqueue(c, "qmv_gdn_out", op, H, VD, gs, gated, xpG, S, ao))) return rc;
     } else {
-      if ((rc = attn_enqueue(c, L.attn, s->kv[i], xpH, S, ao))) return rc;
+      if ((rc = attn_enqueue(c, L.attn, s->kv[i], x, xpH, S, ao))) return rc;
     }
     LAUNCH(c, "hc_norm", launch_hc_norm(sA, ao, jA, S, hc, H, 0, L.mlp_hc.norm_scale, eps, sM, nrm, xpW, st));
     c->ws_used = mark;
@@ -2984,16 +3026,14 @@ int mtpx_head_forward(mtpx_ctx h, mtpx_head hh, mtpx_kv kvh, const int32_t* ids,
   LAUNCH(c, "embed", launch_embed_rows(w.embed.w, w.embed.s, w.embed.b, H, gs, g.vocab, ids, S, e, st));
   LAUNCH(c, "hc_norm", launch_hc_norm(e, nullptr, nullptr, S, 1, H, 0, w.pre_norm_embedding, eps, nullptr, en, xpH,
                                       st));
-  LAUNCH(c, "qmv_fc", launch_qmv(w.fc_embedding.w, w.fc_embedding.s, w.fc_embedding.b, w.fc_embedding.sb, H, H, gs, xpH, S, emb,
-                                 nullptr, st));
+  if ((rc = dense_enqueue(c, "qmv_fc", w.fc_embedding, H, H, gs, en, xpH, S, emb))) return rc;
   LAUNCH(c, "hc_norm", launch_hc_norm(multi, nullptr, nullptr, S, 1, W, 0, w.pre_norm_hidden, eps, nullptr, mn, xpW,
                                       st));
-  LAUNCH(c, "qmv_fc", launch_qmv(w.fc_hidden.w, w.fc_hidden.s, w.fc_hidden.b, w.fc_hidden.sb, H, H, gs, xpW, S * hc, hs, nullptr,
-                                 st));
+  if ((rc = dense_enqueue(c, "qmv_fc", w.fc_hidden, H, H, gs, mn, xpW, S * hc, hs))) return rc;
   // attention block: hyper = e + h; (st0, n) = hc_norm(hyper); (x, j) = mix(attn_hc, n); ao = attn(x)
   LAUNCH(c, "hc_norm", launch_hc_norm(hs, emb, nullptr, S, hc, H, 0, w.attn_hc.norm_scale, eps, st0, nrm, xpW, st));
   if ((rc = hc_mix_enqueue(c, hd, &w.attn_hc, nrm, xpW, S, x, j, xpH))) return rc;
-  if ((rc = attn_enqueue(c, hd->layer, kv, xpH, S, ao))) return rc;
+  if ((rc = attn_enqueue(c, hd->layer, kv, x, xpH, S, ao))) return rc;
   // MoE block
   LAUNCH(c, "hc_norm", launch_hc_norm(st0, ao, j, S, hc, H, 0, w.mlp_hc.norm_scale, eps, st1, nrm, xpW, st));
   if ((rc = hc_mix_enqueue(c, hd, &w.mlp_hc, nrm, xpW, S, x, j, xpH))) return rc;

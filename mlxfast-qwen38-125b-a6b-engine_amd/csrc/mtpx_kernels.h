@@ -67,14 +67,6 @@ __device__ __forceinline__ bool ticket_last(uint32_t* ctr, uint32_t last) {
 // --- dense q4 GEMV and friends (qmv.hip)
 hipError_t launch_xprep(const bf16* x, int M, int K, uint32_t* xp, hipStream_t st);
 // sb: packed scale/bias rows (sb_row_len(K, gs) u32 per row) or null
-// Two few-row matrices (N1, N2 rows; w2 may be null) over one batch of M > MAX_TOKENS prepared
-// tokens, through xmb [M][K/32][XMB_DW] (workspace), where qmv_pair_ok holds (else launch_qmv per
-// matrix).
-constexpr int XMB_DW = 36;
-bool qmv_pair_ok(const uint32_t* sb1, const uint32_t* w2, const uint32_t* sb2, int K, int M);
-hipError_t launch_qmv_pair(const uint32_t* w1, const uint32_t* sb1, int N1, bf16* y1, const uint32_t* w2,
-                           const uint32_t* sb2, int N2, bf16* y2, int K, int gs, const uint32_t* xp, uint32_t* xmb,
-                           int M, hipStream_t st);
 hipError_t launch_qmv(const uint32_t* wq, const bf16* s, const bf16* b, const uint32_t* sb, int N, int K, int gs,
                       const uint32_t* xp, int M, bf16* y, float* yf, hipStream_t st);
 hipError_t launch_pack_sb(const bf16* s, const bf16* b, int64_t N, int K, int gs, uint32_t* out, hipStream_t st);
@@ -150,18 +142,33 @@ struct MoeArgs {
   int32_t* gorder = nullptr;
   // with gorder: the order cut into chunks of at most MQ_CHUNK slots of one expert (k_moe_sort):
   // chunks[c] = (gorder position, count | (expert + 1) << 16, 0 the shared expert), *chunk_n of
-  // them, at most max_chunks; xp_act [slots][F/32][XP_DW]: the gate|up rows prepared for down
+  // them, at most max_chunks
   int32_t* chunks = nullptr;
   int32_t* chunk_n = nullptr;
   int max_chunks = 0;
-  uint32_t* xp_act = nullptr;
 };
-constexpr int MQ_CHUNK = 8;
+constexpr int MQ_CHUNK = 16;  // slots of one expert per chunk of a batch: a token tile of the chunk GEMMs
 inline int moe_max_chunks(int T, int E, int K) {
   return (T + MQ_CHUNK - 1) / MQ_CHUNK + E + (T * K + MQ_CHUNK - 1) / MQ_CHUNK;
 }
-bool moe_qmm_supported(const MoeArgs& a);
-hipError_t launch_moe_qmm_down(const MoeArgs& a, hipStream_t st);
+// --- batch GEMMs (gemm.hip): more than MAX_TOKENS tokens of the model's depths
+// A batch in limb form (k_xlimb): xl [M][K/32][3][32] bf16, sx and xr [M][K/32], big per token and part of K.
+struct XlBatch {
+  uint4* xl;
+  float *sx, *xr;
+  uint32_t* big;
+};
+size_t xl_bytes(int M, int K);                // workspace of one batch
+XlBatch xl_carve(void* ws, int M, int K);     // its arrays in that workspace (256-byte aligned)
+hipError_t launch_xlimb(const bf16* x, int M, int K, const XlBatch& b, hipStream_t st);
+bool gemm_ok(const uint32_t* w, const bf16* s, const bf16* b, int64_t N, int K, int gs, int M);
+// y1 [M, N1] (and y2 [M, N2] where w2 is set) from x; every matrix passes gemm_ok
+hipError_t launch_gemm_pair(const uint32_t* w1, const bf16* s1, const bf16* b1, int N1, bf16* y1, float* yf1,
+                            const uint32_t* w2, const bf16* s2, const bf16* b2, int N2, bf16* y2, int K, int gs,
+                            const XlBatch& x, int M, hipStream_t st);
+bool moe_gemm_ok(const MoeArgs& a);
+hipError_t launch_moe_gemm_gate_up(const MoeArgs& m, const XlBatch& x, hipStream_t st);  // x per token
+hipError_t launch_moe_gemm_down(const MoeArgs& m, const XlBatch& x, hipStream_t st);     // x per slot
 
 constexpr int MOE_TICKETS = 64;
 constexpr int MAX_EXPERTS = 1024;

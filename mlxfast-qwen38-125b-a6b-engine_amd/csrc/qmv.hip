@@ -107,7 +107,6 @@ __global__ __launch_bounds__(64 * NWV) void k_qmv(const uint32_t* __restrict__ w
 // block; the next four blocks' loads are in flight while these are computed.
 constexpr int MMA_TOK = 4;   // tokens per tile (4 tokens x 4 limbs = 16 A rows)
 constexpr int MB_DW = 36;    // LDS block: [limb][word g][even, odd] (32 dwords), p, SX, pad
-static_assert(MB_DW == XMB_DW, "the four-limb block in memory");
 constexpr int MMA_THREADS = 512;
 
 typedef int v4i_t __attribute__((ext_vector_type(4)));
@@ -580,348 +579,6 @@ __global__ __launch_bounds__(QMM_THREADS) void k_qmm(const uint32_t* __restrict_
   }
 }
 
-// ---------------------------------------------------------------------------
-// The MoE down projection of a prefill batch on the matrix cores (same bits as the slot-per-
-// workgroup kernel): the batch's slots sorted by expert are cut into chunks of at most MQ_CHUNK
-// slots of one expert (k_moe_sort), and a workgroup owns one chunk and 128 rows of H of the expert's
-// down matrix, against the slots' prepared activation rows, into the slots' output rows.  The K
-// walk is k_qmm's: chains in the butterfly's bit-reversed leaf order, groups of four folded by a
-// binary counter, each weight operand serving every token group of the chunk that holds a slot.  A phase is one group of four chains: all IT blocks of each for
-// the chunk's tokens are staged in LDS (double buffered, the next phase's activation words loaded
-// during this one), and the weight rows stream one phase ahead (a ring of IT register buffers: an
-// expert's rows are read once per chunk, so the walk waits on HBM unless many loads are in flight).
-template <int L, int IT>
-__global__ __launch_bounds__(QMM_THREADS) void k_moe_qmm(MoeArgs a, int tiles) {
-  constexpr int QT = MQ_CHUNK / MMA_TOK, QTOK = MQ_CHUNK, NB = L * IT;
-  constexpr int LOGL = ilog2(L), LOGQ = LOGL - 2, NPH = L / 4, NBP = 4 * IT;
-  constexpr int TR = 128;                                  // rows of the tile
-  constexpr int PDW = QTOK * NBP * MB_DW;                   // one phase's staging buffer
-  constexpr int NU = (QTOK * NBP * 8 + QMM_THREADS - 1) / QMM_THREADS;  // staging units per thread
-  static_assert(L >= 4 && (1 << LOGL) == L, "groups of four chains");
-  extern __shared__ uint32_t lds[];  // [NPH > 1 ? 2 : 1][QTOK][NBP][MB_DW]
-  __shared__ int slot_l[QTOK];
-  const int ck = (int)blockIdx.x / tiles, tile = (int)blockIdx.x - ck * tiles;
-  if (ck >= *a.chunk_n) return;  // whole workgroup, before any barrier
-  const int2 cv = reinterpret_cast<const int2*>(a.chunks)[ck];
-  const int cnt = min(cv.y & 0xffff, QTOK), ev = cv.y >> 16;  // ev: expert + 1, 0 the shared expert
-  const bool shared = ev == 0;
-  const int e = shared ? 0 : min(ev - 1, a.E - 1);
-  const int H = a.H, F = a.F, gs = a.gs;
-  const int slots = a.nwin * a.M * (a.K + 1);
-  const int K = F, N = H;
-  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
-  const int n = lane & 15, g = lane >> 4;
-  const int row = tile * TR + wave * 16 + n, rc = row < N ? row : N - 1;
-  const int rs = gs == 32 ? 0 : gs == 64 ? 1 : 2;
-  const int P = sb_row_len(K, gs);
-  const size_t rbase = shared ? 0 : (size_t)e * N;
-  const uint32_t* wm = shared ? a.sh_down_w : a.down_w;
-  const uint32_t* sm = shared ? a.sh_down_sb : a.down_sb;
-  const uint32_t* wrow = wm + (rbase + rc) * (size_t)(K / 8);
-  const uint32_t* srow = sm + (rbase + rc) * (size_t)P;
-  auto chain = [](int i) { return (int)(__builtin_bitreverse32((uint32_t)i) >> (32 - LOGL)); };
-  uint4 wr[IT];
-  uint32_t pr[IT][4];
-  auto load_w = [&](int q, int it, uint4& w, uint32_t (&p)[4]) {  // any q: the blocks stay inside the matrix
-    w = *reinterpret_cast<const uint4*>(wrow + (size_t)(chain(4 * q + g) + L * it) * 4);  // cached: an expert's chunks
-#pragma unroll
-    for (int b = 0; b < 4; ++b) p[b] = srow[(chain(4 * q + b) >> rs) * IT + it];
-  };
-#pragma unroll
-  for (int it = 0; it < IT; ++it) load_w(0, it, wr[it], pr[it]);  // the weights first: they come from HBM
-  if (threadIdx.x < QTOK)
-    slot_l[threadIdx.x] = (int)threadIdx.x < cnt ? min(a.gorder[min(cv.x + (int)threadIdx.x, slots - 1)] & 0xffff, slots - 1)
-                                                 : -1;
-  __syncthreads();
-  // staging units (token t, phase block pb = b * IT + it, word/half ge) of this thread, their rows
-  const uint32_t* urow[NU];
-  int uoff[NU];
-#pragma unroll
-  for (int k = 0; k < NU; ++k) {
-    const int u = threadIdx.x + k * QMM_THREADS;
-    const int t = u / (NBP * 8), sl = t < QTOK ? slot_l[t] : -1;
-    uoff[k] = sl >= 0 ? u - t * (NBP * 8) : -1;  // -1: a zero unit (no slot) or past the stage
-    urow[k] = a.xp_act + (size_t)(sl >= 0 ? sl : 0) * NB * XP_DW;
-  }
-  uint32_t aw[NU][4];
-  auto load_act = [&](int q) {
-#pragma unroll
-    for (int k = 0; k < NU; ++k) {
-      const int o = uoff[k] < 0 ? 0 : uoff[k], pb = o >> 3, ge = o & 7, bb = pb / IT, it = pb - bb * IT;
-      const uint32_t* src = urow[k] + (size_t)(chain(4 * q + bb) + L * it) * XP_DW;
-      const uint32_t* sw = src + ((ge & 1) ? 4 : 0) + (ge >> 1);
-      const uint32_t v0 = sw[0], v1 = sw[8], v2 = sw[16], v3 = src[24 + (ge & 1)];
-      const bool in = uoff[k] >= 0;
-      aw[k][0] = in ? v0 : 0u;
-      aw[k][1] = in ? v1 : 0u;
-      aw[k][2] = in ? v2 : 0u;
-      aw[k][3] = in ? v3 : 0u;
-    }
-  };
-  auto store_act = [&](uint32_t* st) {
-#pragma unroll
-    for (int k = 0; k < NU; ++k) {
-      const int u = threadIdx.x + k * QMM_THREADS;
-      if (u < QTOK * NBP * 8) {
-        const int t = u / (NBP * 8), o = u - t * (NBP * 8), pb = o >> 3, ge = o & 7;
-        uint32_t* blk = st + (t * NBP + pb) * MB_DW;
-        uint32_t* dst = blk + 2 * (ge >> 1) + (ge & 1);
-        dst[0] = aw[k][0] & 0x7f7f7f7fu;
-        dst[8] = ((aw[k][0] >> 7) & 0x01010101u) | ((aw[k][1] << 1) & 0x7e7e7e7eu);
-        dst[16] = (aw[k][1] >> 6) & 0x03030303u;
-        dst[24] = aw[k][2];
-        blk[(ge < 2 ? 32 : 34) + (ge & 1)] = aw[k][3];
-      }
-    }
-  };
-  load_act(0);
-  store_act(lds);
-  if (NPH > 1) load_act(1);
-  __syncthreads();
-  const int qte = (cnt + MMA_TOK - 1) / MMA_TOK;  // token groups holding a slot (uniform)
-  float ch[4][QT], stk[LOGQ > 0 ? LOGQ : 1][QT], res[QT];
-#pragma unroll
-  for (int b = 0; b < 4; ++b)
-#pragma unroll
-    for (int tq = 0; tq < QT; ++tq) ch[b][tq] = 0.0f;
-  // A operand of lane: token 4 tq + (lane & 15) / 4, limb lane & 3, word g; (p, SX) of token 4 tq + g
-  const int aoff2 = ((((lane & 15) >> 2) * NBP) * MB_DW + (lane & 3) * 8 + 2 * g) / 2;
-  const int poff2 = ((g * NBP) * MB_DW + 32) / 2;
-  constexpr int TGS = MMA_TOK * NBP * MB_DW / 2;  // one token group, in uint2
-#pragma unroll 1
-  for (int q = 0; q < NPH; ++q) {
-    const uint2* st2 = reinterpret_cast<const uint2*>(lds + (NPH > 1 ? (q & 1) * PDW : 0));
-#pragma unroll
-    for (int it = 0; it < IT; ++it) {
-      const auto p0 = __builtin_amdgcn_permlane32_swap(wr[it].x, wr[it].z, false, false);
-      const auto p1 = __builtin_amdgcn_permlane32_swap(wr[it].y, wr[it].w, false, false);
-      const auto q0 = __builtin_amdgcn_permlane16_swap(p0[0], p1[0], false, false);
-      const auto q1 = __builtin_amdgcn_permlane16_swap(p0[1], p1[1], false, false);
-      const uint32_t T[4] = {q0[0], q0[1], q1[0], q1[1]};
-      uint32_t sbv[4];
-#pragma unroll
-      for (int b = 0; b < 4; ++b) sbv[b] = pr[it][b];
-      load_w(q + 1, it, wr[it], pr[it]);  // the ring slot's block of the next phase
-#pragma unroll
-      for (int b = 0; b < 4; ++b) {
-        const int pb = b * IT + it;
-        const long bop = (long)(T[b] & 0x0f0f0f0fu) | ((long)((T[b] >> 4) & 0x0f0f0f0fu) << 32);
-        const uint32_t sb = sbv[b];
-        v4i_t d[QT];
-#pragma unroll
-        for (int tq = 0; tq < QT; ++tq) {
-          if (tq < qte) {
-            const long aop = *reinterpret_cast<const long*>(st2 + aoff2 + tq * TGS + pb * (MB_DW / 2));
-            const v4i_t z = {0, 0, 0, 0};
-            d[tq] = __builtin_amdgcn_mfma_i32_16x16x32_i8(aop, bop, z, 0, 0, 0);
-          }
-        }
-#pragma unroll
-        for (int tq = 0; tq < QT; ++tq) {
-          if (tq < qte) {
-            const int low = d[tq][0] + 128 * d[tq][1] + 16384 * d[tq][2];
-            const float dx = __builtin_fmaf((float)d[tq][3], 65536.0f, (float)low);
-            const uint2 ps = st2[poff2 + tq * TGS + pb * (MB_DW / 2)];
-            float& acc = ch[b][tq];
-            acc = __builtin_fmaf(__uint_as_float(sb << 16), dx * __uint_as_float(ps.x), acc);
-            acc = __builtin_fmaf(__uint_as_float(sb & 0xffff0000u), __uint_as_float(ps.y), acc);
-          }
-        }
-        __builtin_amdgcn_sched_barrier(0);
-      }
-    }
-    // the group's subtree ((a + b) + (c + d)), then the binary counter over the groups
-#pragma unroll
-    for (int tq = 0; tq < QT; ++tq) {
-      float x = (ch[0][tq] + ch[1][tq]) + (ch[2][tq] + ch[3][tq]);
-      bool open = true;
-#pragma unroll
-      for (int k = 0; k < LOGQ; ++k) {
-        if (open) {
-          if ((q >> k) & 1) {
-            x = stk[k][tq] + x;
-          } else {
-            stk[k][tq] = x;
-            open = false;
-          }
-        }
-      }
-      if (open) res[tq] = x;
-#pragma unroll
-      for (int b = 0; b < 4; ++b) ch[b][tq] = 0.0f;
-    }
-    if (NPH > 1 && q + 1 < NPH) {  // the next phase's words -> the other buffer, then the one after into registers
-      store_act(lds + ((q + 1) & 1) * PDW);
-      load_act(q + 2 < NPH ? q + 2 : q + 1);
-      __syncthreads();
-    }
-  }
-#pragma unroll
-  for (int tq = 0; tq < QT; ++tq) {
-    const int t = tq * MMA_TOK + g;
-    const int sl = slot_l[t];
-    if (sl >= 0 && row < N) a.r[(size_t)sl * H + row] = f2bf(res[tq]);
-  }
-}
-
-// ---------------------------------------------------------------------------
-// Prepared blocks xp [M][NB][XP_DW] -> the matrix cores' four-limb layout in memory, xmb
-// [M][NB][MB_DW] (limbs at dwords 0..31, p and SX at 32, 33): one thread per (token, block, word,
-// even/odd) unit, as the GEMMs' LDS staging converts them.
-__global__ __launch_bounds__(256) void k_xmb(const uint32_t* __restrict__ xp, int units, uint32_t* __restrict__ xmb) {
-  const int u = blockIdx.x * 256 + threadIdx.x;
-  if (u >= units) return;
-  const int blk = u >> 3, ge = u & 7;  // blk = token * NB + block
-  const uint32_t* src = xp + (size_t)blk * XP_DW;
-  const uint32_t* sw = src + ((ge & 1) ? 4 : 0) + (ge >> 1);
-  const uint32_t w0 = sw[0], w1 = sw[8];
-  uint32_t* dst = xmb + (size_t)blk * MB_DW + 2 * (ge >> 1) + (ge & 1);
-  dst[0] = w0 & 0x7f7f7f7fu;                                          // bits 0-6
-  dst[8] = ((w0 >> 7) & 0x01010101u) | ((w1 << 1) & 0x7e7e7e7eu);    // bits 7-13
-  dst[16] = (w1 >> 6) & 0x03030303u;                                  // bits 14-15
-  dst[24] = sw[16];                                                   // bits 16-23 (signed)
-  if (ge < 2) xmb[(size_t)blk * MB_DW + 32 + ge] = src[24 + ge];      // p, SX
-}
-
-// Batch GEMM for matrices of few rows and long K (the hyper-connection mixer's down and inject
-// projections over a prefill batch), same bits as k_qmv: a workgroup owns one 16-row tile of one
-// of two matrices and 4 QT tokens; its four waves take a quarter of the chain groups each (a
-// subtree of L/4 chains of the butterfly's bit-reversed leaf order, folded as in k_qmm), and the
-// quarters meet in LDS as ((n0 + n1) + (n2 + n3)).  A operands and (p, SX) pairs come straight
-// from the four-limb layout in memory (k_xmb), each step's loads in flight during the previous one.
-constexpr int QMN_THREADS = 256;
-
-template <int L, int IT, int QT>
-__global__ __launch_bounds__(QMN_THREADS) void k_qmn(const uint32_t* __restrict__ wq1, const uint32_t* __restrict__ sb1,
-                                                    int N1, bf16* __restrict__ y1, const uint32_t* __restrict__ wq2,
-                                                    const uint32_t* __restrict__ sb2, int N2, bf16* __restrict__ y2,
-                                                    int K, int gs, const uint32_t* __restrict__ xmb, int M, int tiles1,
-                                                    int tiles) {
-  constexpr int NB = L * IT, P = 4, G = L / 4 / P, LOGG = ilog2(G), STEPS = G * IT, LOGL = ilog2(L);
-  static_assert(L >= 16 && (1 << LOGL) == L && (1 << LOGG) == G, "four quarters of whole chain groups");
-  __shared__ float part[P][QT][64];
-  // workgroup id -> (XCD id % 8, k = id / 8): every tile of a token block on one XCD, so its L2 holds
-  // the block's activations for all of them
-  const int xcd = (int)blockIdx.x & 7, kk = (int)blockIdx.x >> 3;
-  const int tb = (kk / tiles) * 8 + xcd, tile = kk - (kk / tiles) * tiles;
-  if (tb * MMA_TOK * QT >= M) return;  // whole workgroup, before the barrier
-  const int p = threadIdx.x >> 6, lane = threadIdx.x & 63, n = lane & 15, g = lane >> 4;
-  const bool second = tile >= tiles1;
-  const uint32_t* wq = second ? wq2 : wq1;
-  const uint32_t* sbp = second ? sb2 : sb1;
-  const int N = second ? N2 : N1;
-  const int row = (second ? tile - tiles1 : tile) * 16 + n, rc = row < N ? row : N - 1;
-  const int rs = gs == 32 ? 0 : gs == 64 ? 1 : 2;
-  const uint32_t* wrow = wq + (size_t)rc * (K / 8);
-  const uint32_t* srow = sbp + (size_t)rc * sb_row_len(K, gs);
-  const int m0 = tb * MMA_TOK * QT;
-  // this lane's A rows (token 4 tq + (lane & 15) / 4, limb lane & 3, word g) and (p, SX) rows (token
-  // 4 tq + g), tokens past M clamped (their sums are not stored)
-  const uint2* xa[QT];
-  const uint2* xs[QT];
-#pragma unroll
-  for (int tq = 0; tq < QT; ++tq) {
-    const int ta = min(m0 + 4 * tq + ((lane & 15) >> 2), M - 1), ts = min(m0 + 4 * tq + g, M - 1);
-    xa[tq] = reinterpret_cast<const uint2*>(xmb + (size_t)ta * NB * MB_DW + (lane & 3) * 8 + 2 * g);
-    xs[tq] = reinterpret_cast<const uint2*>(xmb + (size_t)ts * NB * MB_DW + 32);
-  }
-  auto chain = [](int i) { return (int)(__builtin_bitreverse32((uint32_t)i) >> (32 - LOGL)); };
-  struct Step {
-    uint4 w;
-    uint32_t pr[4];
-    uint2 a[4][QT], ps[4][QT];
-  };
-  auto load = [&](int s, Step& d) {
-    const int q = p * G + s / IT, it = s - (s / IT) * IT;
-    d.w = *reinterpret_cast<const uint4*>(wrow + (size_t)(chain(4 * q + g) + L * it) * 4);  // cached: reread per token block
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const int u = chain(4 * q + b), j = u + L * it;
-      d.pr[b] = srow[(u >> rs) * IT + it];
-#pragma unroll
-      for (int tq = 0; tq < QT; ++tq) {
-        d.a[b][tq] = xa[tq][(size_t)j * (MB_DW / 2)];
-        d.ps[b][tq] = xs[tq][(size_t)j * (MB_DW / 2)];
-      }
-    }
-  };
-  float ch[4][QT], stk[LOGG > 0 ? LOGG : 1][QT], res[QT];
-#pragma unroll
-  for (int b = 0; b < 4; ++b)
-#pragma unroll
-    for (int tq = 0; tq < QT; ++tq) ch[b][tq] = 0.0f;
-  auto compute = [&](int s, const Step& d) {
-    const auto p0 = __builtin_amdgcn_permlane32_swap(d.w.x, d.w.z, false, false);
-    const auto p1 = __builtin_amdgcn_permlane32_swap(d.w.y, d.w.w, false, false);
-    const auto q0 = __builtin_amdgcn_permlane16_swap(p0[0], p1[0], false, false);
-    const auto q1 = __builtin_amdgcn_permlane16_swap(p0[1], p1[1], false, false);
-    const uint32_t T[4] = {q0[0], q0[1], q1[0], q1[1]};
-#pragma unroll
-    for (int b = 0; b < 4; ++b) {
-      const long bop = (long)(T[b] & 0x0f0f0f0fu) | ((long)((T[b] >> 4) & 0x0f0f0f0fu) << 32);
-      const uint32_t sb = d.pr[b];
-      v4i_t dd[QT];
-#pragma unroll
-      for (int tq = 0; tq < QT; ++tq) {
-        long aop;
-        __builtin_memcpy(&aop, &d.a[b][tq], 8);
-        const v4i_t z = {0, 0, 0, 0};
-        dd[tq] = __builtin_amdgcn_mfma_i32_16x16x32_i8(aop, bop, z, 0, 0, 0);
-      }
-#pragma unroll
-      for (int tq = 0; tq < QT; ++tq) {
-        const int low = dd[tq][0] + 128 * dd[tq][1] + 16384 * dd[tq][2];
-        const float dx = __builtin_fmaf((float)dd[tq][3], 65536.0f, (float)low);
-        float& a = ch[b][tq];
-        a = __builtin_fmaf(__uint_as_float(sb << 16), dx * __uint_as_float(d.ps[b][tq].x), a);
-        a = __builtin_fmaf(__uint_as_float(sb & 0xffff0000u), __uint_as_float(d.ps[b][tq].y), a);
-      }
-    }
-    const int ql = s / IT;
-    if (s - ql * IT == IT - 1) {  // the group's subtree, then the binary counter over this quarter's groups
-#pragma unroll
-      for (int tq = 0; tq < QT; ++tq) {
-        float x = (ch[0][tq] + ch[1][tq]) + (ch[2][tq] + ch[3][tq]);
-        bool open = true;
-#pragma unroll
-        for (int k = 0; k < LOGG; ++k) {
-          if (open) {
-            if ((ql >> k) & 1) {
-              x = stk[k][tq] + x;
-            } else {
-              stk[k][tq] = x;
-              open = false;
-            }
-          }
-        }
-        if (open) res[tq] = x;  // the quarter's last group: its whole subtree
-#pragma unroll
-        for (int b = 0; b < 4; ++b) ch[b][tq] = 0.0f;
-      }
-    }
-  };
-  Step d0, d1;
-  load(0, d0);
-#pragma unroll 1
-  for (int s = 0; s < STEPS; s += 2) {
-    load(s + 1 < STEPS ? s + 1 : s, d1);  // in range either way (unused past the end)
-    compute(s, d0);
-    load(s + 2 < STEPS ? s + 2 : s, d0);
-    if (s + 1 < STEPS) compute(s + 1, d1);
-  }
-#pragma unroll
-  for (int tq = 0; tq < QT; ++tq) part[p][tq][lane] = res[tq];
-  __syncthreads();
-  if (p == 0) {
-#pragma unroll
-    for (int tq = 0; tq < QT; ++tq) {
-      const float v = (part[0][tq][lane] + part[1][tq][lane]) + (part[2][tq][lane] + part[3][tq][lane]);
-      const int t = m0 + 4 * tq + g;
-      if (t < M && row < N) (second ? y2 : y1)[(size_t)t * N + row] = f2bf(v);
-    }
-  }
-}
-
 // MLX affine quantisation of bf16 rows; one thread per group
 // (MLX/backend/cpu/quantized.cpp:1158-1220).
 __global__ void k_quantize(const bf16* __restrict__ w, int64_t groups, int gs, uint32_t* __restrict__ wq,
@@ -1258,7 +915,7 @@ static bool qmm_ok(const uint32_t* sb, int N, int K, int M) {
   if (!sb || M <= MAX_TOKENS || N < QMM_MIN_ROWS || nb % L != 0) return false;
   switch (L * 16 + nb / L) {
     case 4 * 16 + 4: case 4 * 16 + 5: case 4 * 16 + 6: case 8 * 16 + 4: case 8 * 16 + 5: case 16 * 16 + 4:
-    case 16 * 16 + 5: case 32 * 16 + 4: case 32 * 16 + 6: case 64 * 16 + 4: case 64 * 16 + 5: return true;
+    case 32 * 16 + 4: return true;  // the model's depths: gemm.hip
     default: return false;
   }
 }
@@ -1273,74 +930,8 @@ static hipError_t qmm(const uint32_t* wq, const uint32_t* sb, int N, int K, int 
     case 8 * 16 + 4: return qmm_lq<8, 4>(wq, sb, N, K, gs, xp, M, y, yf, st);
     case 8 * 16 + 5: return qmm_lq<8, 5>(wq, sb, N, K, gs, xp, M, y, yf, st);
     case 16 * 16 + 4: return qmm_lq<16, 4>(wq, sb, N, K, gs, xp, M, y, yf, st);
-    case 16 * 16 + 5: return qmm_lq<16, 5>(wq, sb, N, K, gs, xp, M, y, yf, st);
     case 32 * 16 + 4: return qmm_lq<32, 4>(wq, sb, N, K, gs, xp, M, y, yf, st);
-    case 32 * 16 + 6: return qmm_lq<32, 6>(wq, sb, N, K, gs, xp, M, y, yf, st);
-    case 64 * 16 + 4: return qmm_lq<64, 4>(wq, sb, N, K, gs, xp, M, y, yf, st);
-    case 64 * 16 + 5: return qmm_lq<64, 5>(wq, sb, N, K, gs, xp, M, y, yf, st);
     default: return hipErrorNotSupported;
-  }
-}
-
-// The MoE down GEMM over the chunk table: grid = max chunks x 128-row tiles of H (chunks past
-// *a.chunk_n exit at once), activations = the gate|up output rows prepared into a.xp_act.
-template <int L, int IT>
-static hipError_t moe_qmm_li(const MoeArgs& a, hipStream_t st) {
-  constexpr size_t lds = (size_t)(L > 4 ? 2 : 1) * MQ_CHUNK * 4 * IT * MB_DW * 4;
-  static size_t cur = 0;
-  const hipError_t le = ensure_lds(k_moe_qmm<L, IT>, lds, cur);
-  if (le != hipSuccess) return le;
-  const int tiles = (a.H + 127) / 128;
-  hipLaunchKernelGGL((k_moe_qmm<L, IT>), dim3(a.max_chunks * tiles), dim3(QMM_THREADS), lds, st, a, tiles);
-  return hipGetLastError();
-}
-
-static bool moe_qmm_shape(int K) {  // the model's expert width (F = 640: four chains of five blocks)
-  const int nb = K / 32, L = lanes_for_blocks(nb);
-  return nb % L == 0 && L * 16 + nb / L == 4 * 16 + 5;
-}
-
-bool moe_qmm_supported(const MoeArgs& a) { return a.down_sb && a.sh_down_sb && moe_qmm_shape(a.F); }
-
-hipError_t launch_moe_qmm_down(const MoeArgs& a, hipStream_t st) {
-  if (!moe_qmm_supported(a) || !a.chunks || !a.chunk_n || !a.xp_act) return hipErrorInvalidValue;
-  return moe_qmm_li<4, 5>(a, st);
-}
-
-// Two few-row matrices over one batch of prepared activations (the mixer's down and inject
-// projections): k_xmb into xmb [M][K/32][MB_DW], then k_qmn.  hipErrorNotSupported: a shape or
-// matrix it does not take (the caller runs launch_qmv per matrix).
-template <int L, int IT>
-static hipError_t qmn_li(const uint32_t* w1, const uint32_t* sb1, int N1, bf16* y1, const uint32_t* w2,
-                         const uint32_t* sb2, int N2, bf16* y2, int K, int gs, const uint32_t* xmb, int M,
-                         hipStream_t st) {
-  constexpr int QT = 4;  // 16 tokens per workgroup (two token groups measured slower at 512-position batches)
-  const int tiles1 = (N1 + 15) / 16, tiles = tiles1 + (w2 ? (N2 + 15) / 16 : 0);
-  const int tblocks = (M + MMA_TOK * QT - 1) / (MMA_TOK * QT);
-  hipLaunchKernelGGL((k_qmn<L, IT, QT>), dim3(tiles * ((tblocks + 7) / 8 * 8)), dim3(QMN_THREADS), 0, st, w1, sb1, N1, y1, w2, sb2, N2,
-                     y2, K, gs, xmb, M, tiles1, tiles);
-  return hipGetLastError();
-}
-
-bool qmv_pair_ok(const uint32_t* sb1, const uint32_t* w2, const uint32_t* sb2, int K, int M) {
-  const int nb = K / 32, L = lanes_for_blocks(nb), IT = nb % L == 0 ? nb / L : 0;
-  return sb1 && (!w2 || sb2) && M > MAX_TOKENS &&
-         (L * 16 + IT == 64 * 16 + 5 || L * 16 + IT == 64 * 16 + 4 || L * 16 + IT == 32 * 16 + 6);
-}
-
-hipError_t launch_qmv_pair(const uint32_t* w1, const uint32_t* sb1, int N1, bf16* y1, const uint32_t* w2,
-                           const uint32_t* sb2, int N2, bf16* y2, int K, int gs, const uint32_t* xp, uint32_t* xmb,
-                           int M, hipStream_t st) {
-  if (!qmv_pair_ok(sb1, w2, sb2, K, M)) return hipErrorNotSupported;
-  const int nb = K / 32, L = lanes_for_blocks(nb), IT = nb / L;
-  const int units = M * nb * 8;
-  hipLaunchKernelGGL(k_xmb, dim3((units + 255) / 256), dim3(256), 0, st, xp, units, xmb);
-  hipError_t e = hipGetLastError();
-  if (e != hipSuccess) return e;
-  switch (L * 16 + IT) {
-    case 64 * 16 + 5: return qmn_li<64, 5>(w1, sb1, N1, y1, w2, sb2, N2, y2, K, gs, xmb, M, st);
-    case 64 * 16 + 4: return qmn_li<64, 4>(w1, sb1, N1, y1, w2, sb2, N2, y2, K, gs, xmb, M, st);
-    default: return qmn_li<32, 6>(w1, sb1, N1, y1, w2, sb2, N2, y2, K, gs, xmb, M, st);
   }
 }
 

@@ -1,0 +1,105 @@
+"""GPU parity of the batch GEMMs (csrc/gemm.hip), bit-exact: every depth they take at the edges of their
+row blocks and 16-token tiles against the oracle, inputs outside the plain walk's exponent range (blocks
+above 4096, denormal and zero blocks, infinities), checkpoint rows that their loads do not take, and the
+expert chunks against the verify path's windows, with ordinary and with large activations."""
+import numpy as np
+import pytest
+import torch
+
+pytestmark = pytest.mark.gpu
+
+from gpu_util import dev, empty_bf16, host, need_gpu, qweights, rand_bf16, write_device  # noqa: E402
+from oracle import oracle as O  # noqa: E402
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    need_gpu()
+    import mtpx
+    c = mtpx.Context(0)
+    yield c
+    c.close()
+
+
+def _check(ctx, wq, s, b, gs, x, ds=None, db=None):
+    M, N = x.shape[0], wq.shape[0]
+    y_o, yf_o = O.qmv(wq, s, b, gs, x)
+    ds, db = dev(s) if ds is None else ds, dev(b) if db is None else db
+    y, yf = empty_bf16(M, N), torch.zeros(M, N, dtype=torch.float32, device="cuda")
+    ctx.qmv(dev(wq), ds, db, gs, dev(x), y, yf)
+    ctx.synchronize()
+    assert np.array_equal(host(yf).view(np.uint32), yf_o.view(np.uint32))
+    assert np.array_equal(host(y), y_o)
+
+
+# row blocks of 128 (K 2560), 64 (6144), 32 (8192, 10240) and 256 (320) rows; tiles of 16 tokens
+@pytest.mark.parametrize("N,K,gs,M", [
+    (1, 2560, 64, 9), (127, 2560, 32, 16), (128, 2560, 64, 17), (385, 2560, 64, 33), (17, 2560, 32, 80),
+    (64, 6144, 64, 16), (65, 6144, 32, 15), (1, 10240, 32, 9), (33, 10240, 64, 31), (31, 8192, 64, 17),
+    (255, 320, 64, 9), (513, 320, 32, 47), (16, 320, 64, 16),
+])
+def test_gemm_edges_bit_exact(ctx, N, K, gs, M):
+    print("case", N, K, gs, M, flush=True)
+    r = np.random.default_rng(N * 7 + K + M)
+    wq, s, b = qweights(r, N, K, gs)
+    _check(ctx, wq, s, b, gs, rand_bf16(r, (M, K)))
+
+
+@pytest.mark.parametrize("K,gs", [(2560, 64), (6144, 32), (10240, 64), (320, 32)])
+def test_gemm_extreme_blocks_bit_exact(ctx, K, gs):
+    """Tiles with and without a token above 4096 side by side, blocks of every size between 2^-120 and 2^100,
+    zero blocks, and an infinity (whose block value the quantiser defines as any other exponent)."""
+    print("case", K, gs, flush=True)
+    r = np.random.default_rng(K)
+    wq, s, b = qweights(r, 70, K, gs)
+    x = r.standard_normal((40, K)).astype(np.float32)
+    x[5, 32:64] *= 3e4                                            # the first tile walks with the factor
+    x[17] *= np.float32(2.0) ** np.repeat(np.linspace(-118, -2, K // 32).astype(int), 32)
+    x[18] = 0
+    x[19, ::2] *= 1e-7
+    x[36] *= np.float32(2.0) ** np.repeat(np.linspace(0, 90, K // 32).astype(int), 32)
+    xb = O.f32_to_bf16(x)
+    xb[37, 64] = 0x7f80
+    _check(ctx, wq, s, b, gs, xb)
+
+
+def test_gemm_two_byte_aligned_scales(ctx):
+    """Scales and biases at an odd bf16 offset: the GEMV paths take the batch."""
+    r = np.random.default_rng(2)
+    wq, s, b = qweights(r, 48, 2560, 64)
+    pad = [torch.zeros(s.size + 1, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
+    for p, a in zip(pad, (s, b)):
+        p[1:] = dev(a).reshape(-1)
+    _check(ctx, wq, s, b, 64, rand_bf16(r, (21, 2560)), *[p[1:].view(48, 40) for p in pad])
+
+
+@pytest.mark.parametrize("large", [False, True])
+@pytest.mark.parametrize("gs,n", [(64, 200), (32, 149)])
+def test_expert_chunks_match_windows(ctx, gs, n, large):
+    """A prompt whose experts run by chunks of 16 slots gives the verify windows' bits; large: the MoE's
+    input scaled so that its blocks and the experts' activations pass 4096."""
+    import mtpx
+    lc = mtpx.LayerConfig(2560, 96, 6, 640, gs, 24, 2, 256, 64, 128, 1e7, 1e-6, 300)
+    cfg = mtpx.TargetConfig(lc, 16, 48, 4, 2, 4, 4, 320, 4000)
+    cfg.ple_layer = -1
+    t = mtpx.Target(ctx, cfg, seed=77)
+    if large:
+        sc = O.f32_to_bf16(np.full(4 * 2560, 1e5, np.float32))
+        for i in range(2):
+            write_device(t.layer_weights(i).mlp_hc.norm_scale, sc)
+    ids = dev(np.random.default_rng(n).integers(0, 4000, n).astype(np.int32))
+    print("case chunks", gs, n, large, flush=True)
+    a, b = mtpx.TargetState(ctx, t), mtpx.TargetState(ctx, t)
+    lg, mt = empty_bf16(4000), empty_bf16(n, 4 * 2560)
+    t.prefill(a, ids, lg, mt)
+    want = []
+    for w in ids.split(8):
+        lw, mw = empty_bf16(len(w), 4000), empty_bf16(len(w), 4 * 2560)
+        t.verify(b, w.contiguous(), lw, mw)
+        b.commit(len(w))
+        want.append(host(mw))
+    assert np.array_equal(host(mt), np.concatenate(want))
+    assert np.array_equal(host(lg), host(lw)[-1])
+    a.close()
+    b.close()
+    t.close()
