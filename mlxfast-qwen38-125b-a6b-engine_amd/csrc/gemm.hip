@@ -64,22 +64,12 @@ __global__ __launch_bounds__(256) void k_xlimb(const bf16* __restrict__ x, int n
     const uint32_t h = x[(size_t)j * 32 + i];
     const int field = (h >> 7) & 0xff;
     const int f = field < 1 ? 1 : field;
-    int E = f;
-    E = max(E, lane_xor_i<16>(E));
-    E = max(E, lane_xor_i<8>(E));
-    E = max(E, lane_xor_i<4>(E));
-    E = max(E, lane_xor_i<2>(E));
-    E = max(E, lane_xor_i<1>(E));
+    const int E = fold_max_i<16>(f);
     const int32_t sig = (int32_t)((field ? 0x80u : 0u) | (h & 0x7fu));
     const int sh = f - E + 15;
     const int32_t mag = (sh >= 0) ? (sig << sh) : ((sh > -31) ? (sig >> (-sh)) : 0);
     const int32_t m = (h & 0x8000u) ? -mag : mag;
-    int32_t sm = m;
-    sm += lane_xor_i<16>(sm);
-    sm += lane_xor_i<8>(sm);
-    sm += lane_xor_i<4>(sm);
-    sm += lane_xor_i<2>(sm);
-    sm += lane_xor_i<1>(sm);
+    const int32_t sm = fold_sum_i<16>(m);
     const int Ec = E < XL_EMAX ? E : XL_EMAX;
     any |= E > XL_EMAX;
     const float sc = __uint_as_float((uint32_t)(Ec + 108) << 23);  // 2^(Ec-19)

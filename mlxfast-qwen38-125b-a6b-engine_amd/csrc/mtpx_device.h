@@ -60,15 +60,54 @@ __device__ __forceinline__ float lane_xor_f(float v) { return __uint_as_float(la
 template <int OFF>
 __device__ __forceinline__ int lane_xor_i(int v) { return (int)lane_xor<OFF>((uint32_t)v); }
 
-// v + v[lane ^ OFF] for OFF = TOP, TOP/2, ..., 1 (highest level first)
-template <int TOP>
-__device__ __forceinline__ float fold_sum(float v) {
-  if constexpr (TOP >= 1) {
-    v = v + lane_xor_f<TOP>(v);
-    return fold_sum<TOP / 2>(v);
+// Reductions over the lanes of a group as a butterfly, highest level first: op(v, v[lane ^ OFF]) for
+// OFF = TOP, TOP/2, ..., 1, op commutative.  A permlane row swap of v with itself gives both rows of a
+// pair, so levels 32 and 16 need no select; once level 8 is done the lanes of a 16-lane row are equal
+// mod 8, so a rotation by 4 is level 4, and levels 8, 4, 2, 1 are one DPP operation each (half_wave_sum:
+// 7 instructions instead of 14; the GDN step, the GEMVs' folds and every activation block preparation
+// are chains of these).
+template <int CTRL>
+__device__ __forceinline__ uint32_t dpp_of(uint32_t v) {  // every lane a valid source (rotations, quad permutes)
+  return (uint32_t)__builtin_amdgcn_mov_dpp((int)v, CTRL, 0xF, 0xF, true);
+}
+template <int TOP, bool MOD8, typename Op>
+__device__ __forceinline__ uint32_t fold_bits(uint32_t v, Op op) {
+  if constexpr (TOP == 32) {
+    const auto p = __builtin_amdgcn_permlane32_swap(v, v, false, false);
+    return fold_bits<16, false>(op(p[0], p[1]), op);
+  } else if constexpr (TOP == 16) {
+    const auto p = __builtin_amdgcn_permlane16_swap(v, v, false, false);
+    return fold_bits<8, false>(op(p[0], p[1]), op);
+  } else if constexpr (TOP == 8) {
+    return fold_bits<4, true>(op(v, dpp_of<0x128>(v)), op);  // row_ror:8
+  } else if constexpr (TOP == 4) {
+    if constexpr (MOD8)
+      return fold_bits<2, false>(op(v, dpp_of<0x124>(v)), op);  // row_ror:4
+    else
+      return fold_bits<2, false>(op(v, lane_xor<4>(v)), op);
+  } else if constexpr (TOP == 2) {
+    return fold_bits<1, false>(op(v, dpp_of<0x4E>(v)), op);  // quad_perm [2,3,0,1]
+  } else if constexpr (TOP == 1) {
+    return op(v, dpp_of<0xB1>(v));  // quad_perm [1,0,3,2]
   } else {
     return v;
   }
+}
+
+// v + v[lane ^ OFF] for OFF = TOP, TOP/2, ..., 1 (highest level first)
+template <int TOP>
+__device__ __forceinline__ float fold_sum(float v) {
+  return __uint_as_float(fold_bits<TOP, false>(__float_as_uint(v), [](uint32_t a, uint32_t b) {
+    return __float_as_uint(__uint_as_float(a) + __uint_as_float(b));
+  }));
+}
+template <int TOP>
+__device__ __forceinline__ int fold_sum_i(int v) {
+  return (int)fold_bits<TOP, false>((uint32_t)v, [](uint32_t a, uint32_t b) { return a + b; });
+}
+template <int TOP>
+__device__ __forceinline__ int fold_max_i(int v) {
+  return (int)fold_bits<TOP, false>((uint32_t)v, [](uint32_t a, uint32_t b) { return (uint32_t)max((int)a, (int)b); });
 }
 
 // exp(x): Cody-Waite split with a two-part ln2, degree-7 Taylor polynomial on
@@ -193,22 +232,12 @@ __device__ inline void xprep_block(const bf16* __restrict__ x32, uint32_t* __res
 __device__ __forceinline__ void xprep_lanes_direct(uint32_t h, int i, uint32_t* __restrict__ dst) {
   const int field = (h >> 7) & 0xff;
   const int f = field < 1 ? 1 : field;
-  int E = f;
-  E = max(E, lane_xor_i<16>(E));
-  E = max(E, lane_xor_i<8>(E));
-  E = max(E, lane_xor_i<4>(E));
-  E = max(E, lane_xor_i<2>(E));
-  E = max(E, lane_xor_i<1>(E));
+  const int E = fold_max_i<16>(f);
   const int32_t sig = (int32_t)((field ? 0x80u : 0u) | (h & 0x7fu));
   const int sh = f - E + 15;
   const int32_t mag = (sh >= 0) ? (sig << sh) : ((sh > -31) ? (sig >> (-sh)) : 0);
   const int32_t m = (h & 0x8000u) ? -mag : mag;
-  int32_t sm = m;
-  sm += lane_xor_i<16>(sm);
-  sm += lane_xor_i<8>(sm);
-  sm += lane_xor_i<4>(sm);
-  sm += lane_xor_i<2>(sm);
-  sm += lane_xor_i<1>(sm);
+  const int32_t sm = fold_sum_i<16>(m);
   const uint32_t u = (uint32_t)m & 0xffffffu;
   const int at = 4 * (i & 6);  // bit offset of this element's byte: byte (i & 7) >> 1 of its word
   uint32_t w0 = (u & 0xffu) << at, w1 = ((u >> 8) & 0xffu) << at, w2 = (u >> 16) << at;
