@@ -33,7 +33,9 @@ namespace mtpx {
 constexpr int GDN_THREADS = 512;  // 16 half-waves
 constexpr int GDN_D = 128;
 constexpr int GDN_SPLIT = 4;      // workgroups per value head, each owning 128 / GDN_SPLIT state rows
-constexpr int GDN_BSPLIT = 8;     // the batch kernel's workgroups per value head (a long recurrence: more, shorter chains)
+constexpr int GDN_BSPLIT = 16;    // the batch kernel's workgroups per value head
+constexpr int GDN_BTHREADS = 256; // and their threads: a state row per half-wave
+constexpr int GDN_BWIN = 16;      // positions it stages at once
 
 // log1p(y), y in [0, 1]: 2 atanh(s), s = y / (2 + y), odd series to s^15.
 __device__ __forceinline__ float log1p_det(float y) {
@@ -328,17 +330,16 @@ __global__ __launch_bounds__(GDN_THREADS) void k_gdn_step(GdnArgs a) {
     }
 }
 
-// A prefill batch through the core (S positions, any count), two launches.
+// A prefill batch through the core (S positions, any count), three launches.
 //   k_gdn_prep_batch: one workgroup per position: the conv, SiLU and q/k norms of every key head's
 //     q and k and every value head's v (a half-wave per 128-channel vector, as the step kernel
 //     does them), and every head's decay and beta gates, into the batch's prep buffers;
-//   k_gdn_batch: the step kernel's workgroup layout with eight workgroups per value head (16 state
-//     rows each: the batch's long recurrence runs as more, shorter chains), the P committed steps of the
-//     previous window replayed onto the state, then the batch's positions in order, the next
-//     window's prepped vectors loaded while the current one's recurrence runs; every position
-//     committed: the state is stored after the last one, the batch's last kc-1 conv input rows
-//     become the conv base (slot nxt), no journal is written; the head's last workgroup runs the
-//     gated norm and the prepared output blocks of every position.
+//   k_gdn_batch: each value head's recurrence, the P committed steps of the previous window replayed
+//     onto the state, then the batch's positions in order, the next positions' prepped vectors loaded
+//     while the current ones' recurrence runs; every position committed: the state is stored after the
+//     last one, the batch's last kc-1 conv input rows become the conv base (slot nxt), no journal is
+//     written; the outputs go to ypub [hv][128][S rounded up to 32] as f32;
+//   k_gdn_norm_batch: the gated norm and the prepared output blocks of every position.
 // The float operations of every position are a verify window's, so the bits are the same.
 template <int KC>
 __global__ __launch_bounds__(GDN_THREADS) void k_gdn_prep_batch(GdnArgs a, GdnBatch b) {
@@ -392,66 +393,59 @@ __global__ __launch_bounds__(GDN_THREADS) void k_gdn_prep_batch(GdnArgs a, GdnBa
   }
 }
 
-template <int KC>
-__global__ __launch_bounds__(GDN_THREADS) void k_gdn_batch(GdnArgs a, GdnBatch b) {
-  __shared__ float qs[2][MAX_TOKENS][GDN_D], ks[2][MAX_TOKENS][GDN_D], vs[2][MAX_TOKENS][GDN_D];
-  __shared__ float dec[2][MAX_TOKENS], bet[2][MAX_TOKENS];
-  __shared__ float ys[MAX_TOKENS][GDN_D];
-  __shared__ bf16 gated[MAX_TOKENS][GDN_D];
+// Sixteen workgroups of four waves per value head, one state row per half-wave (768 workgroups at 48
+// heads: three per CU, three waves per SIMD).  A step is a chain of about 45 instructions per row, most of
+// them issue-bound at that occupancy; the gated norm is a launch of its own (a head's last workgroup
+// running it for the whole batch was a serial tail of about a quarter of the launch), and the outputs
+// stay in registers, one step per lane, until 32 of them go out as one 128-byte store.  512 positions,
+// 48 heads: 438 us with the norm in the launch, eight workgroups of 16 half-waves per head -> 157 + 10 us.
+__global__ __launch_bounds__(GDN_BTHREADS) void k_gdn_batch(GdnArgs a, GdnBatch b) {
+  constexpr int W = GDN_BWIN, RW = GDN_D / GDN_BSPLIT;  // staged positions; state rows of a workgroup
+  static_assert(RW == GDN_BTHREADS / 32 && 2 * GDN_BWIN == 32, "a row per half-wave, two windows per output store");
+  __shared__ float qs[2][W][GDN_D], ks[2][W][GDN_D];
+  __shared__ float vs[2][W][RW], dec[2][W], bet[2][W];
   const int h = blockIdx.x, ratio = a.hv / a.hk, hk = h / ratio;
-  const int r0 = blockIdx.y * (GDN_D / GDN_BSPLIT);  // this workgroup's state rows
+  const int r0 = blockIdx.y * RW;               // this workgroup's state rows
   const bool w0 = blockIdx.y == 0;
-  const bool lead = (h % ratio) == 0 && w0;         // writes the q/k channels' conv base rows
-  const int hw = threadIdx.x >> 5, l = threadIdx.x & 31;
+  const bool lead = (h % ratio) == 0 && w0;     // writes the q/k channels' conv base rows
+  const int tid = threadIdx.x, hw = tid >> 5, l = tid & 31, r = r0 + hw;
   const int S = a.S, P = a.P, KM1 = a.kc - 1;
-  const int ntask = 2 * a.hk + a.hv;
-  constexpr int RPH = GDN_D / GDN_BSPLIT / (GDN_THREADS / 32);
-  // a window's prepped vectors: (q, k, v) x MAX_TOKENS x 128 floats as float4 units, and the gates
-  constexpr int U4 = 3 * MAX_TOKENS * GDN_D / 4;  // float4 units of a window
-  // this thread's units: u0 = threadIdx.x and u1 = threadIdx.x + GDN_THREADS (while < U4) -> (vector which,
-  // position tt, float4 e4); the source offsets (relative to the window's first position) and the LDS targets
-  // are the same every window
-  static_assert(U4 > GDN_THREADS && U4 <= 2 * GDN_THREADS, "two units per thread");
-  auto unit = [&](int u, const float*& src, float*& dst, int& tt) {
-    const int which = u / (MAX_TOKENS * GDN_D / 4), rem = u % (MAX_TOKENS * GDN_D / 4);
-    const int e4 = rem % (GDN_D / 4);
-    tt = rem / (GDN_D / 4);
-    const int vec = which == 0 ? hk : (which == 1 ? a.hk + hk : 2 * a.hk + h);
-    src = b.vecs + (size_t)vec * GDN_D + 4 * e4;
-    dst = (which == 0 ? &qs[0][tt][0] : (which == 1 ? &ks[0][tt][0] : &vs[0][tt][0])) + 4 * e4;
-  };
-  const bool has1 = (int)threadIdx.x + GDN_THREADS < U4;
-  const float *src0, *src1;
-  float *dst0, *dst1;
-  int tt0, tt1;
-  unit((int)threadIdx.x, src0, dst0, tt0);
-  unit(has1 ? (int)threadIdx.x + GDN_THREADS : (int)threadIdx.x, src1, dst1, tt1);
-  const int gt = (int)threadIdx.x / 2, gk = (int)threadIdx.x & 1;  // gate thread: position, decay or beta
-  float4 pv0, pv1;
-  float pg = 0.0f;
-  const size_t pstride = (size_t)ntask * GDN_D;
-  // unconditional loads (clamped position: positions past S are loaded again and not used)
-#define GDN_FETCH(T0)                                                                                       \
-  do {                                                                                                      \
-    pv0 = *reinterpret_cast<const float4*>(src0 + (size_t)min((T0) + tt0, S - 1) * pstride);                \
-    pv1 = *reinterpret_cast<const float4*>(src1 + (size_t)min((T0) + tt1, S - 1) * pstride);                \
-    if ((int)threadIdx.x < 2 * MAX_TOKENS) pg = b.gates[((size_t)min((T0) + gt, S - 1) * a.hv + h) * 2 + gk]; \
-  } while (0)
-#define GDN_STORE(BUF)                                                                                     \
-  do {                                                                                                     \
-    *reinterpret_cast<float4*>(dst0 + (BUF) * MAX_TOKENS * GDN_D) = pv0;                                     \
-    if (has1) *reinterpret_cast<float4*>(dst1 + (BUF) * MAX_TOKENS * GDN_D) = pv1;                           \
-    if ((int)threadIdx.x < 2 * MAX_TOKENS) (gk ? bet : dec)[(BUF)][gt] = pg;                                \
-  } while (0)
-  GDN_FETCH(0);
-  float s[RPH][4];
+  const size_t pstride = (size_t)(2 * a.hk + a.hv) * GDN_D;
+  // staged per window: q and k [W][128] as float4 units (thread -> position tid / 32 + 8 k, float4 l),
+  // v of this workgroup's rows [W][RW] and the gates [W][2] (position clamped: past S loaded, not used)
+  constexpr int U = W * GDN_D / 4 / GDN_BTHREADS;
+  const float* qsrc = b.vecs + (size_t)hk * GDN_D + 4 * l;
+  const float* ksrc = qsrc + (size_t)a.hk * GDN_D;
+  const float* vsrc = b.vecs + (size_t)(2 * a.hk + h) * GDN_D + r0 + (tid & (RW - 1));
+  float4 pq[U], pk[U];
+  float pv, pg;
+  auto fetch = [&](int t0) {
 #pragma unroll
-  for (int i = 0; i < RPH; ++i) {
-    const float4 s4 = *reinterpret_cast<const float4*>(a.ssm + ((size_t)h * GDN_D + r0 + hw + 16 * i) * GDN_D + 4 * l);
-    s[i][0] = s4.x;
-    s[i][1] = s4.y;
-    s[i][2] = s4.z;
-    s[i][3] = s4.w;
+    for (int k = 0; k < U; ++k) {
+      const size_t t = (size_t)min(t0 + hw + k * (GDN_BTHREADS / 32), S - 1) * pstride;
+      pq[k] = *reinterpret_cast<const float4*>(qsrc + t);
+      pk[k] = *reinterpret_cast<const float4*>(ksrc + t);
+    }
+    pv = vsrc[(size_t)min(t0 + (tid / RW) % W, S - 1) * pstride];
+    pg = b.gates[((size_t)min(t0 + (tid >> 1) % W, S - 1) * a.hv + h) * 2 + (tid & 1)];
+  };
+  auto store = [&](int buf) {
+#pragma unroll
+    for (int k = 0; k < U; ++k) {
+      *reinterpret_cast<float4*>(&qs[buf][hw + k * (GDN_BTHREADS / 32)][4 * l]) = pq[k];
+      *reinterpret_cast<float4*>(&ks[buf][hw + k * (GDN_BTHREADS / 32)][4 * l]) = pk[k];
+    }
+    if (tid < W * RW) vs[buf][tid / RW][tid % RW] = pv;
+    if (tid < 2 * W) (tid & 1 ? bet : dec)[buf][tid >> 1] = pg;
+  };
+  fetch(0);
+  float s[4];
+  {
+    const float4 s4 = *reinterpret_cast<const float4*>(a.ssm + ((size_t)h * GDN_D + r) * GDN_D + 4 * l);
+    s[0] = s4.x;
+    s[1] = s4.y;
+    s[2] = s4.z;
+    s[3] = s4.w;
   }
   // the previous window's committed steps, in order
   for (int p = 0; p < P; ++p) {
@@ -459,111 +453,115 @@ __global__ __launch_bounds__(GDN_THREADS) void k_gdn_batch(GdnArgs a, GdnBatch b
     const uint2 kw = *reinterpret_cast<const uint2*>(a.key_cur + ((size_t)p * a.hk + hk) * GDN_D + 4 * l);
     const float kp[4] = {__uint_as_float(kw.x << 16), __uint_as_float(kw.x & 0xffff0000u),
                          __uint_as_float(kw.y << 16), __uint_as_float(kw.y & 0xffff0000u)};
+    const float dl = a.delta_cur[((size_t)p * a.hv + h) * GDN_D + r];
 #pragma unroll
-    for (int i = 0; i < RPH; ++i) {
-      const float dl = a.delta_cur[((size_t)p * a.hv + h) * GDN_D + r0 + hw + 16 * i];
-#pragma unroll
-      for (int c = 0; c < 4; ++c) {
-        s[i][c] = s[i][c] * gd;
-        s[i][c] = __builtin_fmaf(kp[c], dl, s[i][c]);
-      }
+    for (int c = 0; c < 4; ++c) {
+      s[c] = s[c] * gd;
+      s[c] = __builtin_fmaf(kp[c], dl, s[c]);
     }
   }
-  GDN_STORE(0);
+  // one position: the step kernel's operations in its order
+  auto step = [&](int buf, int t, int lane_t, float& yb) {
+    const float gd = dec[buf][t], bt = bet[buf][t], v = vs[buf][t][hw];
+    const float4 k = *reinterpret_cast<const float4*>(&ks[buf][t][4 * l]);
+    const float4 q = *reinterpret_cast<const float4*>(&qs[buf][t][4 * l]);
+    s[0] = s[0] * gd;
+    s[1] = s[1] * gd;
+    s[2] = s[2] * gd;
+    s[3] = s[3] * gd;
+    float kv = 0.0f + s[0] * k.x;
+    float corr = s[1] * k.y, next = kv + corr;
+    float comp = (next - kv) - corr;
+    kv = next;
+    corr = s[2] * k.z - comp;
+    next = kv + corr;
+    comp = (next - kv) - corr;
+    kv = next;
+    corr = s[3] * k.w - comp;
+    kv = kv + corr;
+    const float kvm = half_wave_sum(kv);
+    const float delta = (v - kvm) * bt;
+    s[0] = __builtin_fmaf(k.x, delta, s[0]);
+    s[1] = __builtin_fmaf(k.y, delta, s[1]);
+    s[2] = __builtin_fmaf(k.z, delta, s[2]);
+    s[3] = __builtin_fmaf(k.w, delta, s[3]);
+    float o = __builtin_fmaf(s[0], q.x, 0.0f);
+    o = __builtin_fmaf(s[1], q.y, o);
+    o = __builtin_fmaf(s[2], q.z, o);
+    o = __builtin_fmaf(s[3], q.w, o);
+    const float y = half_wave_sum(o);
+    yb = l == lane_t ? y : yb;
+  };
+  const int sp = (S + 31) & ~31;  // padded positions of an output row
+  float* yrow = a.ypub + ((size_t)h * GDN_D + r) * sp;
+  store(0);
   __syncthreads();
-  for (int t0 = 0, buf = 0; t0 < S; t0 += MAX_TOKENS, buf ^= 1) {
-    const int n = S - t0 < MAX_TOKENS ? S - t0 : MAX_TOKENS;
-    const bool more = t0 + MAX_TOKENS < S;
-    if (more) GDN_FETCH(t0 + MAX_TOKENS);  // in flight during this window's recurrence
-    // position by position, this thread's RPH state rows side by side (independent chains, each with the
-    // step kernel's operations in its order; the position's k, q and gates read once for all of them)
-    for (int t = 0; t < n; ++t) {
-      const float gd = dec[buf][t], bt = bet[buf][t];
-      const float k0 = ks[buf][t][4 * l], k1 = ks[buf][t][4 * l + 1], k2 = ks[buf][t][4 * l + 2],
-                  k3 = ks[buf][t][4 * l + 3];
-      const float q0 = qs[buf][t][4 * l], q1 = qs[buf][t][4 * l + 1], q2 = qs[buf][t][4 * l + 2],
-                  q3 = qs[buf][t][4 * l + 3];
-#pragma unroll
-      for (int i = 0; i < RPH; ++i) {
-        const int r = r0 + hw + 16 * i;
-        s[i][0] = s[i][0] * gd;
-        float kv = 0.0f + s[i][0] * k0;
-        float comp = 0.0f;
-        {
-          s[i][1] = s[i][1] * gd;
-          const float prod = s[i][1] * k1, corr = prod - comp, next = kv + corr;
-          comp = (next - kv) - corr;
-          kv = next;
-        }
-        {
-          s[i][2] = s[i][2] * gd;
-          const float prod = s[i][2] * k2, corr = prod - comp, next = kv + corr;
-          comp = (next - kv) - corr;
-          kv = next;
-        }
-        {
-          s[i][3] = s[i][3] * gd;
-          const float prod = s[i][3] * k3, corr = prod - comp, next = kv + corr;
-          kv = next;
-        }
-        const float kvm = half_wave_sum(kv);
-        const float delta = (vs[buf][t][r] - kvm) * bt;
-        float o = 0.0f;
-        s[i][0] = __builtin_fmaf(k0, delta, s[i][0]);
-        o = __builtin_fmaf(s[i][0], q0, o);
-        s[i][1] = __builtin_fmaf(k1, delta, s[i][1]);
-        o = __builtin_fmaf(s[i][1], q1, o);
-        s[i][2] = __builtin_fmaf(k2, delta, s[i][2]);
-        o = __builtin_fmaf(s[i][2], q2, o);
-        s[i][3] = __builtin_fmaf(k3, delta, s[i][3]);
-        o = __builtin_fmaf(s[i][3], q3, o);
-        const float y = half_wave_sum(o);
-        if (l == 0) st_pub(a.ypub + ((size_t)(t0 + t) * a.hv + h) * GDN_D + r, round_bf(y));
-      }
+  float yb = 0.0f;
+  for (int t0 = 0, buf = 0; t0 < S; t0 += W, buf ^= 1) {
+    const bool more = t0 + W < S;
+    if (more) fetch(t0 + W);  // in flight during this window's recurrence
+    const int base = t0 & W;  // the window's lanes: 0 .. 15 or 16 .. 31
+    if (t0 + W <= S) {
+#pragma unroll 4
+      for (int t = 0; t < W; ++t) step(buf, t, base + t, yb);
+    } else {
+      for (int t = 0; t < S - t0; ++t) step(buf, t, base + t, yb);
     }
-    if (more) GDN_STORE(buf ^ 1);  // the other buffer: last read in the previous window, before its barrier
+    if (base != 0 || !more) yrow[(t0 & ~31) + l] = yb;
+    if (more) store(buf ^ 1);  // the other buffer: last read in the previous window, before its barrier
     __syncthreads();
   }
-#pragma unroll
-  for (int i = 0; i < RPH; ++i)
-    *reinterpret_cast<float4*>(a.ssm + ((size_t)h * GDN_D + r0 + hw + 16 * i) * GDN_D + 4 * l) =
-        make_float4(s[i][0], s[i][1], s[i][2], s[i][3]);
+  *reinterpret_cast<float4*>(a.ssm + ((size_t)h * GDN_D + r) * GDN_D + 4 * l) = make_float4(s[0], s[1], s[2], s[3]);
   // the batch's last kc-1 input rows become the conv base
-  for (int i = threadIdx.x; i < (w0 ? KM1 * 3 * GDN_D : 0); i += GDN_THREADS) {
+  for (int i = tid; i < (w0 ? KM1 * 3 * GDN_D : 0); i += GDN_BTHREADS) {
     const int j = i / (3 * GDN_D), kind = (i / GDN_D) % 3, d = i % GDN_D;
     if (kind < 2 && !lead) continue;
     const int vec = kind == 0 ? hk : (kind == 1 ? a.hk + hk : 2 * a.hk + h);
     const int ch = vec * GDN_D + d;
     a.conv_nxt[(size_t)j * a.cd + ch] = f2bf(gdn_row(a, P + S + j, ch));
   }
-  if (!ticket_last(a.tickets + h, GDN_BSPLIT - 1)) return;
-  for (int t0 = 0; t0 < S; t0 += MAX_TOKENS) {
-    const int n = S - t0 < MAX_TOKENS ? S - t0 : MAX_TOKENS;
-    for (int i = threadIdx.x; i < n * GDN_D; i += GDN_THREADS)
-      ys[i / GDN_D][i % GDN_D] = ld_pub(a.ypub + ((size_t)(t0 + i / GDN_D) * a.hv + h) * GDN_D + i % GDN_D);
-    __syncthreads();
-    for (int t = hw; t < n; t += GDN_THREADS / 32) {
-      float acc = 0.0f;
+}
+
+// The batch's gated norm: one workgroup per 32 positions of a value head.  The outputs [128 rows][32
+// positions] are turned through LDS (rounded to bf16 as the step kernel publishes them), then a
+// half-wave per position runs the step kernel's norm.
+__global__ __launch_bounds__(256) void k_gdn_norm_batch(GdnArgs a) {
+  __shared__ float ys[32][GDN_D + 4];
+  __shared__ bf16 gated[32][GDN_D];
+  const int t0 = blockIdx.x * 32, h = blockIdx.y, S = a.S, sp = (S + 31) & ~31;
+  const int hw = threadIdx.x >> 5, l = threadIdx.x & 31, n = min(32, S - t0);
+  const float* src = a.ypub + (size_t)h * GDN_D * sp + t0 + l;
+  float v[GDN_D / 8];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) acc = __builtin_fmaf(ys[t][4 * l + i], ys[t][4 * l + i], acc);
-      const float inv = 1.0f / sqrtf(half_wave_sum(acc) / 128.0f + a.eps);
+  for (int k = 0; k < GDN_D / 8; ++k) v[k] = src[(size_t)(hw + 8 * k) * sp];
 #pragma unroll
-      for (int i = 0; i < 4; ++i) {
-        const int d = 4 * l + i;
-        const float nv = round_bf(bf2f(a.norm_w[d]) * round_bf(ys[t][d] * inv));
-        const float z = bf2f(a.proj[(size_t)(t0 + t) * a.pw + a.z_off + h * GDN_D + d]);
-        const bf16 out = f2bf(sigmoid_f32(z) * nv);
-        gated[t][d] = out;
-        if (a.gated) a.gated[(size_t)(t0 + t) * a.hv * GDN_D + h * GDN_D + d] = out;
-      }
+  for (int k = 0; k < GDN_D / 8; ++k) ys[l][hw + 8 * k] = round_bf(v[k]);
+  __syncthreads();
+  for (int t = hw; t < n; t += 8) {
+    const size_t row = (size_t)(t0 + t);
+    const uint32_t* zp = reinterpret_cast<const uint32_t*>(a.proj + row * a.pw + a.z_off + h * GDN_D + 4 * l);
+    const uint2 zw = make_uint2(zp[0], zp[1]);  // a row starts at an even element
+    const float4 y4 = *reinterpret_cast<const float4*>(&ys[t][4 * l]);
+    const float y[4] = {y4.x, y4.y, y4.z, y4.w};
+    float acc = 0.0f;
+#pragma unroll
+    for (int i = 0; i < 4; ++i) acc = __builtin_fmaf(y[i], y[i], acc);
+    const float inv = 1.0f / sqrtf(half_wave_sum(acc) / 128.0f + a.eps);
+    uint32_t out[4];
+#pragma unroll
+    for (int i = 0; i < 4; ++i) {
+      const float nv = round_bf(bf2f(a.norm_w[4 * l + i]) * round_bf(y[i] * inv));
+      out[i] = f2bf(sigmoid_f32(kjournal(zw, i)) * nv);
     }
-    __syncthreads();
-    if (a.xp)
-      for (int task = hw; task < 4 * n; task += GDN_THREADS / 32) {
-        const int t = task >> 2, blk = task & 3;
-        xprep_lanes_direct(gated[t][blk * 32 + l], l, a.xp + ((size_t)(t0 + t) * a.hv * 4 + h * 4 + blk) * XP_DW);
-      }
-    __syncthreads();  // ys and gated of the next window
+    const uint2 o2 = make_uint2(out[0] | (out[1] << 16), out[2] | (out[3] << 16));
+    *reinterpret_cast<uint2*>(&gated[t][4 * l]) = o2;
+    if (a.gated) *reinterpret_cast<uint2*>(a.gated + (row * a.hv + h) * GDN_D + 4 * l) = o2;
+  }
+  if (!a.xp) return;
+  __syncthreads();
+  for (int task = hw; task < 4 * n; task += 8) {
+    const int t = task >> 2, blk = task & 3;
+    xprep_lanes_direct(gated[t][blk * 32 + l], l, a.xp + ((size_t)(t0 + t) * a.hv * 4 + h * 4 + blk) * XP_DW);
   }
 }
 
@@ -634,9 +632,10 @@ hipError_t launch_gdn_step(const GdnArgs& a, hipStream_t st) {
 
 template <int KC>
 static hipError_t gdn_batch_kc(const GdnArgs& a, const GdnBatch& b, hipStream_t st) {
-  if (!a.tickets || !a.ypub || !b.vecs || !b.gates || a.S < 1) return hipErrorInvalidValue;
+  if (!a.ypub || !b.vecs || !b.gates || a.S < 1) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_gdn_prep_batch<KC>, dim3(a.S), dim3(GDN_THREADS), 0, st, a, b);
-  hipLaunchKernelGGL(k_gdn_batch<KC>, dim3(a.hv, GDN_BSPLIT), dim3(GDN_THREADS), 0, st, a, b);
+  hipLaunchKernelGGL(k_gdn_batch, dim3(a.hv, GDN_BSPLIT), dim3(GDN_BTHREADS), 0, st, a, b);
+  hipLaunchKernelGGL(k_gdn_norm_batch, dim3((a.S + 31) / 32, a.hv), dim3(256), 0, st, a);
   return hipGetLastError();
 }
 

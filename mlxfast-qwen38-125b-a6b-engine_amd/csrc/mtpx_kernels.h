@@ -291,7 +291,7 @@ struct GdnArgs {
   float* ypub;                                  // [S, hv, 128] recurrence outputs published for the gated norm
 };
 hipError_t launch_gdn_step(const GdnArgs& a, hipStream_t st);
-// a prefill batch of a.S positions (any count), every one committed; a.ypub holds a.S positions
+// a prefill batch of a.S positions (any count), every one committed; a.ypub holds a.S positions rounded up to 32
 struct GdnBatch {
   float* vecs;   // [S, 2*hk + hv, 128] the positions' q (per key head), k (per key head), v (per value head)
   float* gates;  // [S, hv, 2] decay, beta
