@@ -2660,7 +2660,9 @@ int mtpx_target_verify(mtpx_ctx h, mtpx_target th, mtpx_target_state sh, const i
   return rc;
 }
 
-constexpr int PREFILL_PASS = 512;  // positions per prefill batch (workspace: attention partials grow with it)
+// Positions per prefill batch: the experts' chunks fill with it (1003 positions of four layers of 512
+// experts, top 10: one batch 11.5 ms, 512 + 491 12.9 ms); the workspace grows with it.
+constexpr int PREFILL_PASS = 1024;
 
 int mtpx_target_prefill(mtpx_ctx h, mtpx_target th, mtpx_target_state sh, const int32_t* ids, int S,
                         uint16_t* logits, uint16_t* multi) {

@@ -170,7 +170,7 @@ bool moe_gemm_ok(const MoeArgs& a);
 hipError_t launch_moe_gemm_gate_up(const MoeArgs& m, const XlBatch& x, hipStream_t st);  // x per token
 hipError_t launch_moe_gemm_down(const MoeArgs& m, const XlBatch& x, hipStream_t st);     // x per slot
 
-constexpr int MOE_TICKETS = 64;
+constexpr int MOE_TICKETS = 128;
 constexpr int MAX_EXPERTS = 1024;
 // A logit never has these bits: a NaN the GEMV makes carries the payload of a bf16 operand (low 16
 // bits zero) or the default NaN's.

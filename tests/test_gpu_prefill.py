@@ -3,9 +3,9 @@ batch gives every position's multi stream and the last position's logits exactly
 committing it in windows of 8 does, and leaves the same state (the next verify is bit-equal).
 Against the oracle composition's windows at small dims (a prompt of two full windows and a tail,
 with the PLE block), against the GPU's own windowed verify path for a prompt of 600 positions
-(two prefill batches, 75 windows, the batched MoE launches) and at full width (hidden 2560, 512
+(75 windows, the batched MoE launches) and of 1100 (two batches, 1024 + 76) and at full width (hidden 2560, 512
 experts, hyper-connections 4 x 2560, the full PLE table, 4 layers): 45 positions over a
-1024-position prefix, 600 positions (the benched batch of 512, then 88), and a prompt after a
+1024-position prefix, 600 positions, and a prompt after a
 partly committed verify window; and the MTP head over a batch of backlog positions (the drafter's
 flush) against windows of 8."""
 import numpy as np
@@ -132,7 +132,7 @@ def test_prefill_matches_oracle_windows(ctx):
 
 
 def test_prefill_two_batches_matches_windows(ctx):
-    """600 positions: two prefill batches (512 + 88), 75 full windows; then a prefill of 3 more positions
+    """600 positions: one batch, 75 full windows; then a prefill of 3 more positions
     (one short window) and a verify, each against the windowed path's state."""
     import mtpx
     from oracle.target_ref import download_target
@@ -170,13 +170,37 @@ def test_prefill_two_batches_matches_windows(ctx):
     t.close()
 
 
+def test_prefill_past_one_batch_matches_windows(ctx, monkeypatch):
+    """1100 positions after 9: a batch of 1024 committed before one of 76 that attends to it, 128 windows routed in the first."""
+    import mtpx
+    from oracle.target_ref import download_target
+    monkeypatch.setitem(LAYER, "max_positions", 1200)
+    t, cfg = _small_target(ctx, 43)
+    ow = download_target(t, cfg)
+    kinds = [L["kind"] for L in ow["layers"]]
+    geoms = {i: L["gdn"]["geom"] for i, L in enumerate(ow["layers"]) if L["kind"] == 0}
+    V, W = cfg["vocab"], cfg["hc"] * cfg["hidden"]
+    a, b = mtpx.TargetState(ctx, t), mtpx.TargetState(ctx, t)
+    _load_prefix(a, kinds, geoms, cfg, 9, 3)
+    _load_prefix(b, kinds, geoms, cfg, 9, 3)
+    ids = np.random.default_rng(12).integers(0, V, 1100).astype(np.int32)
+    print("case prefill 1100 vs windows", flush=True)
+    got_mt, got_lg = _prefill(t, a, ids, V, W)
+    want_mt, want_lg = _windows(t, b, ids, V, W)
+    assert np.array_equal(got_mt, want_mt)
+    assert np.array_equal(got_lg, want_lg)
+    assert a.info() == b.info() == (1109, 0)
+    a.close()
+    b.close()
+    t.close()
+
+
 @pytest.mark.timeout(600)
 @pytest.mark.parametrize("pre,n,partial", [(1024, 45, False), (400, 600, False), (300, 70, True)],
                          ids=["45-after-1024", "600-after-400", "70-after-partial-window"])
 def test_prefill_full_width_matches_windows(ctx, pre, n, partial):
     """Full width, 4 layers at gs64 (GDN 16/48 heads, attention 24/2 x 256, 512 experts top-10, the PLE
-    block with its full table): a 45-position prompt after a 1024-position prefix; 600 positions (a
-    batch of 512 at the benched size, then 88) after 400; and a prompt after a verify window of 5 of
+    block with its full table): a 45-position prompt after a 1024-position prefix; 600 positions after 400; and a prompt after a verify window of 5 of
     which 3 positions were committed (the batch GDN kernel replays the committed journal steps and
     reads the conv rows of that window)."""
     import mtpx
