@@ -506,6 +506,293 @@ __global__ __launch_bounds__(256) void k_attn_combine(const float* __restrict__ 
   }
 }
 
+// ---------------------------------------------------------------------------
+// Attention of a prefill batch (S queries over their own keys, head dim 256), two launches with the
+// canonical order's bits (scores: sequential fmaf over d; per chunk of ATTN_CHUNK keys the maximum, the
+// exps, l and P.V in key order; chunks folded in order):
+//   k_attn_scores: 128 (query, head) rows x 128 keys per workgroup (64 x 64 for few), 8 x 8 chains per thread, 16
+//     dimensions at a time through LDS as f32 [d][row] (the rows and keys of a thread in two groups of
+//     four, so its 16-byte reads are conflict-free): 64 fmaf per four reads;
+//   k_attn_pv: 24 rows per workgroup (six per wave) walk the chunks in order: V staged once for the
+//     rows, a lane owning four output columns of every row; no partials in memory.
+// The (chunk, kv head, query) launch staged every chunk once per query and wrote 1 KB of partials per
+// row and chunk: 1003 queries of 24 heads over an empty cache 1495 us + 234 us of combine, here 99 us
+// (bound by its 3.1 G fmaf: 62 TFLOP/s) + 186 us (as many, bound by the reads of V and the exps between
+// barriers).  The workspace is 4 B per row and key instead of 32.
+constexpr int AS_D = 16;               // dimensions per step of the scores
+constexpr int PV_ROWS = 24, PV_RW = 6; // rows per workgroup, per wave
+constexpr int PV_MAXCH = 64;           // chunks: T <= 2048
+
+template <int AT>
+__global__ __launch_bounds__(256, 4) void k_attn_scores(const bf16* __restrict__ q, int S, int HQ, int HK,
+                                                        const bf16* __restrict__ kc, int64_t tmax, int T, float scale,
+                                                        int TP, float* __restrict__ sc) {
+  constexpr int D = PP_D, E = AT / 16;  // rows and keys per thread, in groups of four 64 apart
+  __shared__ float qs[2][AS_D][AT], ks[2][AS_D][AT];
+  const int hk = blockIdx.z, G = HQ / HK, R = S * G;
+  const int row0 = blockIdx.x * AT, key0 = blockIdx.y * AT;
+  if (key0 > T - S + min(row0 + AT - 1, R - 1) / G) return;  // no row sees these keys
+  const int tid = threadIdx.x, ty = tid >> 4, tx = tid & 15;
+  // staging, 8 dimensions of a row a load: the threads take a query row and a key each (128), or the
+  // first half the rows and the second half the keys (64)
+  constexpr int NLD = AT / 64;
+  const int lr = tid & (AT - 1), half = (tid / AT) & 1;
+  const int row = min(row0 + lr, R - 1), key = min(key0 + lr, T - 1);
+  const uint4* qp = reinterpret_cast<const uint4*>(q + ((size_t)(row / G) * HQ + hk * G + row % G) * D + 8 * half);
+  const uint4* kp = reinterpret_cast<const uint4*>(kc + ((size_t)hk * tmax + key) * D + 8 * half);
+  const bool isq = NLD == 2 || tid < 128;
+  const uint4* p0 = isq ? qp : kp;
+  float* d0 = (isq ? &qs[0][0][0] : &ks[0][0][0]) + 8 * half * AT + lr;
+  const float f0 = isq ? scale : 1.0f;  // (x * 1.0f is x; a NaN key stays one)
+  uint4 va = p0[0], vb = make_uint4(0u, 0u, 0u, 0u);
+  if (NLD == 2) vb = kp[0];
+  float acc[E][E];
+#pragma unroll
+  for (int i = 0; i < E; ++i)
+#pragma unroll
+    for (int j = 0; j < E; ++j) acc[i][j] = 0.0f;
+  auto put = [&](int buf) {
+    const uint32_t a[4] = {va.x, va.y, va.z, va.w}, b[4] = {vb.x, vb.y, vb.z, vb.w};
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      d0[(buf * AS_D + 2 * k) * AT] = f0 * __uint_as_float(a[k] << 16);
+      d0[(buf * AS_D + 2 * k + 1) * AT] = f0 * __uint_as_float(a[k] & 0xffff0000u);
+      if (NLD == 2) {
+        ks[buf][8 * half + 2 * k][lr] = __uint_as_float(b[k] << 16);
+        ks[buf][8 * half + 2 * k + 1][lr] = __uint_as_float(b[k] & 0xffff0000u);
+      }
+    }
+  };
+  put(0);
+  __syncthreads();
+#pragma unroll 1
+  for (int st = 0; st < D / AS_D; ++st) {
+    const int buf = st & 1;
+    if (st + 1 < D / AS_D) {  // the next step's rows in flight during this one
+      va = p0[(st + 1) * (AS_D / 8)];
+      if (NLD == 2) vb = kp[(st + 1) * (AS_D / 8)];
+    }
+#pragma unroll 4
+    for (int d = 0; d < AS_D; ++d) {
+      float a[E], b[E];
+#pragma unroll
+      for (int p = 0; p < E / 4; ++p) {
+        *reinterpret_cast<float4*>(a + 4 * p) = *reinterpret_cast<const float4*>(&qs[buf][d][64 * p + 4 * ty]);
+        *reinterpret_cast<float4*>(b + 4 * p) = *reinterpret_cast<const float4*>(&ks[buf][d][64 * p + 4 * tx]);
+      }
+#pragma unroll
+      for (int i = 0; i < E; ++i)
+#pragma unroll
+        for (int j = 0; j < E; ++j) acc[i][j] = __builtin_fmaf(a[i], b[j], acc[i][j]);
+    }
+    if (st + 1 < D / AS_D) {
+      put(buf ^ 1);
+      __syncthreads();
+    }
+  }
+#pragma unroll
+  for (int i = 0; i < E; ++i) {
+    const int r = row0 + 64 * (i / 4) + 4 * ty + i % 4;
+    if (r >= R) continue;
+    float* dst = sc + ((size_t)hk * R + r) * TP + key0 + 4 * tx;
+#pragma unroll
+    for (int p = 0; p < E / 4; ++p)
+      if (key0 + 64 * p + 4 * tx < TP)
+        *reinterpret_cast<float4*>(dst + 64 * p) = make_float4(acc[i][4 * p], acc[i][4 * p + 1], acc[i][4 * p + 2], acc[i][4 * p + 3]);
+  }
+}
+
+__global__ __launch_bounds__(256) void k_attn_pv(const float* __restrict__ sc, int S, int HQ, int HK,
+                                                 const bf16* __restrict__ vc, int64_t tmax, int T, int TP,
+                                                 const bf16* __restrict__ qkv, int QW, int gate_off,
+                                                 bf16* __restrict__ out_gated, uint32_t* __restrict__ xp_gated) {
+  constexpr int D = PP_D, C = ATTN_CHUNK, RW = PV_RW;
+  __shared__ uint4 vs[2][C * D / 8];
+  __shared__ float es[4][RW][C + 4];
+  __shared__ float mcs[PV_ROWS][PV_MAXCH + 1];
+  const int hk = blockIdx.y, G = HQ / HK, R = S * G;
+  const int row0 = ((int)gridDim.x - 1 - (int)blockIdx.x) * PV_ROWS;  // the longest rows first
+  const int tid = threadIdx.x, lane = tid & 63, hl = lane & 31, half = lane >> 5;
+  const int wave = __builtin_amdgcn_readfirstlane(tid >> 6);
+  const int wr0 = row0 + wave * RW;  // this wave's rows
+  const float ninf = -__uint_as_float(0x7f800000u);
+  auto vis = [&](int r) { return T - S + min(r, R - 1) / G + 1; };  // keys row r sees (uniform)
+  const int nch = (vis(row0 + PV_ROWS - 1) + C - 1) / C;            // chunks any row of the workgroup sees
+  const float* srow = sc + ((size_t)hk * R) * TP;
+  // chunk maxima of this wave's rows, a chunk per half-wave; a chunk whose sum of exps would not be above
+  // zero (none visible, a NaN, an infinite maximum) is marked by a NaN and left out, as the fold does
+  for (int c0 = 0; c0 < nch; c0 += 2) {
+    const int c = c0 + half, key = c * C + hl;
+    float x[RW];
+#pragma unroll
+    for (int i = 0; i < RW; ++i) x[i] = srow[(size_t)min(wr0 + i, R - 1) * TP + min(key, TP - 1)];
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+      const bool in = key < vis(wr0 + i), nan = in && x[i] != x[i];
+      const float v = in && !nan ? x[i] : ninf;
+      const float m = __uint_as_float(fold_bits<16, false>(__float_as_uint(v), [](uint32_t a, uint32_t b) {
+        return __uint_as_float(a) > __uint_as_float(b) ? a : b;
+      }));
+      const uint64_t nb = __ballot(nan);
+      const bool bad = (uint32_t)(half ? nb >> 32 : nb) != 0u || __builtin_fabsf(m) == -ninf;
+      if (hl == 0 && c < nch) mcs[wave * RW + i][c] = bad ? __uint_as_float(0x7fc00000u) : m;
+    }
+  }
+  // the wave reads what it wrote (LDS operations of one wave complete in order)
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  const int lr = min(lane, RW - 1);  // lanes 0 .. RW-1: a row's maximum, factor and sum each
+  float M = ninf, L = 0.0f;
+  for (int c = 0; c < nch; ++c) {
+    const float m = mcs[wave * RW + lr][c];
+    M = m > M ? m : M;
+  }
+  float O[RW][4];
+#pragma unroll
+  for (int i = 0; i < RW; ++i)
+#pragma unroll
+    for (int d = 0; d < 4; ++d) O[i][d] = 0.0f;
+  const uint4* v4 = reinterpret_cast<const uint4*>(vc) + (size_t)hk * tmax * (D / 8);
+  uint4 vr[4];
+  float sr[3];
+  auto fetch = [&](int c) {  // the chunk's V rows (zeros past T) and this lane's three scores
+#pragma unroll
+    for (int k = 0; k < 4; ++k) {
+      const int u = tid + 256 * k, key = c * C + u / (D / 8);
+      const uint4 v = v4[(size_t)min(key, T - 1) * (D / 8) + u % (D / 8)];
+      vr[k] = key < T ? v : make_uint4(0u, 0u, 0u, 0u);
+    }
+#pragma unroll
+    for (int k = 0; k < 3; ++k)
+      sr[k] = srow[(size_t)min(wr0 + 2 * k + half, R - 1) * TP + min(c * C + hl, TP - 1)];
+  };
+  fetch(0);
+  for (int c = 0; c < nch; ++c) {
+    const int buf = c & 1;
+#pragma unroll
+    for (int k = 0; k < 4; ++k) vs[buf][tid + 256 * k] = vr[k];
+#pragma unroll
+    for (int k = 0; k < 3; ++k) {  // exps of row 2 k + half, key hl
+      const int i = 2 * k + half, n = T - S + min(wr0 + i, R - 1) / G + 1 - c * C;
+      es[wave][i][hl] = hl < n ? expf_det(sr[k] - mcs[wave * RW + i][c]) : 0.0f;
+    }
+    __syncthreads();  // (a buffer is written again two chunks on, after the next barrier)
+    if (c + 1 < nch) fetch(c + 1);
+    const float mc = mcs[wave * RW + lr][c];
+    const float f = mc == mc ? expf_det(mc - M) : 0.0f;
+    float l = 0.0f;
+#pragma unroll
+    for (int j = 0; j < C; j += 4) {  // in key order (a key past the row's adds 0)
+      const float4 e4 = *reinterpret_cast<const float4*>(&es[wave][lr][j]);
+      l = l + e4.x;
+      l = l + e4.y;
+      l = l + e4.z;
+      l = l + e4.w;
+    }
+    if (mc == mc) L = __builtin_fmaf(l, f, L);
+    float o[RW][4];
+#pragma unroll
+    for (int i = 0; i < RW; ++i)
+#pragma unroll
+      for (int d = 0; d < 4; ++d) o[i][d] = 0.0f;
+    const uint2* vb = reinterpret_cast<const uint2*>(&vs[buf][0]) + lane;  // columns 4 lane .. + 3 of a key
+    auto cols = [](uint2 w, float (&v)[4]) {
+      v[0] = __uint_as_float(w.x << 16);
+      v[1] = __uint_as_float(w.x & 0xffff0000u);
+      v[2] = __uint_as_float(w.y << 16);
+      v[3] = __uint_as_float(w.y & 0xffff0000u);
+    };
+    if ((c + 1) * C <= vis(wr0)) {  // every row of the wave sees the whole chunk
+#pragma unroll 2
+      for (int j = 0; j < C; j += 4) {
+        float e[RW][4];
+#pragma unroll
+        for (int i = 0; i < RW; ++i) *reinterpret_cast<float4*>(e[i]) = *reinterpret_cast<const float4*>(&es[wave][i][j]);
+#pragma unroll
+        for (int u = 0; u < 4; ++u) {
+          float v[4];
+          cols(vb[(j + u) * (D / 4)], v);
+#pragma unroll
+          for (int i = 0; i < RW; ++i)
+#pragma unroll
+            for (int d = 0; d < 4; ++d) o[i][d] = __builtin_fmaf(e[i][u], v[d], o[i][d]);
+        }
+      }
+    } else {
+#pragma unroll
+      for (int i = 0; i < RW; ++i) {
+        const int n = min(vis(wr0 + i) - c * C, C);
+        for (int j = 0; j < n; ++j) {
+          float v[4];
+          cols(vb[j * (D / 4)], v);
+          const float e = es[wave][i][j];
+#pragma unroll
+          for (int d = 0; d < 4; ++d) o[i][d] = __builtin_fmaf(e, v[d], o[i][d]);
+        }
+      }
+    }
+#pragma unroll
+    for (int i = 0; i < RW; ++i) {
+      const float mi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(mc), i));
+      const float fi = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(f), i));
+      if (mi == mi) {
+#pragma unroll
+        for (int d = 0; d < 4; ++d) O[i][d] = __builtin_fmaf(o[i][d], fi, O[i][d]);
+      }
+    }
+  }
+  // the gated rows, and their prepared blocks where asked
+  bf16* gl = reinterpret_cast<bf16*>(&vs[0][0]);  // [PV_ROWS][D]
+  if (xp_gated) __syncthreads();
+#pragma unroll
+  for (int i = 0; i < RW; ++i) {
+    const int r = wr0 + i;
+    const float Li = __int_as_float(__builtin_amdgcn_readlane(__float_as_int(L), i));
+    if (r >= R) continue;
+    const int s = r / G, h = hk * G + r % G;
+    const bf16* gp = qkv + (size_t)s * QW + gate_off + h * D + 4 * lane;
+    uint32_t w[4];
+#pragma unroll
+    for (int d = 0; d < 4; ++d) w[d] = f2bf(bf2f(f2bf(O[i][d] / Li)) * sigmoid_bf16(bf2f(gp[d])));
+    const uint2 o2 = make_uint2(w[0] | (w[1] << 16), w[2] | (w[3] << 16));
+    *reinterpret_cast<uint2*>(out_gated + ((size_t)s * HQ + h) * D + 4 * lane) = o2;
+    if (xp_gated) *reinterpret_cast<uint2*>(gl + (wave * RW + i) * D + 4 * lane) = o2;
+  }
+  if (!xp_gated) return;
+  __syncthreads();
+  for (int task = tid >> 5; task < PV_ROWS * (D / 32); task += 8) {
+    const int i = task / (D / 32), blk = task % (D / 32), r = row0 + i;
+    if (r >= R) continue;  // uniform per half-wave pair of a row's blocks
+    const size_t b = ((size_t)(r / G) * HQ + hk * G + r % G) * (D / 32) + blk;
+    xprep_lanes_direct(gl[i * D + blk * 32 + (tid & 31)], tid & 31, xp_gated + b * XP_DW);
+  }
+}
+
+bool attn_batch_ok(int S, int HQ, int HK, int D, int T) {
+  return S > MAX_TOKENS && D == PP_D && HQ % HK == 0 && T <= PV_MAXCH * ATTN_CHUNK;
+}
+
+size_t attn_batch_floats(int S, int HQ, int T) { return (size_t)S * HQ * ((T + 31) & ~31); }
+
+hipError_t launch_attn_batch(const bf16* q, int S, int HQ, int HK, const bf16* kc, const bf16* vc, int64_t tmax, int T,
+                             float scale, float* scores, const bf16* qkv, int QW, int gate_off, bf16* out_gated,
+                             uint32_t* xp_gated, hipStream_t st) {
+  if (!attn_batch_ok(S, HQ, HK, PP_D, T) || T < S) return hipErrorInvalidValue;
+  const int R = S * (HQ / HK), TP = (T + 31) & ~31;
+  // tiles of 64 rows x 64 keys where those of 128 would not give each CU one: 75 queries
+  // (16 tiles of 128) 44 us with the large tile, 17 us with the small
+  const auto tiles = [&](int t) { return dim3((R + t - 1) / t, (T + t - 1) / t, HK); };
+  const dim3 big = tiles(128);
+  if (big.x * big.y * big.z < 256)
+    hipLaunchKernelGGL((k_attn_scores<64>), tiles(64), dim3(256), 0, st, q, S, HQ, HK, kc, tmax, T, scale, TP, scores);
+  else
+    hipLaunchKernelGGL((k_attn_scores<128>), big, dim3(256), 0, st, q, S, HQ, HK, kc, tmax, T, scale, TP, scores);
+  hipLaunchKernelGGL(k_attn_pv, dim3((R + PV_ROWS - 1) / PV_ROWS, HK), dim3(256), 0, st, scores, S, HQ, HK, vc, tmax, T,
+                     TP, qkv, QW, gate_off, out_gated, xp_gated);
+  return hipGetLastError();
+}
+
 // Row RMSNorm, 256 threads per row: h = x or bf16(x + resid); y = bf16(w * bf16(h * inv)).
 // With xp != nullptr also writes the prepared activation blocks of y (32 lanes per block).
 // grid (M, ceil(H/256)): every workgroup folds the whole row's sum of squares

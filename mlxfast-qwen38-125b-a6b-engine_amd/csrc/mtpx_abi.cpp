@@ -528,6 +528,11 @@ int layer_create(Ctx* c, const mtpx_layer_config* cfg, uint64_t seed, Layer** ou
   return MTPX_OK;
 }
 
+// A batch's scores, or the chunks' partials.
+size_t attn_ws_floats(int M, int HQ, int HK, int D, int T) {
+  return attn_batch_ok(M, HQ, HK, D, T) ? attn_batch_floats(M, HQ, T) : attn_partial_floats(M, HQ, D, T);
+}
+
 // Attention sublayer for M tokens x whose prepared input blocks are in xp:
 // qkv GEMV, q/k norm + RoPE + KV append, verify attention with the output gate,
 // o_proj GEMV -> o [M, H].  xp is reused for the gated attention output, so it
@@ -539,7 +544,8 @@ int attn_enqueue(Ctx* c, const Layer* L, Kv* kv, const uint16_t* x, uint32_t* xp
   uint16_t* qkv = ws_take<uint16_t>(c, (size_t)M * QW);
   uint16_t* q = ws_take<uint16_t>(c, (size_t)M * HQ * D);
   uint16_t* att = ws_take<uint16_t>(c, (size_t)M * HQ * D);
-  float* part = ws_take<float>(c, attn_partial_floats(M, HQ, D, T));
+  const bool batch = attn_batch_ok(M, HQ, HK, D, T);
+  float* part = ws_take<float>(c, attn_ws_floats(M, HQ, HK, D, T));
   hipStream_t st = c->stream;
   int rc = dense_enqueue(c, "qmv_qkv", {L->w.qkv_w, L->w.qkv_s, L->w.qkv_b, L->w.qkv_sb}, QW, H, gs, x, xp, M, qkv);
   if (rc) return rc;
@@ -547,10 +553,16 @@ int attn_enqueue(Ctx* c, const Layer* L, Kv* kv, const uint16_t* x, uint32_t* xp
     LAUNCH(c, "attn_partial", launch_attn_partial_prep(qkv, QW, M, HQ, HK, D, g.rot_dims, L->w.q_norm, L->w.k_norm,
                                                        g.eps, L->w.rope_cos, L->w.rope_sin, kv->k, kv->v, kv->tmax, T,
                                                        1.0f / std::sqrt((float)D), part, st));
-  } else {
+  } else {  // a batch: the prep over all positions, then its own attention where the geometry allows
     LAUNCH(c, "attn_prep", launch_attn_prep(qkv, M, QW, HQ, HK, D, g.rot_dims, L->w.q_norm, L->w.k_norm, g.eps,
                                             L->w.rope_cos, L->w.rope_sin, (int)kv->offset, q, kv->k, kv->v,
                                             kv->tmax, st));
+    if (batch) {
+      const bool gemm = gemm_ok(L->w.o_w, L->w.o_s, L->w.o_b, H, HQ * D, gs, M);
+      LAUNCH(c, "attn_batch", launch_attn_batch(q, M, HQ, HK, kv->k, kv->v, kv->tmax, T, 1.0f / std::sqrt((float)D), part,
+                                                qkv, QW, HQ * D, att, gemm ? nullptr : xp, st));
+      return dense_enqueue(c, "qmv_o", {L->w.o_w, L->w.o_s, L->w.o_b, L->w.o_sb}, H, HQ * D, gs, att, xp, M, o);
+    }
     LAUNCH(c, "attn_partial", launch_attn_partial(q, M, HQ, HK, D, kv->k, kv->v, kv->tmax, T,
                                                   1.0f / std::sqrt((float)D), part, st));
   }
@@ -561,7 +573,7 @@ int attn_enqueue(Ctx* c, const Layer* L, Kv* kv, const uint16_t* x, uint32_t* xp
 size_t attn_ws_bytes(const Layer* L, int M, int T) {
   const mtpx_layer_config& g = L->cfg;
   const int HQ = g.heads, D = g.head_dim;
-  return al(2 * (size_t)M * L->QW) + al(2 * (size_t)M * HQ * D) * 2 + al(4 * attn_partial_floats(M, HQ, D, T)) +
+  return al(2 * (size_t)M * L->QW) + al(2 * (size_t)M * HQ * D) * 2 + al(4 * attn_ws_floats(M, HQ, g.kv_heads, D, T)) +
          xl_ws(M, g.hidden > HQ * D ? g.hidden : HQ * D);
 }
 

@@ -207,6 +207,13 @@ hipError_t launch_attn_partial(const bf16* q, int S, int HQ, int HK, int D, cons
                                int64_t tmax, int T, float scale, float* part, hipStream_t st);
 hipError_t launch_attn_combine(int S, int HQ, int HK, int D, int T, const float* part, const bf16* qkv, int QW,
                                int gate_off, bf16* out, bf16* out_gated, uint32_t* xp_gated, hipStream_t st);
+// A prefill batch (S > MAX_TOKENS, head dim 256, T <= 2048): scores [HQ][S][T rounded up to 32] in the
+// workspace, then the gated output rows (and their prepared blocks where xp_gated is not null).
+bool attn_batch_ok(int S, int HQ, int HK, int D, int T);
+size_t attn_batch_floats(int S, int HQ, int T);
+hipError_t launch_attn_batch(const bf16* q, int S, int HQ, int HK, const bf16* kc, const bf16* vc, int64_t tmax, int T,
+                             float scale, float* scores, const bf16* qkv, int QW, int gate_off, bf16* out_gated,
+                             uint32_t* xp_gated, hipStream_t st);
 hipError_t launch_rmsnorm(const bf16* x, const bf16* resid, int M, int H, const bf16* w, float eps,
                           bf16* sum_out, bf16* y, uint32_t* xp, hipStream_t st);
 hipError_t launch_add(const bf16* a, const bf16* b, int64_t n, bf16* out, hipStream_t st);
