@@ -25,11 +25,14 @@
 // 3 * 16.8 + 28 * 2.5 = 120 cycles of a SIMD; the rest is the operands' way: two workgroups of eight
 // waves per CU (128 registers), each with its next segments in flight (LDS-direct loads, the wait
 // counted so that the later ones stay in flight).  Measured against the i8 batch GEMM and the slot walk
-// it replaced, 512 tokens, group size 64: GDN in-projection 431 -> 208 us, K = 6144 projections 236 ->
-// 127, mixer down and inject 94 -> 43 (and their layout pass), mixer up 71 -> 22, expert gate|up 1000 ->
+// it replaced, 512 tokens, group size 64: GDN in-projection 431 -> 190 us, K = 6144 projections 236 ->
+// 127 (before the split below), mixer down and inject 94 -> 43 (and their layout pass), mixer up 71 -> 22, expert gate|up 1000 ->
 // 340 (HBM floor about 200), expert down 213 -> 160.  On the way (in-projection): segments through
 // registers 423 us, one segment ahead 313, a token's limbs in four 16-byte runs instead of one of 64
-// bytes 246, limb reads with bank conflicts 232.
+// bytes 246, limb reads with bank conflicts 232, a register for every rotation of sx (spilled ones make
+// the walk wait for all loads) 202.  K = 6144 with eight classes of 64 rows, one segment ahead and spills:
+// 1003 tokens 219 us, with four classes and two ahead 158.  One workgroup of 16 waves per CU, twice the rows
+// per limb byte: 490 us where two of eight waves take 400 (they all wait at its barrier).
 #include <algorithm>
 #include <type_traits>
 
@@ -258,7 +261,7 @@ __global__ __launch_bounds__(GT_THREADS, MINW) void k_gemm(std::conditional_t<MO
     }
   }
   auto xrow_at = [&](int t) -> uint32_t { return __shfl((int)xrow_n, t, 64); };
-  const uint32_t xrow_l = xrow_at(lane >> 2);
+  const uint32_t xrow_l = xrow_at(lane >> 2), xoff = (xrow_l * NB + ((lane & 3) ^ g) * 4) * 4;
   // row of row-in-block r, clamped: rows past the end repeat the last one (computed, not stored)
   auto lrow = [&](int r) { return min(row0 + (MODE == GT_GATE_UP && r >= R / 2 ? r - R / 2 : r), rows_w - 1); };
   auto my_tile = [&](int rt) {  // row tile of this wave's tile rt
@@ -307,6 +310,7 @@ __global__ __launch_bounds__(GT_THREADS, MINW) void k_gemm(std::conditional_t<MO
   // once: s, b and sx parts shared over the waves (the block's scale rows are contiguous).
   const uint32_t coff = WHOLE ? 0u : (uint32_t)lrow(((wave % SI) * 64 + lane) / (GW / 8 ? GW / 8 : 1)) * (ng * 2) +
                                          (uint32_t)(lane % (GW / 8 ? GW / 8 : 1)) * 16;
+  const uint32_t soff = 2 * SI < 8 ? sel(wave == 2 * SI, xoff, coff) : xoff;  // one register where a wave loads one
   auto scale_load = [&](uint4* d, int q) {
     if constexpr (WHOLE) {
 #pragma unroll
@@ -324,10 +328,10 @@ __global__ __launch_bounds__(GT_THREADS, MINW) void k_gemm(std::conditional_t<MO
       }
     } else {
       if (wave < 2 * SI)
-        __builtin_amdgcn_raw_ptr_buffer_load_lds(rC, (lds_void_t*)(d + wave * 64), 16, coff, q * (GW * 2), 0, 0);
+        __builtin_amdgcn_raw_ptr_buffer_load_lds(rC, (lds_void_t*)(d + wave * 64), 16, 2 * SI < 8 ? soff : coff, q * (GW * 2), 0, 0);
       if (wave == 2 * SI % 8)
         __builtin_amdgcn_raw_ptr_buffer_load_lds(rX, (lds_void_t*)(d + 2 * SI * 64), 16,
-                                                 (xrow_l * NB + ((lane & 3) ^ (lane >> 4)) * 4) * 4, q * 64, 0, 0);
+                                                 soff, q * 64, 0, 0);
     }
   };
   constexpr int NBP = (NB + XL_PART - 1) / XL_PART;
@@ -347,6 +351,7 @@ __global__ __launch_bounds__(GT_THREADS, MINW) void k_gemm(std::conditional_t<MO
   const int al = n * 4 + (g ^ ((4 - (n >> 2)) & 3));  // limb unit of token n, word group g
   const int wl = (n * SEG + slot(n, c)) * 4 + g;      // weight word of row n (the slot depends on the row mod 16)
   const int sl = n * GW + c / SH;
+  const int xl0 = g * 68 + (c & 3);  // sx of token 4 g: its four words rotated by g
   auto step = [&](auto bigc, int u, const uint4* d, const uint4* ds, int sseg, int seg) {
     constexpr bool BIG = decltype(bigc)::value;
     bf16x8_t av3[3];
@@ -358,11 +363,13 @@ __global__ __launch_bounds__(GT_THREADS, MINW) void k_gemm(std::conditional_t<MO
     const uint32_t* dw = reinterpret_cast<const uint32_t*>(d + AI * 64);
     const uint16_t* dh = reinterpret_cast<const uint16_t*>(ds);
     const float* dx = reinterpret_cast<const float*>(ds + 2 * SI * 64);
+    int xa = xl0;
+    asm volatile("" : "+v"(xa));  // one register, not one per rotation
     float sx4[4], r4[4];
 #pragma unroll
     for (int i = 0; i < 4; ++i)
       sx4[i] = WHOLE ? dx[(4 * g + i) * GB + sseg * SEG + c]
-                     : dx[(4 * g + i) * 16 + (((sseg * SEG + c) >> 2) ^ g) * 4 + (c & 3)];
+                     : dx[(xa ^ ((sseg * SEG + c) >> 2) * 4) + i * 16];
     if constexpr (BIG) {
 #pragma unroll
       for (int i = 0; i < 4; ++i) r4[i] = a.x.xr[(size_t)xrow_at(4 * g + i) * NB + seg * SEG + c];
@@ -533,7 +540,7 @@ hipError_t launch_gemm_pair(const uint32_t* w1, const bf16* s1, const bf16* b1, 
   const bool g32 = gs == 32;
   switch (gemm_shape(K)) {
     case 16 * 16 + 5: return dense_li<16, 5, 4, 4, 3, 4>(a, g32, st);
-    case 32 * 16 + 6: return dense_li<32, 6, 8, 4, 2, 4>(a, g32, st);
+    case 32 * 16 + 6: return dense_li<32, 6, 4, 2, 3, 4>(a, g32, st);
     case 64 * 16 + 5: return dense_li<64, 5, 8, 2, 2, 4>(a, g32, st);
     case 64 * 16 + 4: return dense_li<64, 4, 8, 2, 2, 4>(a, g32, st);
     case 2 * 16 + 5: return dense_li<2, 5, 2, 4, 2, 4>(a, g32, st);
