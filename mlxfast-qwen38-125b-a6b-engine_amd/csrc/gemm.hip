@@ -41,17 +41,13 @@
 namespace mtpx {
 
 constexpr int GT_THREADS = 512;  // eight waves
-constexpr int XL_PART = 32;      // blocks per workgroup of the limb conversion
-constexpr int XL_EMAX = 138;     // largest block exponent whose limbs fit bf16 with the 2^(E-19) scale
 
 typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
-// The limb form of a batch (XlBatch), from x [M][K]: xl [M][nb][3][32] bf16 (each word group g of eight
-// elements in the order 0, 4, 1, 5, 2, 6, 3, 7 that the shifted nibble pairs of a weight word give), sx
-// and xr [M][nb], big [M][ceil(nb / XL_PART)] (any block of the part above XL_EMAX).  One workgroup per
-// token and part, 32 lanes per block as in xprep_lanes_direct; the lanes of elements e and e + 4 of a
-// word group join into one word.  (One workgroup per token: 17 us at 75 tokens of K = 10240.)
+// The limb form of a batch (XlBatch), from x [M][K]: xl [M][nb][3][32] bf16, sx and xr [M][nb], big
+// [M][ceil(nb / XL_PART)] (nonzero somewhere in a token's if any of its blocks is above XL_EMAX).  One
+// workgroup per token and part.  (One workgroup per token: 17 us at 75 tokens of K = 10240.)
 __global__ __launch_bounds__(256) void k_xlimb(const bf16* __restrict__ x, int nb, uint32_t* __restrict__ xl,
                                                float* __restrict__ sx, float* __restrict__ xr,
                                                uint32_t* __restrict__ big) {
@@ -64,27 +60,7 @@ __global__ __launch_bounds__(256) void k_xlimb(const bf16* __restrict__ x, int n
   const int part = blockIdx.y, end = min(nb, (part + 1) * XL_PART);
   int any = 0;
   for (int j = part * XL_PART + (int)(threadIdx.x >> 5); j < end; j += 8) {
-    const uint32_t h = x[(size_t)j * 32 + i];
-    const int field = (h >> 7) & 0xff;
-    const int f = field < 1 ? 1 : field;
-    const int E = fold_max_i<16>(f);
-    const int32_t sig = (int32_t)((field ? 0x80u : 0u) | (h & 0x7fu));
-    const int sh = f - E + 15;
-    const int32_t mag = (sh >= 0) ? (sig << sh) : ((sh > -31) ? (sig >> (-sh)) : 0);
-    const int32_t m = (h & 0x8000u) ? -mag : mag;
-    const int32_t sm = fold_sum_i<16>(m);
-    const int Ec = E < XL_EMAX ? E : XL_EMAX;
-    any |= E > XL_EMAX;
-    const float sc = __uint_as_float((uint32_t)(Ec + 108) << 23);  // 2^(Ec-19)
-    const int32_t limb[3] = {m & 0xff, (m >> 8) & 0xff, m >> 16};
-#pragma unroll
-    for (int k = 0; k < 3; ++k) {
-      uint32_t v = __float_as_uint((float)limb[k] * sc) >> 16;  // exact: eight significant bits
-      v |= lane_xor<4>(v) << 16;
-      if ((i & 4) == 0) xl[(size_t)j * 48 + k * 16 + (i >> 3) * 4 + (i & 3)] = v;
-    }
-    if (i == 4) sx[j] = (float)sm * block_scale(E);
-    if (i == 5) xr[j] = __uint_as_float((uint32_t)(127 + E - Ec) << 23);
+    any |= xlimb_lanes(x[(size_t)j * 32 + i], i, xl + (size_t)j * 48, sx + j, xr + j);
   }
   any = __syncthreads_or(any);
   if (threadIdx.x == 0) big[t * gridDim.y + part] = any ? 1u : 0u;

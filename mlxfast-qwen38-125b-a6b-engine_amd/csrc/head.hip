@@ -103,6 +103,64 @@ __global__ __launch_bounds__(256) void k_hc_norm(const bf16* __restrict__ residu
   if (xp && d < H) xprep_lanes_direct(n, t & 31, xp + (base + d) / 32 * XP_DW);
 }
 
+// The same over a batch: grid (hc, S), a workgroup its whole row of a stream (the launch above loads and
+// folds the row once per 256 elements of it: with thousands of rows that is ten times the work, 85 us at
+// 1003 x 4 rows of 2560, here 47 us with the limb form), and the normed row in limb form instead of xp where xl.xl is set
+// (a pass of 28 us over it saved; 126 MB).
+template <int IT, bool EXACT, int MODE>
+__global__ __launch_bounds__(256) void k_hc_norm_batch(const bf16* __restrict__ residual, const bf16* __restrict__ out,
+                                                       const bf16* __restrict__ inject, int hc, int H, int tile,
+                                                       const bf16* __restrict__ scale, float eps,
+                                                       bf16* __restrict__ stream, bf16* __restrict__ normed,
+                                                       uint32_t* __restrict__ xp, XlBatch xl) {
+  __shared__ float wsum[4];
+  const int c = blockIdx.x, s = blockIdx.y, t = threadIdx.x;
+  const size_t W = (size_t)hc * H;
+  const size_t base = (size_t)s * W + (size_t)c * H;
+  const bf16* rr = tile ? residual + (size_t)s * H : residual + base;
+  const bf16* orow = MODE > 0 ? out + (size_t)s * H : rr;
+  const float inj = MODE == 2 ? bf2f(inject[(size_t)s * hc + c]) : 0.0f;
+  float v[IT];
+  float acc = 0.0f;
+#pragma unroll
+  for (int j = 0; j < IT; ++j) {
+    const int dj = t + 256 * j;
+    const bool in = EXACT || dj < H;
+    const int dd = in ? dj : H - 1;
+    float x = bf2f(rr[dd]);
+    if (MODE > 0) {
+      const float o = bf2f(orow[dd]);
+      x = round_bf(x + (MODE == 2 ? round_bf(o * inj) : o));
+    }
+    v[j] = in ? x : 0.0f;
+    if (in) acc = __builtin_fmaf(v[j], v[j], acc);
+  }
+  acc = wave_fold64(acc);
+  if ((t & 63) == 0) wsum[t >> 6] = acc;
+  __syncthreads();
+  const float total = ((wsum[0] + wsum[1]) + wsum[2]) + wsum[3];
+  const float inv = 1.0f / sqrtf(total / (float)H + eps);
+  int any = 0;
+#pragma unroll
+  for (int j = 0; j < IT; ++j) {
+    const int d = t + 256 * j;
+    if (!EXACT && d >= H) break;  // H % 32 == 0: whole blocks
+    const bf16 n = f2bf(bf2f(scale[(size_t)c * H + d]) * round_bf(v[j] * inv));
+    if (stream) stream[base + d] = f2bf(v[j]);
+    if (normed) normed[base + d] = n;
+    const size_t b = (base + d) / 32;
+    if (xl.xl)
+      any |= xlimb_lanes(n, t & 31, reinterpret_cast<uint32_t*>(xl.xl) + b * 48, xl.sx + b, xl.xr + b);
+    else if (xp)
+      xprep_lanes_direct(n, t & 31, xp + b * XP_DW);
+  }
+  if (xl.xl) {  // the token's parts: each written by one of its workgroups, with what that one saw
+    any = __syncthreads_or(any);
+    const int parts = (int)(W / 32 + XL_PART - 1) / XL_PART;
+    for (int p = c + hc * t; p < parts; p += 256 * hc) xl.big[(size_t)s * parts + p] = any ? 1u : 0u;
+  }
+}
+
 // grid (S, ceil(LW/256)), 256 threads; LW % 32 == 0.
 __global__ __launch_bounds__(256) void k_silu_xprep(const bf16* __restrict__ lo, int LW, bf16* __restrict__ act,
                                                     uint32_t* __restrict__ xp) {
@@ -145,6 +203,21 @@ hipError_t launch_embed_rows(const uint32_t* wq, const bf16* s, const bf16* b, i
 }
 
 template <int IT, bool EXACT>
+static void hc_norm_batch_mode(const dim3& grid, const bf16* residual, const bf16* out, const bf16* inject, int hc,
+                               int H, int tile, const bf16* scale, float eps, bf16* stream, bf16* normed,
+                               uint32_t* xp, const XlBatch& xl, hipStream_t st) {
+  if (!out)
+    hipLaunchKernelGGL((k_hc_norm_batch<IT, EXACT, 0>), grid, dim3(256), 0, st, residual, out, inject, hc, H, tile,
+                       scale, eps, stream, normed, xp, xl);
+  else if (!inject)
+    hipLaunchKernelGGL((k_hc_norm_batch<IT, EXACT, 1>), grid, dim3(256), 0, st, residual, out, inject, hc, H, tile,
+                       scale, eps, stream, normed, xp, xl);
+  else
+    hipLaunchKernelGGL((k_hc_norm_batch<IT, EXACT, 2>), grid, dim3(256), 0, st, residual, out, inject, hc, H, tile,
+                       scale, eps, stream, normed, xp, xl);
+}
+
+template <int IT, bool EXACT>
 static void hc_norm_mode(const dim3& grid, const bf16* residual, const bf16* out, const bf16* inject, int hc, int H,
                          int tile, const bf16* scale, float eps, bf16* stream, bf16* normed, uint32_t* xp,
                          hipStream_t st) {
@@ -161,7 +234,19 @@ static void hc_norm_mode(const dim3& grid, const bf16* residual, const bf16* out
 
 hipError_t launch_hc_norm(const bf16* residual, const bf16* out, const bf16* inject, int S, int hc, int H,
                           int tile, const bf16* scale, float eps, bf16* stream, bf16* normed, uint32_t* xp,
-                          hipStream_t st) {
+                          hipStream_t st, const XlBatch* xl) {
+  if (S > MAX_TOKENS) {
+    const XlBatch x = xl ? *xl : XlBatch{};
+    const dim3 grid(hc, S);
+    if (H == 2560)
+      hc_norm_batch_mode<10, true>(grid, residual, out, inject, hc, H, tile, scale, eps, stream, normed, xp, x, st);
+    else if (H <= 256 * 16)
+      hc_norm_batch_mode<16, false>(grid, residual, out, inject, hc, H, tile, scale, eps, stream, normed, xp, x, st);
+    else
+      hc_norm_batch_mode<48, false>(grid, residual, out, inject, hc, H, tile, scale, eps, stream, normed, xp, x, st);
+    return hipGetLastError();
+  }
+  if (xl) return hipErrorInvalidValue;
   const dim3 grid(hc, S, (H + 255) / 256);
   if (H == 2560)
     hc_norm_mode<10, true>(grid, residual, out, inject, hc, H, tile, scale, eps, stream, normed, xp, st);

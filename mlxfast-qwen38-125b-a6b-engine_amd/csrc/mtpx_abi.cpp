@@ -619,12 +619,12 @@ size_t head_ws_bytes(const Head* hd, int S, int T) {
   const int XB = (H > HQ * D ? H : HQ * D) / 32;
   // per mixer call (three per step): lo, act [S, LW]; inj [S, hc]; xpL; w [S, W]
   const size_t mix = al(2 * (size_t)S * LW) * 2 + al(2 * (size_t)S * g.hc) + al(4 * (size_t)S * (LW / 32) * XP_DW) +
-                     al(2 * (size_t)S * W) + xl_ws(S, W);
+                     al(2 * (size_t)S * W) + xl_ws(S, LW);
   const size_t moe = S > MAX_TOKENS ? moe_windows_ws_bytes(&hd->w.layer.moe, S) : moe_ws_bytes(&hd->w.layer.moe, S);
   return moe + attn_ws_bytes(hd->layer, S, T) + 3 * mix + al(2 * (size_t)S * H) * 6 +
          al(2 * (size_t)S * W) * 5 + al(2 * (size_t)S * g.hc) + al(4 * (size_t)S * XB * XP_DW) +
          al(4 * (size_t)S * (W / 32) * XP_DW) + al(2 * (size_t)hd->w.shortlist_rows) +
-         al(4 * argmax_work_items(1, hd->w.shortlist_rows)) * 2 + xl_ws(S * g.hc, H) + 8192;
+         al(4 * argmax_work_items(1, hd->w.shortlist_rows)) * 2 + xl_ws(S * g.hc, H) + xl_ws(S, W) + 8192;
 }
 
 // One hyper-connection mixer over the normed rows (prepared blocks in xpW):
@@ -634,8 +634,15 @@ struct HcGeom {
   int H, hc, LW, gs;  // hidden, streams, low rank, group size
 };
 
+// Whether a batch's down and inject rows run as the batch GEMM, on the normed rows in limb form.
+bool mix_batch_ok(const HcGeom& g, const mtpx_hc_weights* hw, int S) {
+  const int W = g.hc * g.H;
+  return gemm_ok(hw->down.w, hw->down.s, hw->down.b, g.LW, W, g.gs, S) &&
+         (!hw->inject.w || gemm_ok(hw->inject.w, hw->inject.s, hw->inject.b, g.hc, W, g.gs, S));
+}
+
 int hc_mix_enqueue(Ctx* c, const HcGeom& g, const mtpx_hc_weights* hw, const uint16_t* normed, const uint32_t* xpW,
-                   int S, uint16_t* x, uint16_t* j, uint32_t* xpH) {
+                   const XlBatch& xlW, int S, uint16_t* x, uint16_t* j, uint32_t* xpH) {
   const int H = g.H, W = g.hc * H, LW = g.LW, gs = g.gs;
   hipStream_t st = c->stream;
   if (mix_supported(H, g.hc, LW, S)) {
@@ -664,15 +671,10 @@ int hc_mix_enqueue(Ctx* c, const HcGeom& g, const mtpx_hc_weights* hw, const uin
   uint16_t* wm = ws_take<uint16_t>(c, (size_t)S * W);
   const bool inj_on = hw->inject.w != nullptr;
   int rc;
-  if (gemm_ok(hw->down.w, hw->down.s, hw->down.b, LW, W, gs, S) &&
-      (!inj_on || gemm_ok(hw->inject.w, hw->inject.s, hw->inject.b, g.hc, W, gs, S))) {  // a batch: both in one launch
-    const size_t mark = c->ws_used;
-    const XlBatch xl = xl_take(c, S, W);
-    LAUNCH(c, "xlimb", launch_xlimb(reinterpret_cast<const bf16*>(normed), S, W, xl, st));
+  if (mix_batch_ok(g, hw, S)) {  // both in one launch
     LAUNCH(c, "hc_down_inject",
            launch_gemm_pair(hw->down.w, hw->down.s, hw->down.b, LW, reinterpret_cast<bf16*>(lo), nullptr, hw->inject.w,
-                            hw->inject.s, hw->inject.b, inj_on ? g.hc : 0, reinterpret_cast<bf16*>(inj), W, gs, xl, S, st));
-    c->ws_used = mark;
+                            hw->inject.s, hw->inject.b, inj_on ? g.hc : 0, reinterpret_cast<bf16*>(inj), W, gs, xlW, S, st));
   } else {
     if ((rc = dense_enqueue(c, "hc_down", hw->down, LW, W, gs, normed, xpW, S, lo))) return rc;
     if (inj_on && (rc = dense_enqueue(c, "hc_inject", hw->inject, g.hc, W, gs, normed, xpW, S, inj))) return rc;
@@ -683,10 +685,13 @@ int hc_mix_enqueue(Ctx* c, const HcGeom& g, const mtpx_hc_weights* hw, const uin
   return MTPX_OK;
 }
 
-int hc_mix_enqueue(Ctx* c, const Head* hd, const mtpx_hc_weights* hw, const uint16_t* normed, const uint32_t* xpW,
-                   int S, uint16_t* x, uint16_t* j, uint32_t* xpH) {
-  const HcGeom g{hd->cfg.layer.hidden, hd->cfg.hc, hd->cfg.lowrank, hd->cfg.layer.group_size};
-  return hc_mix_enqueue(c, g, hw, normed, xpW, S, x, j, xpH);
+// The rows' norm before a mixer: prepared blocks in xpW, or a batch's limb form in xlW where its GEMM takes them.
+int hc_norm_enqueue(Ctx* c, const HcGeom& g, const mtpx_hc_weights* hw, const uint16_t* residual, const uint16_t* out,
+                    const uint16_t* inject, int S, int tile, float eps, uint16_t* stream, uint16_t* normed,
+                    uint32_t* xpW, const XlBatch& xlW) {
+  LAUNCH(c, "hc_norm", launch_hc_norm(residual, out, inject, S, g.hc, g.H, tile, hw->norm_scale, eps, stream, normed,
+                                      xpW, c->stream, mix_batch_ok(g, hw, S) ? &xlW : nullptr));
+  return MTPX_OK;
 }
 
 // One hyper-connection mixer's weights (random init): hc_norm weight 1/hc (a
@@ -2732,7 +2737,7 @@ int target_verify_enqueue(Ctx* c, Target* t, TargetState* s, const int32_t* ids,
   const int T = (int)s->offset + S;
   const size_t mix = al(2 * (size_t)S * g.lowrank) * 2 + al(2 * (size_t)S * hc) +
                      al(4 * (size_t)S * (g.lowrank / 32) * XP_DW) + al(2 * (size_t)S * W) +
-                     xl_ws(S, W);
+                     xl_ws(S, g.lowrank);
   const Layer* any_attn = nullptr;
   for (const TargetLayer& L : t->layers)
     if (L.attn) any_attn = L.attn;
@@ -2747,7 +2752,7 @@ int target_verify_enqueue(Ctx* c, Target* t, TargetState* s, const int32_t* ids,
   const size_t fixed = al(2 * (size_t)S * H) * 5 + al(2 * (size_t)S * W) * 4 + al(2 * (size_t)S * hc) * 2 +
                        al(4 * (size_t)S * (W / 32) * XP_DW) + al(4 * (size_t)S * XB * XP_DW) +
                        al(4 * (size_t)S * (VD / 32) * XP_DW) + al(2 * (size_t)S * gg.pw) +
-                       (prefill ? al(2 * (size_t)S * VD) : 0) + xl_ws(S, std::max(H, VD)) + 4096;
+                       (prefill ? al(2 * (size_t)S * VD) : 0) + xl_ws(S, std::max(H, VD)) + xl_ws(S, W) + 4096;
   int rc = ws_reserve(c, fixed + per_layer);
   if (rc) return rc;
   ws_begin(c);
@@ -2763,6 +2768,7 @@ int target_verify_enqueue(Ctx* c, Target* t, TargetState* s, const int32_t* ids,
   uint16_t* jA = ws_take<uint16_t>(c, (size_t)S * hc);
   uint16_t* jM = ws_take<uint16_t>(c, (size_t)S * hc);
   uint32_t* xpW = ws_take<uint32_t>(c, (size_t)S * (W / 32) * XP_DW);
+  const XlBatch xlW = S > MAX_TOKENS ? xl_take(c, S, W) : XlBatch{};
   uint32_t* xpH = ws_take<uint32_t>(c, (size_t)S * XB * XP_DW);
   uint32_t* xpG = ws_take<uint32_t>(c, (size_t)S * (VD / 32) * XP_DW);
   uint16_t* proj = ws_take<uint16_t>(c, (size_t)S * gg.pw);
@@ -2778,7 +2784,7 @@ int target_verify_enqueue(Ctx* c, Target* t, TargetState* s, const int32_t* ids,
     if (i == g.ple_layer && t->ple) {
       // the stream of the first inject-norm goes through the PLE block, then is normed again
       LAUNCH(c, "hc_norm", launch_hc_norm(first ? e : sM, first ? nullptr : mo, first ? nullptr : jM, S, hc, H,
-                                          first ? 1 : 0, L.attn_hc.norm_scale, eps, sA, nrm, nullptr, st));
+                                          first ? 1 : 0, L.attn_hc.norm_scale, eps, sA, nullptr, nullptr, st));
       uint16_t* sp = ws_take<uint16_t>(c, (size_t)S * W);
       const size_t mark2 = c->ws_used;
       for (int w0 = 0; w0 < S; w0 += MAX_TOKENS) {  // window by window (one window when verifying)
@@ -2789,14 +2795,13 @@ int target_verify_enqueue(Ctx* c, Target* t, TargetState* s, const int32_t* ids,
           return rc;
         if (prefill) s->ple->committed = n;
       }
-      LAUNCH(c, "hc_norm", launch_hc_norm(sp, nullptr, nullptr, S, hc, H, 0, L.attn_hc.norm_scale, eps, sA, nrm, xpW,
-                                          st));
-    } else {
-      LAUNCH(c, "hc_norm", launch_hc_norm(first ? e : sM, first ? nullptr : mo, first ? nullptr : jM, S, hc, H,
-                                          first ? 1 : 0, L.attn_hc.norm_scale, eps, sA, nrm, xpW, st));
+      if ((rc = hc_norm_enqueue(c, hg, &L.attn_hc, sp, nullptr, nullptr, S, 0, eps, sA, nrm, xpW, xlW))) return rc;
+    } else if ((rc = hc_norm_enqueue(c, hg, &L.attn_hc, first ? e : sM, first ? nullptr : mo, first ? nullptr : jM, S,
+                                     first ? 1 : 0, eps, sA, nrm, xpW, xlW))) {
+      return rc;
     }
     c->ws_used = mark;
-    if ((rc = hc_mix_enqueue(c, hg, &L.attn_hc, nrm, xpW, S, x, jA, xpH))) return rc;
+    if ((rc = hc_mix_enqueue(c, hg, &L.attn_hc, nrm, xpW, xlW, S, x, jA, xpH))) return rc;
     if (L.kind == MTPX_LAYER_GDN) {
       const mtpx_q4& ip = L.gdn->w.in_proj;
       const mtpx_q4& op = L.gdn->w.out_proj;
@@ -2812,9 +2817,9 @@ int target_verify_enqueue(Ctx* c, Target* t, TargetState* s, const int32_t* ids,
     } else {
       if ((rc = attn_enqueue(c, L.attn, s->kv[i], x, xpH, S, ao))) return rc;
     }
-    LAUNCH(c, "hc_norm", launch_hc_norm(sA, ao, jA, S, hc, H, 0, L.mlp_hc.norm_scale, eps, sM, nrm, xpW, st));
+    if ((rc = hc_norm_enqueue(c, hg, &L.mlp_hc, sA, ao, jA, S, 0, eps, sM, nrm, xpW, xlW))) return rc;
     c->ws_used = mark;
-    if ((rc = hc_mix_enqueue(c, hg, &L.mlp_hc, nrm, xpW, S, x, jM, xpH))) return rc;
+    if ((rc = hc_mix_enqueue(c, hg, &L.mlp_hc, nrm, xpW, xlW, S, x, jM, xpH))) return rc;
     if (prefill) {
       if ((rc = moe_enqueue_windows(c, &L.moe, x, S, mo, xpH))) return rc;
     } else if ((rc = moe_enqueue(c, &L.moe, x, S, mo, nullptr, nullptr, nullptr, nullptr, nullptr, xpH,
@@ -2822,13 +2827,17 @@ int target_verify_enqueue(Ctx* c, Target* t, TargetState* s, const int32_t* ids,
       return rc;
     }
   }
-  LAUNCH(c, "hc_norm", launch_hc_norm(sM, mo, jM, S, hc, H, 0, t->final_hc.norm_scale, eps, mt, nrm, xpW, st));
   c->ws_used = mark;
-  if ((rc = hc_mix_enqueue(c, hg, &t->final_hc, nrm, xpW, S, mx, nullptr, xpH))) return rc;
+  const size_t r0 = prefill ? S - 1 : 0;  // prefill: every position's stream, but only the last one's mix and logits
+  if (r0) LAUNCH(c, "hc_norm", launch_hc_norm(sM, mo, jM, (int)r0, hc, H, 0, t->final_hc.norm_scale, eps, mt, nullptr, nullptr, st));
+  const int SF = S - (int)r0;
+  if ((rc = hc_norm_enqueue(c, hg, &t->final_hc, sM + r0 * W, mo + r0 * H, jM + r0 * hc, SF, 0, eps, mt + r0 * W, nrm,
+                            xpW, xlW)))
+    return rc;
+  if ((!prefill || logits) && (rc = hc_mix_enqueue(c, hg, &t->final_hc, nrm, xpW, xlW, SF, mx, nullptr, xpH))) return rc;
   if (logits) {
-    const int r0 = prefill ? S - 1 : 0;  // prefill: the last position's row only
     LAUNCH(c, "qmv_lm_head", launch_qmv(t->lm_head.w, t->lm_head.s, t->lm_head.b, t->lm_head.sb, (int)g.vocab, H, gs,
-                                        xpH + (size_t)r0 * (H / 32) * XP_DW, S - r0, logits, nullptr, st));
+                                        xpH, SF, logits, nullptr, st));
   }
   for (Kv* kv : s->kv)
     if (kv) kv->offset = s->offset + S;
@@ -3036,7 +3045,9 @@ int mtpx_head_forward(mtpx_ctx h, mtpx_head hh, mtpx_kv kvh, const int32_t* ids,
   uint16_t* j = ws_take<uint16_t>(c, (size_t)S * hc);
   uint32_t* xpH = ws_take<uint32_t>(c, (size_t)S * XB * XP_DW);
   uint32_t* xpW = ws_take<uint32_t>(c, (size_t)S * (W / 32) * XP_DW);
+  const XlBatch xlW = S > MAX_TOKENS ? xl_take(c, S, W) : XlBatch{};
   hipStream_t st = c->stream;
+  const HcGeom hg{H, hc, g.lowrank, gs};
   // e = fc_embedding(rms(embed(ids))); h = fc_hidden(rms_W(multi)) per stream
   LAUNCH(c, "embed", launch_embed_rows(w.embed.w, w.embed.s, w.embed.b, H, gs, g.vocab, ids, S, e, st));
   LAUNCH(c, "hc_norm", launch_hc_norm(e, nullptr, nullptr, S, 1, H, 0, w.pre_norm_embedding, eps, nullptr, en, xpH,
@@ -3046,21 +3057,20 @@ int mtpx_head_forward(mtpx_ctx h, mtpx_head hh, mtpx_kv kvh, const int32_t* ids,
                                       st));
   if ((rc = dense_enqueue(c, "qmv_fc", w.fc_hidden, H, H, gs, mn, xpW, S * hc, hs))) return rc;
   // attention block: hyper = e + h; (st0, n) = hc_norm(hyper); (x, j) = mix(attn_hc, n); ao = attn(x)
-  LAUNCH(c, "hc_norm", launch_hc_norm(hs, emb, nullptr, S, hc, H, 0, w.attn_hc.norm_scale, eps, st0, nrm, xpW, st));
-  if ((rc = hc_mix_enqueue(c, hd, &w.attn_hc, nrm, xpW, S, x, j, xpH))) return rc;
+  if ((rc = hc_norm_enqueue(c, hg, &w.attn_hc, hs, emb, nullptr, S, 0, eps, st0, nrm, xpW, xlW))) return rc;
+  if ((rc = hc_mix_enqueue(c, hg, &w.attn_hc, nrm, xpW, xlW, S, x, j, xpH))) return rc;
   if ((rc = attn_enqueue(c, hd->layer, kv, x, xpH, S, ao))) return rc;
   // MoE block
-  LAUNCH(c, "hc_norm", launch_hc_norm(st0, ao, j, S, hc, H, 0, w.mlp_hc.norm_scale, eps, st1, nrm, xpW, st));
-  if ((rc = hc_mix_enqueue(c, hd, &w.mlp_hc, nrm, xpW, S, x, j, xpH))) return rc;
+  if ((rc = hc_norm_enqueue(c, hg, &w.mlp_hc, st0, ao, j, S, 0, eps, st1, nrm, xpW, xlW))) return rc;
+  if ((rc = hc_mix_enqueue(c, hg, &w.mlp_hc, nrm, xpW, xlW, S, x, j, xpH))) return rc;
   if (S > MAX_TOKENS) {  // a batch of the drafter's backlog: the MoE as windows of MAX_TOKENS
     if ((rc = moe_enqueue_windows(c, &w.layer.moe, x, S, ao, xpH))) return rc;
   } else if ((rc = moe_enqueue(c, &w.layer.moe, x, S, ao, nullptr, nullptr, nullptr, nullptr, nullptr, xpH))) {
     return rc;
   }
   // final mixer: multi_next = st1 + m*j; sample = mix(final_hc, hc_norm(multi_next))
-  LAUNCH(c, "hc_norm", launch_hc_norm(st1, ao, j, S, hc, H, 0, w.final_hc.norm_scale, eps, multi_next, nrm, xpW,
-                                      st));
-  if ((rc = hc_mix_enqueue(c, hd, &w.final_hc, nrm, xpW, S, samp, nullptr, xpH))) return rc;
+  if ((rc = hc_norm_enqueue(c, hg, &w.final_hc, st1, ao, j, S, 0, eps, multi_next, nrm, xpW, xlW))) return rc;
+  if ((rc = hc_mix_enqueue(c, hg, &w.final_hc, nrm, xpW, xlW, S, samp, nullptr, xpH))) return rc;
   if (draft) {
     const int NS = w.shortlist_rows;
     const size_t n = argmax_work_items(1, NS);

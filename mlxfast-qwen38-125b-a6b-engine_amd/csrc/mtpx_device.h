@@ -261,6 +261,36 @@ __device__ __forceinline__ void xprep_lanes_direct(uint32_t h, int i, uint32_t* 
   }
 }
 
+// One block of the batch GEMM's limb form, 32 lanes a block, lane i holding element i (bf16 bits h): the
+// three bytes of the block's fixed-point values, each times 2^(min(E, XL_EMAX) - 19) as bf16, in dst[3][16]
+// words (a word group of eight elements in the order 0, 4, 1, 5, 2, 6, 3, 7 that the shifted nibble pairs
+// of a weight word give: the lanes of elements e and e + 4 join), SX in *sx, 2^(E - min(E, XL_EMAX)) in *xr.
+// Returns 1 where E is above XL_EMAX, the largest exponent whose limbs fit bf16 with that scale.
+constexpr int XL_EMAX = 138;
+__device__ __forceinline__ int xlimb_lanes(uint32_t h, int i, uint32_t* __restrict__ dst, float* __restrict__ sx,
+                                           float* __restrict__ xr) {
+  const int field = (h >> 7) & 0xff;
+  const int f = field < 1 ? 1 : field;
+  const int E = fold_max_i<16>(f);
+  const int32_t sig = (int32_t)((field ? 0x80u : 0u) | (h & 0x7fu));
+  const int sh = f - E + 15;
+  const int32_t mag = (sh >= 0) ? (sig << sh) : ((sh > -31) ? (sig >> (-sh)) : 0);
+  const int32_t m = (h & 0x8000u) ? -mag : mag;
+  const int32_t sm = fold_sum_i<16>(m);
+  const int Ec = E < XL_EMAX ? E : XL_EMAX;
+  const float sc = __uint_as_float((uint32_t)(Ec + 108) << 23);  // 2^(Ec-19)
+  const int32_t limb[3] = {m & 0xff, (m >> 8) & 0xff, m >> 16};
+#pragma unroll
+  for (int k = 0; k < 3; ++k) {
+    uint32_t v = __float_as_uint((float)limb[k] * sc) >> 16;  // exact: eight significant bits
+    v |= lane_xor<4>(v) << 16;
+    if ((i & 4) == 0) dst[k * 16 + (i >> 3) * 4 + (i & 3)] = v;
+  }
+  if (i == 4) *sx = (float)sm * block_scale(E);
+  if (i == 5) *xr = __uint_as_float((uint32_t)(127 + E - Ec) << 23);
+  return E > XL_EMAX;
+}
+
 // Exact nibble x limb sums of one 32-element block; w = 4 packed words.
 // Returns DXraw = fmaf((float)D2, 65536, (float)(D1*256 + D0)).
 __device__ __forceinline__ float block_dot(const uint32_t w[4], const uint32_t* __restrict__ xl) {

@@ -153,6 +153,7 @@ inline int moe_max_chunks(int T, int E, int K) {
 }
 // --- batch GEMMs (gemm.hip): more than MAX_TOKENS tokens of the model's depths
 // A batch in limb form (k_xlimb): xl [M][K/32][3][32] bf16, sx and xr [M][K/32], big per token and part of K.
+constexpr int XL_PART = 32;  // blocks of a part
 struct XlBatch {
   uint4* xl;
   float *sx, *xr;
@@ -250,9 +251,11 @@ hipError_t launch_argmax_rows_bf16(const bf16* x, int rows, int64_t V, float* pv
 // --- MTP head pieces (head.hip)
 hipError_t launch_embed_rows(const uint32_t* wq, const bf16* s, const bf16* b, int H, int gs, int64_t V,
                              const int32_t* ids, int S, bf16* out, hipStream_t st);
+// stream, normed, xp: each may be null.  More than MAX_TOKENS rows: the normed rows [S, hc*H] in limb form
+// where xl is given, instead of xp.
 hipError_t launch_hc_norm(const bf16* residual, const bf16* out, const bf16* inject, int S, int hc, int H,
                           int tile, const bf16* scale, float eps, bf16* stream, bf16* normed, uint32_t* xp,
-                          hipStream_t st);
+                          hipStream_t st, const XlBatch* xl = nullptr);
 hipError_t launch_silu_xprep(const bf16* lo, int S, int LW, bf16* act, uint32_t* xp, hipStream_t st);
 hipError_t launch_hc_mix(const bf16* w, const bf16* normed, const bf16* inj, int S, int hc, int H, bf16* input,
                          bf16* inject_out, uint32_t* xp, hipStream_t st);

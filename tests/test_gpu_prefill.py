@@ -285,3 +285,52 @@ def test_head_batch_matches_windows(ctx, n):
     kva.close()
     kvb.close()
     head.close()
+
+
+@pytest.mark.parametrize("n", [9, 41])
+def test_head_batch_at_width_matches_windows(ctx, n):
+    """The head's batch at hidden 2560 (the batch norm's limb form, the mixers' batch GEMMs) against windows of 8:
+    one position more than a window, and a ragged token tile."""
+    import mtpx
+    layer = dict(LAYER, hidden=2560, group_size=64, max_positions=64)
+    hc, vocab = 4, 1000
+    head = mtpx.MTPHead(ctx, mtpx.HeadConfig(mtpx.LayerConfig(**layer), hc, 320, vocab, 500, 980), seed=29)
+    W = hc * 2560
+    r = np.random.default_rng(n)
+    ids, multi = dev(r.integers(0, vocab, n).astype(np.int32)), dev(rand_bf16(r, (n, W)))
+    kva, kvb = (mtpx.KVCache(ctx, layer["kv_heads"], layer["head_dim"], 64) for _ in range(2))
+    print("case head batch at width", n, flush=True)
+    na, sa, nb, sb = empty_bf16(n, W), empty_bf16(n, 2560), empty_bf16(n, W), empty_bf16(n, 2560)
+    head.forward(kva, ids, multi, na, sa)
+    for w0 in range(0, n, 8):
+        w1 = min(n, w0 + 8)
+        head.forward(kvb, ids[w0:w1], multi[w0:w1], nb[w0:w1], sb[w0:w1])
+    assert np.array_equal(host(na), host(nb))
+    assert np.array_equal(host(sa), host(sb))
+    kva.close()
+    kvb.close()
+    head.close()
+
+
+@pytest.mark.parametrize("n", [1, 8, 9, 30])
+def test_prefill_outputs_are_optional(ctx, n):
+    """Without logits, without streams, without both: what is asked for has the same bits, and so has the state."""
+    import mtpx
+    t, cfg = _small_target(ctx, 47)
+    V, W = cfg["vocab"], cfg["hc"] * cfg["hidden"]
+    ids = dev(np.random.default_rng(n).integers(0, V, n).astype(np.int32))
+    nxt = dev(np.array([3, 1, 4, 1], np.int32))
+    print("case prefill optional outputs", n, flush=True)
+    ref = None
+    for want_lg, want_mt in ((True, True), (False, True), (True, False), (False, False)):
+        st = mtpx.TargetState(ctx, t)
+        lg, mt, after = empty_bf16(1, V), empty_bf16(n, W), empty_bf16(4, V)
+        t.prefill(st, ids, lg[0] if want_lg else None, mt if want_mt else None)
+        t.verify(st, nxt, after)
+        got = host(lg), host(mt), host(after)
+        ref = ref or got
+        assert not want_lg or np.array_equal(got[0], ref[0])
+        assert not want_mt or np.array_equal(got[1], ref[1])
+        assert np.array_equal(got[2], ref[2])
+        st.close()
+    t.close()
