@@ -225,15 +225,14 @@ __global__ __launch_bounds__(GT_THREADS, MINW) void k_gemm(std::conditional_t<MO
       b0 = b1 = (e1 ? m.down_b : m.sh_down_b) + r * ng;
     }
     yp = MODE == GT_GATE_UP ? m.act : m.r;
-    // order entry -> slot (window w: w * M (K + 1) + m * K + k routed, + M * K + m shared) -> token
-    const int wslots = m.M * (m.K + 1), slots = m.nwin * wslots;
+    // order entry -> slot (m * K + k routed, M * K + m shared) -> token
+    const int slots = m.M * (m.K + 1);
     const int sl = min(m.gorder[min(pos + min(n, cnt - 1), slots - 1)] & 0xffff, slots - 1);
     yrow_n = sl;
     if (MODE == GT_DOWN) {
       xrow_n = sl;
     } else {
-      const int w = sl / wslots, ls = sl - w * wslots;
-      xrow_n = w * m.M + (ls >= m.M * m.K ? ls - m.M * m.K : ls / m.K);
+      xrow_n = sl >= m.M * m.K ? sl - m.M * m.K : sl / m.K;
     }
   }
   auto xrow_at = [&](int t) -> uint32_t { return __shfl((int)xrow_n, t, 64); };
@@ -526,7 +525,7 @@ hipError_t launch_gemm_pair(const uint32_t* w1, const bf16* s1, const bf16* b1, 
 
 // ---- MoE ----
 bool moe_gemm_ok(const MoeArgs& a) {
-  return gemm_shape(a.H) == 16 * 16 + 5 && gemm_shape(a.F) == 4 * 16 + 5 && a.nwin * a.M * (a.K + 1) < 65536 &&
+  return gemm_shape(a.H) == 16 * 16 + 5 && gemm_shape(a.F) == 4 * 16 + 5 && a.M * (a.K + 1) < 65536 &&
          mat_ok(a.gate_w, a.gate_s, a.gate_b) && mat_ok(a.up_w, a.up_s, a.up_b) && mat_ok(a.down_w, a.down_s, a.down_b) &&
          mat_ok(a.sh_gate_w, a.sh_gate_s, a.sh_gate_b) && mat_ok(a.sh_up_w, a.sh_up_s, a.sh_up_b) &&
          mat_ok(a.sh_down_w, a.sh_down_s, a.sh_down_b);
@@ -534,7 +533,7 @@ bool moe_gemm_ok(const MoeArgs& a) {
 
 hipError_t launch_moe_gemm_gate_up(const MoeArgs& m, const XlBatch& x, hipStream_t st) {
   if (!moe_gemm_ok(m) || !m.gorder || !m.chunks || !m.chunk_n) return hipErrorInvalidValue;
-  const MoeGemmArgs a{m, x, (uint32_t)((size_t)m.nwin * m.M * m.H * 6)};
+  const MoeGemmArgs a{m, x, (uint32_t)((size_t)m.M * m.H * 6)};
   const int grid = (m.max_chunks * (m.F / 64) + 7) / 8 * 8;
   if (m.gs == 32)
     hipLaunchKernelGGL((k_gemm<GT_GATE_UP, 16, 5, 4, 4, true, 3, 4>), dim3(grid), dim3(GT_THREADS), 0, st, a);
@@ -545,7 +544,7 @@ hipError_t launch_moe_gemm_gate_up(const MoeArgs& m, const XlBatch& x, hipStream
 
 hipError_t launch_moe_gemm_down(const MoeArgs& m, const XlBatch& x, hipStream_t st) {
   if (!moe_gemm_ok(m) || !m.gorder || !m.chunks || !m.chunk_n) return hipErrorInvalidValue;
-  const MoeGemmArgs a{m, x, (uint32_t)((size_t)m.nwin * m.M * (m.K + 1) * m.F * 6)};
+  const MoeGemmArgs a{m, x, (uint32_t)((size_t)m.M * (m.K + 1) * m.F * 6)};
   const int grid = (m.max_chunks * (m.H / 128) + 7) / 8 * 8;
   if (m.gs == 32)
     hipLaunchKernelGGL((k_gemm<GT_DOWN, 4, 5, 4, 4, true, 2, 6>), dim3(grid), dim3(GT_THREADS), 0, st, a);

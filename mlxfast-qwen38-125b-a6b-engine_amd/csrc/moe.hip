@@ -93,6 +93,80 @@ __device__ __forceinline__ int route_count_ge(const uint32_t (&key)[EPER], uint3
   return n;
 }
 
+// One token by one wave: its K largest of the E logits in x (register j of a lane: expert lane + 64 j),
+// value descending, expert ascending; lane k < K returns the k-th expert and its softmax weight over the K.
+// ckey, cidx, cval: LDS of this wave, MAX_TOPK each.
+template <int EPER>
+__device__ __forceinline__ void route_token(const float (&x)[EPER], int E, int K, uint32_t* ckey, int* cidx,
+                                            float* cval, int& mys, float& myw) {
+  const int lane = threadIdx.x & 63;
+  float v[EPER];
+  uint32_t key[EPER];
+#pragma unroll
+  for (int j = 0; j < EPER; ++j) {
+    const int e = lane + 64 * j;
+    v[j] = (e < E && x[j] == x[j]) ? x[j] : -__uint_as_float(0x7f800000u);  // a NaN logit ranks as -inf
+    key[j] = e < E ? route_key(v[j]) : 0u;
+  }
+  // T: the K-th largest key, the largest t with at least K keys >= t, found bit by bit from the
+  // top.  A count of exactly K ends the search early: t then parts the K largest from the rest.
+  // T >= key(-inf) > 0 (K <= E), so no lane past E is selected.
+  uint32_t T = 0u;
+  for (int b = 31; b >= 0; --b) {
+    const uint32_t c = T | (1u << b);
+    const int n = route_count_ge<EPER>(key, c);
+    if (n >= K) {
+      T = c;
+      if (n == K) break;
+    }
+  }
+  // selected: every key above T, and of the keys equal to T the lowest experts, K in all
+  // (value descending, expert ascending); compacted into LDS in expert order
+  const int need = K - route_count_ge<EPER>(key, T + 1u);
+  int ties = 0, before = 0;
+#pragma unroll
+  for (int j = 0; j < EPER; ++j) {
+    const uint64_t eq = __ballot(key[j] == T);
+    const bool s = key[j] > T || (key[j] == T && ties + lanes_below(eq) < need);
+    const uint64_t sm = __ballot(s);
+    if (s) {
+      const int p = before + lanes_below(sm);
+      ckey[p] = key[j];
+      cidx[p] = lane + 64 * j;
+      cval[p] = v[j];
+    }
+    ties += __popcll(eq);
+    before += __popcll(sm);
+  }
+  // the wave reads what it wrote (LDS operations of one wave complete in order)
+  __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
+  __builtin_amdgcn_wave_barrier();
+  __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
+  // lane p < K: entry p's rank among the K, then each entry pushed to the lane of its rank
+  int rank = lane;
+  float pv = 0.0f;
+  int pe = 0;
+  if (lane < K) {
+    const uint32_t kp = ckey[lane];
+    rank = 0;
+    for (int q = 0; q < K; ++q) {
+      const uint32_t kq = ckey[q];
+      rank += (kq > kp || (kq == kp && q < lane)) ? 1 : 0;
+    }
+    pv = cval[lane];
+    pe = cidx[lane];
+  }
+  // lane k < K: the k-th selected logit and expert
+  const float myv = __int_as_float(__builtin_amdgcn_ds_permute(rank * 4, __float_as_int(pv)));
+  mys = __builtin_amdgcn_ds_permute(rank * 4, pe);
+  // softmax over the K selected: exp per lane, sum in rank order (lane values read uniformly)
+  const float ev = expf_det(myv - readlane_f(myv, 0));
+  float sum = 0.0f;
+  for (int k = 0; k < K; ++k) sum = sum + readlane_f(ev, k);
+  sum = 1.0f / sum;
+  myw = ev * sum;
+}
+
 // EPER = ceil(E / 64) rounded up to 8 or 16: the logits per lane (expert lane + 64 j in register j).
 // POLL: the logits come from the publish buffer a.pub, each token's wave loading them until none is
 // the sentinel (at most ROUTE_SPIN polls), then copying them to a.logits and putting the sentinel
@@ -144,74 +218,13 @@ __device__ void route_body(const MoeArgs& a) {
         x[j] = (e < E) ? ld_pub(lr + e) : 0.0f;
       }
     }
-    float v[EPER];
-    uint32_t key[EPER];
-#pragma unroll
-    for (int j = 0; j < EPER; ++j) {
-      const int e = lane + 64 * j;
-      v[j] = (e < E && x[j] == x[j]) ? x[j] : -__uint_as_float(0x7f800000u);  // a NaN logit ranks as -inf
-      key[j] = e < E ? route_key(v[j]) : 0u;
-    }
-    // T: the K-th largest key, the largest t with at least K keys >= t, found bit by bit from the
-    // top.  A count of exactly K ends the search early: t then parts the K largest from the rest.
-    // T >= key(-inf) > 0 (K <= E), so no lane past E is selected.
-    uint32_t T = 0u;
-    for (int b = 31; b >= 0; --b) {
-      const uint32_t c = T | (1u << b);
-      const int n = route_count_ge<EPER>(key, c);
-      if (n >= K) {
-        T = c;
-        if (n == K) break;
-      }
-    }
-    // selected: every key above T, and of the keys equal to T the lowest experts, K in all
-    // (value descending, expert ascending); compacted into LDS in expert order
-    const int need = K - route_count_ge<EPER>(key, T + 1u);
-    int ties = 0, before = 0;
-#pragma unroll
-    for (int j = 0; j < EPER; ++j) {
-      const uint64_t eq = __ballot(key[j] == T);
-      const bool s = key[j] > T || (key[j] == T && ties + lanes_below(eq) < need);
-      const uint64_t sm = __ballot(s);
-      if (s) {
-        const int p = before + lanes_below(sm);
-        ckey[wave][p] = key[j];
-        cidx[wave][p] = lane + 64 * j;
-        cval[wave][p] = v[j];
-      }
-      ties += __popcll(eq);
-      before += __popcll(sm);
-    }
-    // the wave reads what it wrote (LDS operations of one wave complete in order)
-    __builtin_amdgcn_fence(__ATOMIC_RELEASE, "wavefront");
-    __builtin_amdgcn_wave_barrier();
-    __builtin_amdgcn_fence(__ATOMIC_ACQUIRE, "wavefront");
-    // lane p < K: entry p's rank among the K, then each entry pushed to the lane of its rank
-    int rank = lane;
-    float pv = 0.0f;
-    int pe = 0;
-    if (lane < K) {
-      const uint32_t kp = ckey[wave][lane];
-      rank = 0;
-      for (int q = 0; q < K; ++q) {
-        const uint32_t kq = ckey[wave][q];
-        rank += (kq > kp || (kq == kp && q < lane)) ? 1 : 0;
-      }
-      pv = cval[wave][lane];
-      pe = cidx[wave][lane];
-    }
-    // lane k < K: the k-th selected logit and expert
-    const float myv = __int_as_float(__builtin_amdgcn_ds_permute(rank * 4, __float_as_int(pv)));
-    const int mys = __builtin_amdgcn_ds_permute(rank * 4, pe);
-    // softmax over the K selected: exp per lane, sum in rank order (lane values read uniformly)
-    const float ev = expf_det(myv - readlane_f(myv, 0));
-    float sum = 0.0f;
-    for (int k = 0; k < K; ++k) sum = sum + readlane_f(ev, k);
-    sum = 1.0f / sum;
+    int mys;
+    float myw;
+    route_token<EPER>(x, E, K, ckey[wave], cidx[wave], cval[wave], mys, myw);
     if (lane < K) {
       sel[wave * K + lane] = mys;
       a.idx[wave * K + lane] = mys;
-      a.w[wave * K + lane] = ev * sum;
+      a.w[wave * K + lane] = myw;
     }
   }
   __syncthreads();
@@ -389,6 +402,148 @@ __global__ __launch_bounds__(RR_THREADS) void k_moe_router_route(MoeArgs a0, int
     route_body<16, false>(a);
 }
 
+
+// ---------------------------------------------------------------------------
+// The router rows over a batch of T tokens: four waves of RW rows each (a bf16 gate row as row E), their
+// weights in registers as f32, against the tokens of the workgroup's range, RB_TOK at a time through LDS
+// (the next ones in flight).  Chains and fold of k_moe_router_route; the first two levels of the fold take
+// the four rows' values together (a permlane swap puts one row's lower lanes beside the other's), so every
+// quarter of the wave goes on with one row.  What bounds it: 220 vector instructions per token and wave at
+// H = 2560 (160 fmaf, 40 to widen x) where the window launch spends 140 per token and row: 1003 tokens of
+// 513 rows BEFORE -> AFTER us.
+constexpr int RB_TOK = 4;
+
+template <int NIT, bool EXACT, int RW>
+__global__ __launch_bounds__(256, 2) void k_moe_router_batch(MoeArgs a, int per) {
+  static_assert(RW == 1 || RW == 4, "rows per wave");
+  extern __shared__ uint4 xs[];  // [2][RB_TOK][H/8]
+  const int H = a.H, E = a.E, T = a.M, nc = H / 8;
+  const int rows = a.sg_w ? E : E + 1;
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int r0 = ((int)blockIdx.x * 4 + wave) * RW;
+  const int t0 = blockIdx.y * per, t1 = min(t0 + per, T);
+  if (t0 >= T) return;
+  float w[RW][8 * NIT];
+#pragma unroll
+  for (int q = 0; q < RW; ++q) {
+    const int r = min(r0 + q, rows - 1);
+    const uint4* wrow = reinterpret_cast<const uint4*>(r < E ? a.router + (size_t)r * H : a.shared_gate);
+#pragma unroll
+    for (int i = 0; i < NIT; ++i) {
+      const int c = lane + 64 * i;
+      const uint4 v = wrow[EXACT || c < nc ? c : nc - 1];
+      const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+      for (int k = 0; k < 4; ++k) {
+        w[q][8 * i + 2 * k] = __uint_as_float(u[k] << 16);
+        w[q][8 * i + 2 * k + 1] = __uint_as_float(u[k] & 0xffff0000u);
+      }
+    }
+  }
+  const uint4* x4 = reinterpret_cast<const uint4*>(a.x);
+  const int un = RB_TOK * nc;  // 16-byte units of a stage; past the last token: its last unit again
+  auto stage = [&](int t, int buf) {
+    for (int u0 = wave * 64; u0 < un; u0 += 256) {
+      const size_t u = (size_t)t * nc + min(u0 + lane, un - 1), last = (size_t)T * nc - 1;
+      if (u0 + lane < un) lds_dma16(xs + buf * un + u0, x4 + (u < last ? u : last));
+    }
+  };
+  stage(t0, 0);
+  for (int t = t0, buf = 0; t < t1; t += RB_TOK, buf ^= 1) {
+    lds_dma_wait();
+    __syncthreads();  // this stage landed; the other one's readers are done
+    if (t + RB_TOK < t1) stage(t + RB_TOK, buf ^ 1);
+    uint4 xv[NIT];  // the next token's chunks, read while this one's are used
+    auto fetch = [&](int m) {
+#pragma unroll
+      for (int i = 0; i < NIT; ++i) xv[i] = xs[buf * un + m * nc + min(lane + 64 * i, nc - 1)];
+    };
+    fetch(0);
+    const int nt = min(RB_TOK, t1 - t);
+    for (int m = 0; m < nt; ++m) {
+      uint4 xc[NIT];
+#pragma unroll
+      for (int i = 0; i < NIT; ++i) xc[i] = xv[i];
+      fetch(min(m + 1, RB_TOK - 1));
+      asm volatile("" ::: "memory");
+      float acc[RW];
+#pragma unroll
+      for (int q = 0; q < RW; ++q) acc[q] = 0.0f;
+#pragma unroll
+      for (int i = 0; i < NIT; ++i) {
+        const int c = lane + 64 * i;
+        if (EXACT || c < nc) {
+          const uint4 v = xc[i];
+          const uint32_t u[4] = {v.x, v.y, v.z, v.w};
+#pragma unroll
+          for (int k = 0; k < 4; ++k) {
+            const float lo = __uint_as_float(u[k] << 16), hi = __uint_as_float(u[k] & 0xffff0000u);
+#pragma unroll
+            for (int q = 0; q < RW; ++q) acc[q] = __builtin_fmaf(w[q][8 * i + 2 * k], lo, acc[q]);
+#pragma unroll
+            for (int q = 0; q < RW; ++q) acc[q] = __builtin_fmaf(w[q][8 * i + 2 * k + 1], hi, acc[q]);
+          }
+        }
+      }
+      float s;
+      int r = r0;
+      if constexpr (RW == 4) {
+        auto pair32 = [](float x, float y) {
+          const auto p = __builtin_amdgcn_permlane32_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+          return __uint_as_float(p[0]) + __uint_as_float(p[1]);
+        };
+        const float s01 = pair32(acc[0], acc[1]), s23 = pair32(acc[2], acc[3]);
+        const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(s01), __float_as_uint(s23), false, false);
+        s = fold_sum<8>(__uint_as_float(p[0]) + __uint_as_float(p[1]));
+        r += ((lane >> 4) & 1) * 2 + (lane >> 5);  // the quarters hold rows 0, 2, 1, 3
+      } else {
+        s = wave_fold64(acc[0]);
+      }
+      if ((lane & (RW == 4 ? 15 : 63)) == 0 && r < rows) {
+        if (r < E)
+          a.logits[(size_t)(t + m) * E + r] = s;
+        else
+          a.gate_logit[t + m] = s;
+      }
+    }
+  }
+}
+
+// The batch's routes, a wave per token: experts and weights only (the expert order of a batch is k_moe_sort's).
+template <int EPER>
+__global__ __launch_bounds__(RR_THREADS) void k_moe_route_batch(MoeArgs a) {
+  __shared__ uint32_t ckey[MAX_TOKENS][MAX_TOPK];
+  __shared__ int cidx[MAX_TOKENS][MAX_TOPK];
+  __shared__ float cval[MAX_TOKENS][MAX_TOPK];
+  const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
+  const int t = blockIdx.x * MAX_TOKENS + wave;
+  if (t >= a.M) return;
+  float x[EPER];
+#pragma unroll
+  for (int j = 0; j < EPER; ++j) {
+    const int e = lane + 64 * j;
+    x[j] = e < a.E ? a.logits[(size_t)t * a.E + e] : 0.0f;
+  }
+  int mys;
+  float myw;
+  route_token<EPER>(x, a.E, a.K, ckey[wave], cidx[wave], cval[wave], mys, myw);
+  if (lane < a.K) {
+    a.idx[(size_t)t * a.K + lane] = mys;
+    a.w[(size_t)t * a.K + lane] = myw;
+  }
+}
+static_assert(RR_THREADS == 64 * MAX_TOKENS, "a wave per token");
+
+// A batch's q4 gate row, a workgroup per MAX_TOKENS tokens.
+template <int GL, int GIT>
+__global__ __launch_bounds__(RR_THREADS) void k_moe_gate_batch(MoeArgs a) {
+  extern __shared__ uint4 xs[];
+  const int t0 = blockIdx.x * MAX_TOKENS;
+  a.x += (size_t)t0 * a.H;
+  a.gate_logit += t0;
+  a.M = min(MAX_TOKENS, a.M - t0);
+  shared_gate_q4<GL, GIT>(a, reinterpret_cast<uint32_t*>(xs));
+}
 
 // ---------------------------------------------------------------------------
 // gate|up + SwiGLU, one workgroup of GU_THREADS = 512 threads per CU over the
@@ -706,8 +861,7 @@ template <int L>
 constexpr int dd_gate_up_rows() { return 4 * (64 / L) > 16 ? 4 * (64 / L) : 16; }
 
 template <int L, int IT, bool PK, bool CB>
-__global__ __launch_bounds__(DD_THREADS) void k_moe_gate_up_dd(MoeArgs a0) {
-  const MoeArgs a = a0.gorder ? a0 : moe_window(a0, blockIdx.y);
+__global__ __launch_bounds__(DD_THREADS) void k_moe_gate_up_dd(MoeArgs a) {
   extern __shared__ uint32_t lds[];  // [H/32][XP_DW]: the slot's token
   constexpr int RW = 64 / L;
   constexpr int UR = dd_gate_up_rows<L>();
@@ -715,16 +869,15 @@ __global__ __launch_bounds__(DD_THREADS) void k_moe_gate_up_dd(MoeArgs a0) {
   static_assert(4 * RW * NP == UR, "four waves cover the rows of a unit");
   const int H = a.H, F = a.F, gs = a.gs, M = a.M, K = a.K;
   const int nb = H / 32, ng = H / gs, P = sb_row_len(H, gs), nfb = F / UR;
-  const int wslots = M * (K + 1), slots = a.gorder ? a.nwin * wslots : wslots;
+  const int slots = M * (K + 1);
   const int n_units = slots * nfb;
   const int w = dd_unit(n_units);
   if (w >= n_units) return;
   const int o = w / nfb, f0 = (w % nfb) * UR;
   const int ov = a.gorder ? a.gorder[o] : a.disp->order[o];
   const int sl = min(ov & 0xffff, slots - 1);  // (clamps: never out of the weights, whatever the table holds)
-  const int win = sl / wslots, ls = sl - win * wslots;  // window and its slot (window 0 without gorder)
-  const bool shared = ls >= M * K;
-  const int m = win * M + (shared ? ls - M * K : ls / K);
+  const bool shared = sl >= M * K;
+  const int m = shared ? sl - M * K : sl / K;
   const int e = shared ? 0 : min(max((ov >> 16) - 1, 0), a.E - 1);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int sub = lane % L, grp = lane / L;
@@ -771,22 +924,21 @@ template <int L, int NW = 4>
 constexpr int dd_down_rows() { return NW * (64 / L); }
 
 template <int L, int IT, bool PK, int NW>
-__global__ __launch_bounds__(64 * NW) void k_moe_down_dd(MoeArgs a0) {
-  const MoeArgs a = a0.gorder ? a0 : moe_window(a0, blockIdx.y);
+__global__ __launch_bounds__(64 * NW) void k_moe_down_dd(MoeArgs a) {
   extern __shared__ uint32_t lds[];  // [F/32][XP_DW]
   constexpr int RW = 64 / L;
   constexpr int DR = dd_down_rows<L, NW>();
   constexpr int NT = 64 * NW;
   const int H = a.H, F = a.F, gs = a.gs, M = a.M, K = a.K;
   const int nb = F / 32, ng = F / gs, P = sb_row_len(F, gs), nhb = (H + DR - 1) / DR;
-  const int wslots = M * (K + 1), slots = a.gorder ? a.nwin * wslots : wslots;
+  const int slots = M * (K + 1);
   const int n_units = slots * nhb;
   const int wu = dd_unit(n_units);
   if (wu >= n_units) return;
   const int o = wu / nhb, hb = wu % nhb, h0 = hb * DR;
   const int ov = a.gorder ? a.gorder[o] : a.disp->order[o];
   const int sl = min(ov & 0xffff, slots - 1);  // (clamps: never out of the weights, whatever the table holds)
-  const bool shared = sl % wslots >= M * K;
+  const bool shared = sl >= M * K;
   const int e = shared ? 0 : min(max((ov >> 16) - 1, 0), a.E - 1);
   const int wave = threadIdx.x >> 6, lane = threadIdx.x & 63;
   const int sub = lane % L, grp = lane / L;
@@ -837,6 +989,54 @@ static hipError_t router_route_go(const MoeArgs& a, hipStream_t st) {
   hipLaunchKernelGGL((k_moe_router_route<GL, GIT>), dim3(gx + (poll ? 1 : 0), a.nwin), dim3(RR_THREADS), lds, st, a,
                      row_wgs, poll ? gx : -1);
   return hipGetLastError();
+}
+
+template <int GL, int GIT>
+static hipError_t gate_batch_go(const MoeArgs& a, hipStream_t st) {
+  const size_t lds = (size_t)MAX_TOKENS * (a.H / 32) * XP_DW * 4;
+  static size_t cur = 0;
+  const hipError_t e = ensure_lds(k_moe_gate_batch<GL, GIT>, lds, cur);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((k_moe_gate_batch<GL, GIT>), dim3((a.M + MAX_TOKENS - 1) / MAX_TOKENS), dim3(RR_THREADS), lds, st, a);
+  return hipGetLastError();
+}
+
+template <int NIT, bool EXACT, int RW>
+static hipError_t router_batch_go(const MoeArgs& a, hipStream_t st) {
+  const int rows = a.sg_w ? a.E : a.E + 1, rg = (rows + 4 * RW - 1) / (4 * RW);
+  // two workgroups per CU, each its rows' weights once: the tokens in as many ranges as that takes
+  const int split = std::max(1, 512 / rg);
+  const int per = ((a.M + split - 1) / split + RB_TOK - 1) / RB_TOK * RB_TOK;
+  const size_t lds = (size_t)2 * RB_TOK * a.H * 2;
+  static size_t cur = 0;
+  const hipError_t e = ensure_lds(k_moe_router_batch<NIT, EXACT, RW>, lds, cur);
+  if (e != hipSuccess) return e;
+  hipLaunchKernelGGL((k_moe_router_batch<NIT, EXACT, RW>), dim3(rg, (a.M + per - 1) / per), dim3(256), lds, st, a, per);
+  return hipGetLastError();
+}
+
+hipError_t launch_moe_route_batch(const MoeArgs& a, hipStream_t st) {
+  if (a.M <= MAX_TOKENS || a.H % 8 != 0 || a.H / 8 > ROUTER_IT * 64 || !a.xp_ready) return hipErrorInvalidValue;
+  hipError_t e = a.H / 8 == 5 * 64 ? router_batch_go<5, true, 4>(a, st) : router_batch_go<ROUTER_IT, false, 1>(a, st);
+  if (e != hipSuccess) return e;
+  const dim3 grid((a.M + MAX_TOKENS - 1) / MAX_TOKENS);
+  if (a.E <= 512)
+    hipLaunchKernelGGL(k_moe_route_batch<8>, grid, dim3(RR_THREADS), 0, st, a);
+  else
+    hipLaunchKernelGGL(k_moe_route_batch<16>, grid, dim3(RR_THREADS), 0, st, a);
+  if ((e = hipGetLastError()) != hipSuccess || !a.sg_w) return e;
+  const int nb = a.H / 32, L = lanes_for_blocks(nb);
+  if (a.H % 32 != 0 || nb > L * QMV_IT) return hipErrorInvalidValue;
+  if (L == 16 && nb == 80) return gate_batch_go<16, 5>(a, st);
+  switch (L) {
+    case 1: return gate_batch_go<1, 0>(a, st);
+    case 2: return gate_batch_go<2, 0>(a, st);
+    case 4: return gate_batch_go<4, 0>(a, st);
+    case 8: return gate_batch_go<8, 0>(a, st);
+    case 16: return gate_batch_go<16, 0>(a, st);
+    case 32: return gate_batch_go<32, 0>(a, st);
+    default: return gate_batch_go<64, 0>(a, st);
+  }
 }
 
 hipError_t launch_moe_router_route(const MoeArgs& a, hipStream_t st) {
@@ -964,15 +1164,15 @@ hipError_t launch_moe_combine(const MoeArgs& a, hipStream_t st) {
 
 
 // ---------------------------------------------------------------------------
-// The batch's expert order (one workgroup): every window's slots grouped by expert -- the
+// The batch's expert order (one workgroup): its slots grouped by expert -- the
 // shared expert's slots first, then each routed expert's -- by a counting sort over the routes'
-// expert ids (a.idx of all windows, consecutive).  The order inside an expert's group follows the
+// expert ids.  The order inside an expert's group follows the
 // atomics and is free: every slot's outputs are its own.
 constexpr int SORT_THREADS = 1024;
 
 __global__ __launch_bounds__(SORT_THREADS) void k_moe_sort(MoeArgs a) {
   __shared__ int cnt[1024], base[1024], cbase[1024];
-  const int E = a.E, K = a.K, M = a.M, T = a.nwin * M, wslots = M * (K + 1);
+  const int E = a.E, K = a.K, T = a.M;
   for (int e = threadIdx.x; e < E; e += SORT_THREADS) cnt[e] = 0;
   __syncthreads();
   for (int i = threadIdx.x; i < T * K; i += SORT_THREADS) atomicAdd(&cnt[min(max(a.idx[i], 0), E - 1)], 1);
@@ -1001,6 +1201,10 @@ __global__ __launch_bounds__(SORT_THREADS) void k_moe_sort(MoeArgs a) {
       crun += __shfl(cincl, 63, 64);
     }
     if (threadIdx.x == 0 && a.chunk_n) *a.chunk_n = crun;
+    int nu = 0;  // distinct routed experts of the batch
+    for (int e = threadIdx.x; e < E; e += 64) nu += cnt[e] > 0;
+    nu = fold_sum_i<32>(nu);
+    if (threadIdx.x == 0) a.disp->n_unique = nu;
   }
   __syncthreads();
   if (a.chunks) {  // chunks of at most MQ_CHUNK slots of one expert: (order position, count | (expert + 1) << 16)
@@ -1015,18 +1219,16 @@ __global__ __launch_bounds__(SORT_THREADS) void k_moe_sort(MoeArgs a) {
       }
     __syncthreads();  // base[] is the scatter's cursor below
   }
-  for (int t = threadIdx.x; t < T; t += SORT_THREADS)  // shared slots: window t / M, slot M*K + t % M
-    a.gorder[t] = (t / M) * wslots + M * K + t % M;
+  for (int t = threadIdx.x; t < T; t += SORT_THREADS) a.gorder[t] = T * K + t;  // the shared expert's slots
   for (int i = threadIdx.x; i < T * K; i += SORT_THREADS) {
     const int e = min(max(a.idx[i], 0), E - 1);
-    const int t = i / K, k = i % K;
     const int pos = atomicAdd(&base[e], 1);
-    a.gorder[pos] = ((t / M) * wslots + (t % M) * K + k) | ((e + 1) << 16);
+    a.gorder[pos] = i | ((e + 1) << 16);
   }
 }
 
 hipError_t launch_moe_sort(const MoeArgs& a, hipStream_t st) {
-  if (!a.gorder || a.E > 1024 || (size_t)a.nwin * a.M * (a.K + 1) > 0xffff) return hipErrorInvalidValue;
+  if (!a.gorder || a.nwin != 1 || a.E > 1024 || (size_t)a.M * (a.K + 1) > 0xffff) return hipErrorInvalidValue;
   hipLaunchKernelGGL(k_moe_sort, dim3(1), dim3(SORT_THREADS), 0, st, a);
   return hipGetLastError();
 }
@@ -1044,13 +1246,12 @@ static hipError_t gate_up_dd_pk(const MoeArgs& a, hipStream_t st) {
                             : ensure_lds(k_moe_gate_up_dd<L, IT, PK, false>, lds, cur);
     if (e != hipSuccess) return e;
     if (a.F % dd_gate_up_rows<L>() != 0) return hipErrorInvalidValue;
-    const int nw = a.gorder ? 1 : a.nwin;  // the global order: every window's units in one row of the grid
-    const int units = a.M * (a.K + 1) * (a.gorder ? a.nwin : 1) * (a.F / dd_gate_up_rows<L>());
+    const int units = a.M * (a.K + 1) * (a.F / dd_gate_up_rows<L>());
     // the global order reads an expert's rows once per slot of the batch, side by side on one XCD: cached loads
     if (a.gorder)
-      hipLaunchKernelGGL((k_moe_gate_up_dd<L, IT, PK, true>), dim3((units + 7) / 8 * 8, nw), dim3(DD_THREADS), lds, st, a);
+      hipLaunchKernelGGL((k_moe_gate_up_dd<L, IT, PK, true>), dim3((units + 7) / 8 * 8), dim3(DD_THREADS), lds, st, a);
     else
-      hipLaunchKernelGGL((k_moe_gate_up_dd<L, IT, PK, false>), dim3((units + 7) / 8 * 8, nw), dim3(DD_THREADS), lds, st, a);
+      hipLaunchKernelGGL((k_moe_gate_up_dd<L, IT, PK, false>), dim3((units + 7) / 8 * 8), dim3(DD_THREADS), lds, st, a);
     return hipGetLastError();
   }
 }
@@ -1063,13 +1264,12 @@ static hipError_t gate_up_dd_li(const MoeArgs& a, hipStream_t st) {
 template <int L, int IT, bool PK>
 static hipError_t down_dd_pk(const MoeArgs& a, hipStream_t st) {
   const size_t lds = (size_t)(a.F / 32) * XP_DW * 4;
-  const int nw = a.gorder ? 1 : a.nwin;
-  const int slots = a.M * (a.K + 1) * (a.gorder ? a.nwin : 1);
+  const int slots = a.M * (a.K + 1);
   auto go = [&](auto kern, size_t& cur, int dr, int nthr) {
     hipError_t e = ensure_lds(kern, lds, cur);
     if (e != hipSuccess) return e;
     const int units = slots * ((a.H + dr - 1) / dr);
-    hipLaunchKernelGGL(kern, dim3((units + 7) / 8 * 8, nw), dim3(nthr), lds, st, a);
+    hipLaunchKernelGGL(kern, dim3((units + 7) / 8 * 8), dim3(nthr), lds, st, a);
     return hipGetLastError();
   };
   static size_t c4 = 0, c8 = 0;

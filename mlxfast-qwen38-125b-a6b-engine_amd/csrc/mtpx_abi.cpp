@@ -231,19 +231,27 @@ int moe_check(const mtpx_moe_weights* w, int M) {
   return MTPX_OK;
 }
 
+// A prefill batch whose slots run in one expert order (else: windows of MAX_TOKENS).
+bool moe_batch_ok(const mtpx_moe_weights* w, int S) {
+  return S > MAX_TOKENS && moe_dd_supported(w->hidden, w->expert_width, w->top_k) && w->experts <= 1024 &&
+         (size_t)S * (w->top_k + 1) <= 0xffff;
+}
+
+// M tokens (more than MAX_TOKENS: a batch), or nwin windows of M.
 size_t moe_ws_bytes(const mtpx_moe_weights* w, int M, int nwin = 1) {
   const int H = w->hidden, E = w->experts, K = w->top_k, F = w->expert_width;
   const size_t T = (size_t)M * nwin, slots = T * (K + 1);
   return al(4 * T * E) + al(4 * T) + al(4 * T * K) * 2 + al(sizeof(MoeDispatch) * (size_t)nwin) +
          al(4 * T * (H / 32) * XP_DW) + al(2 * slots * F) + al(2 * slots * H) +
-         (nwin > 1 ? al(4 * slots) + al(8 * (size_t)moe_max_chunks((int)T, E, K)) + al(4) +
-                         al(xl_bytes((int)T, H)) + al(xl_bytes((int)slots, F))
-                   : 0) +
+         (M > MAX_TOKENS ? al(4 * slots) + al(8 * (size_t)moe_max_chunks(M, E, K)) + al(4) + al(xl_bytes(M, H)) +
+                               al(xl_bytes((int)slots, F))
+                         : 0) +
          4096;
 }
 
 // Workspace of S tokens through moe_enqueue_windows (its launches reuse one region in turn).
 size_t moe_windows_ws_bytes(const mtpx_moe_weights* w, int S) {
+  if (moe_batch_ok(w, S)) return moe_ws_bytes(w, S);
   const int full = S / MAX_TOKENS < MOE_TICKETS ? S / MAX_TOKENS : MOE_TICKETS, tail = S % MAX_TOKENS;
   return std::max(full ? moe_ws_bytes(w, MAX_TOKENS, full) : (size_t)0, tail ? moe_ws_bytes(w, tail) : (size_t)0);
 }
@@ -290,16 +298,20 @@ int moe_enqueue(Ctx* c, const mtpx_moe_weights* w, const uint16_t* x, int M, uin
   a.resid = resid;
   a.y2 = y2;
   a.ticket = c->tickets;
-  a.pub = nwin == 1 ? c->route_pub : nullptr;
+  a.pub = nwin == 1 && M <= MAX_TOKENS ? c->route_pub : nullptr;
   a.nu_out = nu_out;
   c->last_disp = a.disp;
   c->last_H = a.H;
   c->last_E = a.E;
   c->last_F = a.F;
   c->last_gs = a.gs;
-  LAUNCH(c, "moe_router_route", launch_moe_router_route(a, c->stream));
+  const bool batch = M > MAX_TOKENS;
+  if (batch)
+    LAUNCH(c, "moe_route_batch", launch_moe_route_batch(a, c->stream));
+  else
+    LAUNCH(c, "moe_router_route", launch_moe_router_route(a, c->stream));
   if (moe_dd_supported(a.H, a.F, a.K)) {  // one workgroup per (slot, row block), slots in dispatch order
-    if (nwin > 1) {  // a batch of windows: one order of all their slots, grouped by expert
+    if (batch) {  // one order of its slots, grouped by expert
       a.gorder = ws_take<int32_t>(c, slots);
       a.chunks = ws_take<int32_t>(c, 2 * (size_t)moe_max_chunks((int)T, a.E, a.K));
       a.chunk_n = ws_take<int32_t>(c, 1);
@@ -333,11 +345,13 @@ int moe_enqueue(Ctx* c, const mtpx_moe_weights* w, const uint16_t* x, int M, uin
   return MTPX_OK;
 }
 
-// S tokens of a prefill batch through the MoE block as windows of MAX_TOKENS tokens, routed and
-// computed as separate windows would be (each token's output is the window's): the full windows
-// in one batched launch per kernel, the remaining tokens as one more window.
+// S tokens of a prefill batch through the MoE block, each token's output that of a window of
+// MAX_TOKENS: the whole batch in one expert order where its kernels take the geometry, else the full
+// windows in one batched launch per kernel and the remaining tokens as one more window.
 int moe_enqueue_windows(Ctx* c, const mtpx_moe_weights* w, const uint16_t* x, int S, uint16_t* y,
                         uint32_t* xp_ready) {
+  if (moe_batch_ok(w, S))
+    return moe_enqueue(c, w, x, S, y, nullptr, nullptr, nullptr, nullptr, nullptr, xp_ready);
   const int full = S / MAX_TOKENS, tail = S % MAX_TOKENS, H = w->hidden;
   const size_t mark = c->ws_used;
   int rc;

@@ -133,12 +133,12 @@ struct MoeArgs {
   // ROUTE_SENTINEL at rest (the route puts it back), polled by the route; null: the ticket
   float* pub = nullptr;
   int32_t* nu_out;     // if set: the route also writes the distinct routed expert count here
-  // windows of M tokens in one launch (a prefill batch): window w's tokens, slots, dispatch table,
-  // ticket and count follow window w-1's, each window routed and computed as its own launch would
+  // windows of M tokens in one launch: window w's tokens, slots, dispatch table, ticket and count follow
+  // window w-1's, each window routed and computed as its own launch would
   int nwin = 1;
-  // with nwin > 1: all windows' slots in one order grouped by expert (entry = global slot
-  // w * M * (K + 1) + slot | (expert + 1) << 16), walked by the expert kernels in one 1-D grid, so
-  // an expert's weight rows are fetched once for the whole batch; null: each window's own table
+  // a prefill batch (M tokens, more than a window, nwin = 1): its slots in one order grouped by expert
+  // (entry = slot | (expert + 1) << 16), walked by the expert kernels, so an expert's weight rows are
+  // fetched once for the whole batch; null: the window's own table
   int32_t* gorder = nullptr;
   // with gorder: the order cut into chunks of at most MQ_CHUNK slots of one expert (k_moe_sort):
   // chunks[c] = (gorder position, count | (expert + 1) << 16, 0 the shared expert), *chunk_n of
@@ -177,6 +177,8 @@ constexpr int MAX_EXPERTS = 1024;
 // bits zero) or the default NaN's.
 constexpr uint32_t ROUTE_SENTINEL = 0xffffffffu;
 constexpr int ROUTE_SPIN = 1 << 20;  // polls of the publish buffer before the route goes on regardless
+// A batch (more than MAX_TOKENS tokens, xp_x ready): logits, gate_logit, idx and w of every token.
+hipError_t launch_moe_route_batch(const MoeArgs& a, hipStream_t st);
 hipError_t launch_moe_router_route(const MoeArgs& a, hipStream_t st);
 hipError_t launch_moe_gate_up(const MoeArgs& a, hipStream_t st);
 hipError_t launch_moe_down(const MoeArgs& a, hipStream_t st);

@@ -1,0 +1,56 @@
+"""The MoE block of a prefill batch (its own router launch, one expert order for all its tokens), bit-exact against the
+same positions in windows of 8: one position more than a window, a tail that is no window, expert counts that do not
+fill a wave's or a workgroup's rows, the largest counts, both widths of the router launch, and the shared expert's gate
+as a bf16 row and as a q4 row."""
+import numpy as np
+import pytest
+
+pytestmark = pytest.mark.gpu
+
+from gpu_util import dev, empty_bf16, host, need_gpu, rand_bf16  # noqa: E402
+
+
+@pytest.fixture(scope="module")
+def ctx():
+    need_gpu()
+    import mtpx
+    c = mtpx.Context(0)
+    yield c
+    c.close()
+
+
+@pytest.mark.parametrize("H,E,K,n,q4", [
+    (256, 16, 4, 9, False), (256, 1024, 16, 37, True), (256, 31, 1, 255, False), (2560, 33, 3, 13, True),
+    (2560, 520, 10, 30, False), (2560, 16, 10, 70, False)])
+def test_moe_batch_matches_windows(ctx, H, E, K, n, q4):
+    import mtpx
+    layer = dict(hidden=H, experts=E, top_k=K, expert_width=128, group_size=32, heads=4, kv_heads=2, head_dim=64,
+                 rot_dims=16, index_dim=32, rope_theta=1e7, eps=1e-6, max_positions=256)
+    hc, V = 4, 1000
+    cfg = mtpx.HeadConfig(mtpx.LayerConfig(**layer), hc, 64, V, 500, 980)
+    head = mtpx.MTPHead(ctx, cfg, seed=31 + n)
+    r = np.random.default_rng(E + n)
+    used = head
+    if q4:
+        w = head.weights()
+        row = [dev(r.integers(0, 2 ** 32, (1, H // 8), dtype=np.uint32).view(np.int32)),
+               dev(rand_bf16(r, (1, H // 32), 0.01)), dev(rand_bf16(r, (1, H // 32), 0.05))]
+        m = w.layer.moe
+        m.shared_gate, m.shared_gate_sb = None, None
+        m.shared_gate_w, m.shared_gate_s, m.shared_gate_b = (t.data_ptr() for t in row)
+        used = mtpx.MTPHead.adopt(ctx, cfg, w)
+    W = hc * H
+    ids, multi = dev(r.integers(0, V, n).astype(np.int32)), dev(rand_bf16(r, (n, W)))
+    kva, kvb = (mtpx.KVCache(ctx, 2, 64, 256) for _ in range(2))
+    print("case MoE batch", H, E, K, n, q4, flush=True)
+    got, want = empty_bf16(n, W), empty_bf16(n, W)
+    used.forward(kva, ids, multi, got)
+    for w0 in range(0, n, 8):
+        w1 = min(n, w0 + 8)
+        used.forward(kvb, ids[w0:w1], multi[w0:w1], want[w0:w1])
+    assert np.array_equal(host(got), host(want))
+    kva.close()
+    kvb.close()
+    if used is not head:
+        used.close()
+    head.close()
