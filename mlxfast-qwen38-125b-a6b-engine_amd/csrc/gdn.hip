@@ -394,11 +394,13 @@ __global__ __launch_bounds__(GDN_THREADS) void k_gdn_prep_batch(GdnArgs a, GdnBa
 }
 
 // Sixteen workgroups of four waves per value head, one state row per half-wave (768 workgroups at 48
-// heads: three per CU, three waves per SIMD).  A step is a chain of about 45 instructions per row, most of
-// them issue-bound at that occupancy; the gated norm is a launch of its own (a head's last workgroup
-// running it for the whole batch was a serial tail of about a quarter of the launch), and the outputs
-// stay in registers, one step per lane, until 32 of them go out as one 128-byte store.  512 positions,
-// 48 heads: 438 us with the norm in the launch, eight workgroups of 16 half-waves per head -> 157 + 10 us.
+// heads: three per CU, three waves per SIMD).  A step is about 45 vector instructions per row pair, at four
+// cycles each and three waves 540 cycles a position: what it takes (575 measured).  So the rows' output sums
+// of two positions share their fold (the first level puts one position in the lower, the other in the upper
+// 16 lanes), the outputs stay in registers until 32 of them go out as one 128-byte store, and the gated norm
+// is a launch of its own.  1003 positions, 48 heads: 333 us with a fold per position and the staged rows in
+// an array (the compiler kept it in scratch, so the prefetch waited for its loads) -> 275 us; two rows per
+// half-wave, sharing the k and q reads and both folds, 315 us (1.5 waves per SIMD do not spread evenly).
 __global__ __launch_bounds__(GDN_BTHREADS) void k_gdn_batch(GdnArgs a, GdnBatch b) {
   constexpr int W = GDN_BWIN, RW = GDN_D / GDN_BSPLIT;  // staged positions; state rows of a workgroup
   static_assert(RW == GDN_BTHREADS / 32 && 2 * GDN_BWIN == 32, "a row per half-wave, two windows per output store");
@@ -413,28 +415,27 @@ __global__ __launch_bounds__(GDN_BTHREADS) void k_gdn_batch(GdnArgs a, GdnBatch 
   const size_t pstride = (size_t)(2 * a.hk + a.hv) * GDN_D;
   // staged per window: q and k [W][128] as float4 units (thread -> position tid / 32 + 8 k, float4 l),
   // v of this workgroup's rows [W][RW] and the gates [W][2] (position clamped: past S loaded, not used)
-  constexpr int U = W * GDN_D / 4 / GDN_BTHREADS;
+  constexpr int TP = GDN_BTHREADS / 32;
+  static_assert(W == 2 * TP, "two positions per half-wave (named registers: an array of them went to scratch)");
   const float* qsrc = b.vecs + (size_t)hk * GDN_D + 4 * l;
   const float* ksrc = qsrc + (size_t)a.hk * GDN_D;
   const float* vsrc = b.vecs + (size_t)(2 * a.hk + h) * GDN_D + r0 + (tid & (RW - 1));
-  float4 pq[U], pk[U];
+  float4 pq0, pq1, pk0, pk1;
   float pv, pg;
   auto fetch = [&](int t0) {
-#pragma unroll
-    for (int k = 0; k < U; ++k) {
-      const size_t t = (size_t)min(t0 + hw + k * (GDN_BTHREADS / 32), S - 1) * pstride;
-      pq[k] = *reinterpret_cast<const float4*>(qsrc + t);
-      pk[k] = *reinterpret_cast<const float4*>(ksrc + t);
-    }
+    const size_t ta = (size_t)min(t0 + hw, S - 1) * pstride, tb = (size_t)min(t0 + hw + TP, S - 1) * pstride;
+    pq0 = *reinterpret_cast<const float4*>(qsrc + ta);
+    pk0 = *reinterpret_cast<const float4*>(ksrc + ta);
+    pq1 = *reinterpret_cast<const float4*>(qsrc + tb);
+    pk1 = *reinterpret_cast<const float4*>(ksrc + tb);
     pv = vsrc[(size_t)min(t0 + (tid / RW) % W, S - 1) * pstride];
     pg = b.gates[((size_t)min(t0 + (tid >> 1) % W, S - 1) * a.hv + h) * 2 + (tid & 1)];
   };
   auto store = [&](int buf) {
-#pragma unroll
-    for (int k = 0; k < U; ++k) {
-      *reinterpret_cast<float4*>(&qs[buf][hw + k * (GDN_BTHREADS / 32)][4 * l]) = pq[k];
-      *reinterpret_cast<float4*>(&ks[buf][hw + k * (GDN_BTHREADS / 32)][4 * l]) = pk[k];
-    }
+    *reinterpret_cast<float4*>(&qs[buf][hw][4 * l]) = pq0;
+    *reinterpret_cast<float4*>(&ks[buf][hw][4 * l]) = pk0;
+    *reinterpret_cast<float4*>(&qs[buf][hw + TP][4 * l]) = pq1;
+    *reinterpret_cast<float4*>(&ks[buf][hw + TP][4 * l]) = pk1;
     if (tid < W * RW) vs[buf][tid / RW][tid % RW] = pv;
     if (tid < 2 * W) (tid & 1 ? bet : dec)[buf][tid >> 1] = pg;
   };
@@ -460,8 +461,8 @@ __global__ __launch_bounds__(GDN_BTHREADS) void k_gdn_batch(GdnArgs a, GdnBatch 
       s[c] = __builtin_fmaf(kp[c], dl, s[c]);
     }
   }
-  // one position: the step kernel's operations in its order
-  auto step = [&](int buf, int t, int lane_t, float& yb) {
+  // one position: the step kernel's operations in its order, the row's q dot before its sum over the lanes
+  auto step = [&](int buf, int t) -> float {
     const float gd = dec[buf][t], bt = bet[buf][t], v = vs[buf][t][hw];
     const float4 k = *reinterpret_cast<const float4*>(&ks[buf][t][4 * l]);
     const float4 q = *reinterpret_cast<const float4*>(&qs[buf][t][4 * l]);
@@ -488,26 +489,38 @@ __global__ __launch_bounds__(GDN_BTHREADS) void k_gdn_batch(GdnArgs a, GdnBatch 
     float o = __builtin_fmaf(s[0], q.x, 0.0f);
     o = __builtin_fmaf(s[1], q.y, o);
     o = __builtin_fmaf(s[2], q.z, o);
-    o = __builtin_fmaf(s[3], q.w, o);
-    const float y = half_wave_sum(o);
-    yb = l == lane_t ? y : yb;
+    return __builtin_fmaf(s[3], q.w, o);
+  };
+  // half_wave_sum of two positions' dots: the first level puts x in the lower 16 lanes, y in the upper
+  auto fold2 = [](float x, float y) {
+    const auto p = __builtin_amdgcn_permlane16_swap(__float_as_uint(x), __float_as_uint(y), false, false);
+    return fold_sum<8>(__uint_as_float(p[0]) + __uint_as_float(p[1]));
   };
   const int sp = (S + 31) & ~31;  // padded positions of an output row
   float* yrow = a.ypub + ((size_t)h * GDN_D + r) * sp;
   store(0);
   __syncthreads();
-  float yb = 0.0f;
+  float yb = 0.0f;  // lane l of a row: position 2 (l & 15) + l / 16 of 32
   for (int t0 = 0, buf = 0; t0 < S; t0 += W, buf ^= 1) {
     const bool more = t0 + W < S;
     if (more) fetch(t0 + W);  // in flight during this window's recurrence
-    const int base = t0 & W;  // the window's lanes: 0 .. 15 or 16 .. 31
+    const int base = (t0 & W) / 2;  // the window's pairs: 0 .. 7 or 8 .. 15
     if (t0 + W <= S) {
-#pragma unroll 4
-      for (int t = 0; t < W; ++t) step(buf, t, base + t, yb);
+#pragma unroll 2
+      for (int t = 0; t < W; t += 2) {
+        const float o0 = step(buf, t), o1 = step(buf, t + 1);
+        const float y = fold2(o0, o1);
+        yb = (l & 15) == base + t / 2 ? y : yb;
+      }
     } else {
-      for (int t = 0; t < S - t0; ++t) step(buf, t, base + t, yb);
+      for (int t = 0; t < S - t0; t += 2) {
+        const float o0 = step(buf, t);
+        const float o1 = t + 1 < S - t0 ? step(buf, t + 1) : 0.0f;  // (a position past S: the row's pad)
+        const float y = fold2(o0, o1);
+        yb = (l & 15) == base + t / 2 ? y : yb;
+      }
     }
-    if (base != 0 || !more) yrow[(t0 & ~31) + l] = yb;
+    if (base != 0 || !more) yrow[(t0 & ~31) + 2 * (l & 15) + (l >> 4)] = yb;
     if (more) store(buf ^ 1);  // the other buffer: last read in the previous window, before its barrier
     __syncthreads();
   }
