@@ -770,7 +770,11 @@ __global__ __launch_bounds__(256) void k_attn_pv(const float* __restrict__ sc, i
 }
 
 bool attn_batch_ok(int S, int HQ, int HK, int D, int T) {
-  return S > MAX_TOKENS && D == PP_D && HQ % HK == 0 && T <= PV_MAXCH * ATTN_CHUNK;
+  // A row walks its chunks one after the other, so with few workgroups the (chunk, kv head, query) launch is
+  // faster at every cache length, and with many this one is (a head step of 24 heads, us by rows / by chunks: 64
+  // queries after 1 / 700 / 1500 positions 752 / 742, 841 / 806, 941 / 890; 128 queries 957 / 973, 1049 / 1093,
+  // 1179 / 1266; 16 queries after 700 650 / 565).
+  return S * HQ >= 96 * PV_ROWS && S > MAX_TOKENS && D == PP_D && HQ % HK == 0 && T <= PV_MAXCH * ATTN_CHUNK;
 }
 
 size_t attn_batch_floats(int S, int HQ, int T) { return (size_t)S * HQ * ((T + 31) & ~31); }
@@ -780,8 +784,8 @@ hipError_t launch_attn_batch(const bf16* q, int S, int HQ, int HK, const bf16* k
                              uint32_t* xp_gated, hipStream_t st) {
   if (!attn_batch_ok(S, HQ, HK, PP_D, T) || T < S) return hipErrorInvalidValue;
   const int R = S * (HQ / HK), TP = (T + 31) & ~31;
-  // tiles of 64 rows x 64 keys where those of 128 would not give each CU one: 75 queries
-  // (16 tiles of 128) 44 us with the large tile, 17 us with the small
+  // tiles of 64 rows x 64 keys where those of 128 would not give each CU one (75 queries of 24 heads, 16 tiles
+  // of 128: 44 us with the large tile, 17 us with the small)
   const auto tiles = [&](int t) { return dim3((R + t - 1) / t, (T + t - 1) / t, HK); };
   const dim3 big = tiles(128);
   if (big.x * big.y * big.z < 256)

@@ -210,7 +210,7 @@ hipError_t launch_attn_partial(const bf16* q, int S, int HQ, int HK, int D, cons
                                int64_t tmax, int T, float scale, float* part, hipStream_t st);
 hipError_t launch_attn_combine(int S, int HQ, int HK, int D, int T, const float* part, const bf16* qkv, int QW,
                                int gate_off, bf16* out, bf16* out_gated, uint32_t* xp_gated, hipStream_t st);
-// A prefill batch (S > MAX_TOKENS, head dim 256, T <= 2048): scores [HQ][S][T rounded up to 32] in the
+// A prefill batch (enough queries, head dim 256, T <= 2048): scores [HQ][S][T rounded up to 32] in the
 // workspace, then the gated output rows (and their prepared blocks where xp_gated is not null).
 bool attn_batch_ok(int S, int HQ, int HK, int D, int T);
 size_t attn_batch_floats(int S, int HQ, int T);

@@ -1,7 +1,7 @@
 """The attention of a prefill batch (head dim 256, more than a window of positions: scores in one launch,
 the chunks of 32 keys folded per row in another), bit-exact against the same positions in windows of 8:
-query counts around the 128-row and 24-row tiles, prefixes around a chunk's and a tile's edge, group sizes
-1, 6 and 12, the last keys that a cache of 2048 holds, and keys whose scores are infinite or NaN (such a
+query counts around the least that takes it (96 at 24 heads), ragged row tiles, prefixes around a chunk's and
+a tile's edge, group sizes 1, 2, 8 and 12, the last keys that a cache of 2048 holds, and keys whose scores are infinite or NaN (such a
 chunk adds nothing to any query that sees it)."""
 import numpy as np
 import pytest
@@ -21,9 +21,9 @@ def ctx():
 
 
 @pytest.mark.parametrize("HQ,HK,pre,n,odd", [
-    (6, 1, 0, 17, False), (6, 1, 31, 33, False), (4, 4, 96, 32, False), (4, 4, 127, 129, False),
-    (12, 1, 33, 23, False), (12, 2, 1792, 256, False), (12, 2, 2001, 47, False), (6, 1, 40, 90, True),
-    (4, 2, 257, 200, True)])
+    (24, 2, 0, 96, False), (24, 2, 31, 95, False), (24, 24, 33, 97, False), (12, 12, 127, 193, False),
+    (32, 4, 96, 73, False), (12, 1, 1792, 256, False), (24, 2, 1900, 148, False), (24, 2, 40, 101, True),
+    (16, 8, 257, 200, True)])
 def test_attention_batch_matches_windows(ctx, HQ, HK, pre, n, odd):
     import mtpx
     layer = dict(hidden=256, experts=16, top_k=4, expert_width=128, group_size=32, heads=HQ, kv_heads=HK,
