@@ -607,9 +607,9 @@ int mtpx_target_commit(mtpx_target_state st, int n);
  * equal those of verifying and committing the tokens in windows of 8 in turn; the work runs over
  * batches of up to 1024 positions at once: one launch per kernel for the whole batch where each
  * position's result is its own (the dense projections as GEMMs on the matrix cores, norms, mixers,
- * attention -- every query attends to the keys up to its own position --, the MoE routed as windows
- * of 8 and its experts over the batch's slots sorted by expert, the GDN recurrence over the batch),
- * the PLE recurrence window by window.  Replaces the runner's prompt prefill windows (Runner/FastModel/TrackP12Prefill.swift:1-237,
+ * attention -- every query attends to the keys up to its own position --, the MoE over the batch's
+ * slots sorted by expert, the GDN recurrence over the batch), the PLE recurrence window by window.
+ * Replaces the runner's prompt prefill windows (Runner/FastModel/TrackP12Prefill.swift:1-237,
  * TrackPrefillSort.swift:1-201, TrackPrefillIndirect.swift:5-227), with the decode path's arithmetic
  * instead of MLX's steel GEMM: the prompt's positions get the bits the verify path gives them.
  * ids (device int32 [S]) in plain host memory: MTPX_ERR_ARG before anything runs. */

@@ -1,8 +1,8 @@
 """The attention of a prefill batch (head dim 256, more than a window of positions: scores in one launch,
 the chunks of 32 keys folded per row in another), bit-exact against the same positions in windows of 8:
 query counts around the least that takes it (96 at 24 heads), ragged row tiles, prefixes around a chunk's and
-a tile's edge, group sizes 1, 2, 8 and 12, the last keys that a cache of 2048 holds, and keys whose scores are infinite or NaN (such a
-chunk adds nothing to any query that sees it)."""
+a tile's edge, group sizes 1, 2, 8 and 12, the last keys that a cache of 2048 holds, and keys whose scores are
+infinite or NaN (such a chunk adds nothing to any query that sees it)."""
 import numpy as np
 import pytest
 
