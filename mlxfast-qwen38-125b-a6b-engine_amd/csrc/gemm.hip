@@ -46,11 +46,11 @@ typedef __bf16 bf16x8_t __attribute__((ext_vector_type(8)));
 typedef float f32x4_t __attribute__((ext_vector_type(4)));
 
 // The limb form of a batch (XlBatch), from x [M][K]: xl [M][nb][3][32] bf16, sx and xr [M][nb], big
-// [M][ceil(nb / XL_PART)] (nonzero somewhere in a token's if any of its blocks is above XL_EMAX).  One
-// workgroup per token and part.  (One workgroup per token: 17 us at 75 tokens of K = 10240.)
+// [M][XL_FLAGS] (nonzero somewhere in a token's if any of its blocks is above XL_EMAX).  One workgroup per
+// token and part.  (One workgroup per token: 17 us at 75 tokens of K = 10240.)
 __global__ __launch_bounds__(256) void k_xlimb(const bf16* __restrict__ x, int nb, uint32_t* __restrict__ xl,
                                                float* __restrict__ sx, float* __restrict__ xr,
-                                               uint32_t* __restrict__ big) {
+                                               uint8_t* __restrict__ big) {
   const size_t t = blockIdx.x;
   x += t * nb * 32;
   xl += t * nb * 48;
@@ -62,13 +62,12 @@ __global__ __launch_bounds__(256) void k_xlimb(const bf16* __restrict__ x, int n
   for (int j = part * XL_PART + (int)(threadIdx.x >> 5); j < end; j += 8) {
     any |= xlimb_lanes(x[(size_t)j * 32 + i], i, xl + (size_t)j * 48, sx + j, xr + j);
   }
-  any = __syncthreads_or(any);
-  if (threadIdx.x == 0) big[t * gridDim.y + part] = any ? 1u : 0u;
+  xl_flag(big, t, part, gridDim.y, __syncthreads_or(any));
 }
 
 size_t xl_bytes(int M, int K) {
   const size_t nb = K / 32;
-  return (size_t)M * nb * (192 + 8) + 4 * (size_t)M * ((nb + XL_PART - 1) / XL_PART) + 1024;
+  return (size_t)M * nb * (192 + 8) + (size_t)M * XL_FLAGS + 1024;
 }
 
 XlBatch xl_carve(void* ws, int M, int K) {
@@ -82,12 +81,15 @@ XlBatch xl_carve(void* ws, int M, int K) {
   p += up(n * 4);
   b.xr = reinterpret_cast<float*>(p);
   p += up(n * 4);
-  b.big = reinterpret_cast<uint32_t*>(p);
+  b.big = reinterpret_cast<uint8_t*>(p);
   return b;
 }
 
 hipError_t launch_xlimb(const bf16* x, int M, int K, const XlBatch& b, hipStream_t st) {
-  hipLaunchKernelGGL(k_xlimb, dim3(M, (K / 32 + XL_PART - 1) / XL_PART), dim3(256), 0, st, x, K / 32, reinterpret_cast<uint32_t*>(b.xl), b.sx, b.xr, b.big);
+  const int parts = (K / 32 + XL_PART - 1) / XL_PART;
+  if (parts > XL_FLAGS) return hipErrorInvalidValue;
+  hipLaunchKernelGGL(k_xlimb, dim3(M, parts), dim3(256), 0, st, x, K / 32, reinterpret_cast<uint32_t*>(b.xl), b.sx, b.xr,
+                     b.big);
   return hipGetLastError();
 }
 
@@ -309,11 +311,9 @@ __global__ __launch_bounds__(GT_THREADS, MINW) void k_gemm(std::conditional_t<MO
                                                  soff, q * 64, 0, 0);
     }
   };
-  constexpr int NBP = (NB + XL_PART - 1) / XL_PART;
-  uint32_t bigs = 0;
-#pragma unroll
-  for (int p = 0; p < NBP; ++p) bigs |= a.x.big[xrow_n * NBP + p];
-  const bool big = __any(bigs != 0u);
+  static_assert(XL_FLAGS == 16, "a token's flags in one load");
+  const uint4 bigs = reinterpret_cast<const uint4*>(a.x.big)[xrow_n];
+  const bool big = __any((bigs.x | bigs.y | bigs.z | bigs.w) != 0u);
   float acc[RT][4][LC];
 #pragma unroll
   for (int rt = 0; rt < RT; ++rt)

@@ -154,11 +154,7 @@ __global__ __launch_bounds__(256) void k_hc_norm_batch(const bf16* __restrict__ 
     else if (xp)
       xprep_lanes_direct(n, t & 31, xp + b * XP_DW);
   }
-  if (xl.xl) {  // the token's parts: each written by one of its workgroups, with what that one saw
-    any = __syncthreads_or(any);
-    const int parts = (int)(W / 32 + XL_PART - 1) / XL_PART;
-    for (int p = c + hc * t; p < parts; p += 256 * hc) xl.big[(size_t)s * parts + p] = any ? 1u : 0u;
-  }
+  if (xl.xl) xl_flag(xl.big, s, c, hc, __syncthreads_or(any));
 }
 
 // grid (S, ceil(LW/256)), 256 threads; LW % 32 == 0.
@@ -236,6 +232,7 @@ hipError_t launch_hc_norm(const bf16* residual, const bf16* out, const bf16* inj
                           int tile, const bf16* scale, float eps, bf16* stream, bf16* normed, uint32_t* xp,
                           hipStream_t st, const XlBatch* xl) {
   if (S > MAX_TOKENS) {
+    if (xl && hc > XL_FLAGS) return hipErrorInvalidValue;
     const XlBatch x = xl ? *xl : XlBatch{};
     const dim3 grid(hc, S);
     if (H == 2560)

@@ -152,13 +152,22 @@ inline int moe_max_chunks(int T, int E, int K) {
   return (T + MQ_CHUNK - 1) / MQ_CHUNK + E + (T * K + MQ_CHUNK - 1) / MQ_CHUNK;
 }
 // --- batch GEMMs (gemm.hip): more than MAX_TOKENS tokens of the model's depths
-// A batch in limb form (k_xlimb): xl [M][K/32][3][32] bf16, sx and xr [M][K/32], big per token and part of K.
-constexpr int XL_PART = 32;  // blocks of a part
+// A batch in limb form (k_xlimb): xl [M][K/32][3][32] bf16, sx and xr [M][K/32], big [M][XL_FLAGS].
+constexpr int XL_PART = 32;  // blocks of a part of K, a workgroup's of k_xlimb
+// Flag bytes of a token, one load of the GEMM: at least as many as workgroups make a token's blocks (a part of
+// K each, or a stream each).
+constexpr int XL_FLAGS = 16;
 struct XlBatch {
   uint4* xl;
   float *sx, *xr;
-  uint32_t* big;
+  uint8_t* big;
 };
+// Workgroup `who` of the `of` <= XL_FLAGS that make token t's blocks stores what it saw in places who, who + of, ..,
+// so each of the token's flags is written once whatever `of` is.
+__device__ __forceinline__ void xl_flag(uint8_t* big, size_t t, int who, int of, bool any) {
+  const int p = who + of * (int)threadIdx.x;
+  if (p < XL_FLAGS) big[t * XL_FLAGS + p] = any ? 1 : 0;
+}
 size_t xl_bytes(int M, int K);                // workspace of one batch
 XlBatch xl_carve(void* ws, int M, int K);     // its arrays in that workspace (256-byte aligned)
 hipError_t launch_xlimb(const bf16* x, int M, int K, const XlBatch& b, hipStream_t st);

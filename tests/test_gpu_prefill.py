@@ -15,6 +15,7 @@ import torch
 pytestmark = pytest.mark.gpu
 
 from gpu_util import dev, empty_bf16, host, need_gpu, rand_bf16, write_device  # noqa: E402
+from oracle import oracle as O  # noqa: E402
 
 LAYER = dict(hidden=256, experts=16, top_k=4, expert_width=128, group_size=32, heads=4, kv_heads=2, head_dim=64,
              rot_dims=16, index_dim=32, rope_theta=1e7, eps=1e-6, max_positions=700)
@@ -301,6 +302,37 @@ def test_head_batch_at_width_matches_windows(ctx, n):
     kva, kvb = (mtpx.KVCache(ctx, layer["kv_heads"], layer["head_dim"], 64) for _ in range(2))
     print("case head batch at width", n, flush=True)
     na, sa, nb, sb = empty_bf16(n, W), empty_bf16(n, 2560), empty_bf16(n, W), empty_bf16(n, 2560)
+    head.forward(kva, ids, multi, na, sa)
+    for w0 in range(0, n, 8):
+        w1 = min(n, w0 + 8)
+        head.forward(kvb, ids[w0:w1], multi[w0:w1], nb[w0:w1], sb[w0:w1])
+    assert np.array_equal(host(na), host(nb))
+    assert np.array_equal(host(sa), host(sb))
+    kva.close()
+    kvb.close()
+    head.close()
+
+
+# streams x hidden whose mixer depths the batch GEMM takes with fewer parts of K than streams (2560: 3, 6144: 6, the
+# model's 10240: 10)
+@pytest.mark.parametrize("hc,H", [(4, 640), (5, 512), (8, 320), (8, 768), (4, 2560)])
+def test_head_batch_large_last_stream_matches_windows(ctx, hc, H):
+    """Normed rows above 4096 in the last stream alone (its norm scales 1e5 in every mixer): the batch's mixers
+    walk with the blocks' factors whichever stream holds them, bit-equal to windows of 8."""
+    import mtpx
+    layer = dict(LAYER, hidden=H, max_positions=64)
+    head = mtpx.MTPHead(ctx, mtpx.HeadConfig(mtpx.LayerConfig(**layer), hc, 64, 1000, 500, 980), seed=37)
+    w = head.weights()
+    for m in (w.attn_hc, w.mlp_hc, w.final_hc):
+        sc = O.f32_to_bf16(np.ones((hc, H), np.float32))
+        sc[hc - 1] = O.f32_to_bf16(np.full(H, 1e5, np.float32))
+        write_device(m.norm_scale, sc)
+    n, W = 21, hc * H
+    r = np.random.default_rng(H + hc)
+    ids, multi = dev(r.integers(0, 1000, n).astype(np.int32)), dev(rand_bf16(r, (n, W)))
+    kva, kvb = (mtpx.KVCache(ctx, layer["kv_heads"], layer["head_dim"], 64) for _ in range(2))
+    print("case head batch, large last stream", hc, H, flush=True)
+    na, sa, nb, sb = empty_bf16(n, W), empty_bf16(n, H), empty_bf16(n, W), empty_bf16(n, H)
     head.forward(kva, ids, multi, na, sa)
     for w0 in range(0, n, 8):
         w1 = min(n, w0 + 8)
