@@ -203,7 +203,7 @@ __global__ __launch_bounds__(GT_THREADS, MINW) void k_gemm(std::conditional_t<MO
   } else {
     const MoeArgs& m = a.m;
     // units of one chunk side by side on one XCD
-    const int fb = MODE == GT_GATE_UP ? m.F / (R / 2) : m.H / R;  // row blocks
+    const int fb = MODE == GT_GATE_UP ? m.F / (R / 2) : (m.H + R - 1) / R;  // row blocks
     const int n_units = min(*m.chunk_n, m.max_chunks) * fb, per = (n_units + 7) / 8;
     const int unit = (blockIdx.x % 8) * per + blockIdx.x / 8;
     if ((int)blockIdx.x / 8 >= per || unit >= n_units) return;
@@ -524,15 +524,21 @@ hipError_t launch_gemm_pair(const uint32_t* w1, const bf16* s1, const bf16* b1, 
 }
 
 // ---- MoE ----
-bool moe_gemm_ok(const MoeArgs& a) {
-  return gemm_shape(a.H) == 16 * 16 + 5 && gemm_shape(a.F) == 4 * 16 + 5 && a.M * (a.K + 1) < 65536 &&
-         mat_ok(a.gate_w, a.gate_s, a.gate_b) && mat_ok(a.up_w, a.up_s, a.up_b) && mat_ok(a.down_w, a.down_s, a.down_b) &&
-         mat_ok(a.sh_gate_w, a.sh_gate_s, a.sh_gate_b) && mat_ok(a.sh_up_w, a.sh_up_s, a.sh_up_b) &&
+// The model's expert width, at any hidden size (1024 wide, 512 experts top-10, 256 tokens: by slots 157 us, by chunks 64 + 9).
+bool moe_gemm_down_ok(const MoeArgs& a) {
+  return gemm_shape(a.F) == 4 * 16 + 5 && a.M * (a.K + 1) < 65536 && mat_ok(a.down_w, a.down_s, a.down_b) &&
          mat_ok(a.sh_down_w, a.sh_down_s, a.sh_down_b);
 }
 
+// The model's hidden size and expert width.
+bool moe_gemm_gate_up_ok(const MoeArgs& a) {
+  return gemm_shape(a.H) == 16 * 16 + 5 && gemm_shape(a.F) == 4 * 16 + 5 && a.M * (a.K + 1) < 65536 &&
+         mat_ok(a.gate_w, a.gate_s, a.gate_b) && mat_ok(a.up_w, a.up_s, a.up_b) &&
+         mat_ok(a.sh_gate_w, a.sh_gate_s, a.sh_gate_b) && mat_ok(a.sh_up_w, a.sh_up_s, a.sh_up_b);
+}
+
 hipError_t launch_moe_gemm_gate_up(const MoeArgs& m, const XlBatch& x, hipStream_t st) {
-  if (!moe_gemm_ok(m) || !m.gorder || !m.chunks || !m.chunk_n) return hipErrorInvalidValue;
+  if (!moe_gemm_gate_up_ok(m) || !m.gorder || !m.chunks || !m.chunk_n) return hipErrorInvalidValue;
   const MoeGemmArgs a{m, x, (uint32_t)((size_t)m.M * m.H * 6)};
   const int grid = (m.max_chunks * (m.F / 64) + 7) / 8 * 8;
   if (m.gs == 32)
@@ -543,9 +549,9 @@ hipError_t launch_moe_gemm_gate_up(const MoeArgs& m, const XlBatch& x, hipStream
 }
 
 hipError_t launch_moe_gemm_down(const MoeArgs& m, const XlBatch& x, hipStream_t st) {
-  if (!moe_gemm_ok(m) || !m.gorder || !m.chunks || !m.chunk_n) return hipErrorInvalidValue;
+  if (!moe_gemm_down_ok(m) || !m.gorder || !m.chunks || !m.chunk_n) return hipErrorInvalidValue;
   const MoeGemmArgs a{m, x, (uint32_t)((size_t)m.M * (m.K + 1) * m.F * 6)};
-  const int grid = (m.max_chunks * (m.H / 128) + 7) / 8 * 8;
+  const int grid = (m.max_chunks * ((m.H + 127) / 128) + 7) / 8 * 8;
   if (m.gs == 32)
     hipLaunchKernelGGL((k_gemm<GT_DOWN, 4, 5, 4, 4, true, 2, 6>), dim3(grid), dim3(GT_THREADS), 0, st, a);
   else

@@ -317,12 +317,12 @@ int moe_enqueue(Ctx* c, const mtpx_moe_weights* w, const uint16_t* x, int M, uin
       a.chunk_n = ws_take<int32_t>(c, 1);
       a.max_chunks = moe_max_chunks((int)T, a.E, a.K);
       LAUNCH(c, "moe_sort", launch_moe_sort(a, c->stream));
-      if (moe_gemm_ok(a)) {  // the experts over their chunks on the matrix cores
+      if (moe_gemm_down_ok(a)) {  // the experts over their chunks on the matrix cores
         // gate|up: a chunk costs 16 tokens whatever it holds, so below about 2.7 slots per expert the walk of
         // one slot per workgroup is faster (whole prefill of four layers, 128 / 160 tokens of 512 experts
         // top-10: 3515 / 3804 us by chunks, 3487 / 3959 by slots; 75 tokens: 2900 / 2650; 512: 7000 / 9700)
         const XlBatch xt = xl_take(c, (int)T, a.H), xs = xl_take(c, (int)slots, a.F);
-        if (T * a.K * 3 >= (size_t)a.E * 8) {
+        if (moe_gemm_gate_up_ok(a) && T * a.K * 3 >= (size_t)a.E * 8) {
           LAUNCH(c, "xlimb", launch_xlimb(a.x, (int)T, a.H, xt, c->stream));
           LAUNCH(c, "moe_gate_up", launch_moe_gemm_gate_up(a, xt, c->stream));
         } else {

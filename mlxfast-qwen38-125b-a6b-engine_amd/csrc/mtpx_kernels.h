@@ -176,7 +176,8 @@ bool gemm_ok(const uint32_t* w, const bf16* s, const bf16* b, int64_t N, int K, 
 hipError_t launch_gemm_pair(const uint32_t* w1, const bf16* s1, const bf16* b1, int N1, bf16* y1, float* yf1,
                             const uint32_t* w2, const bf16* s2, const bf16* b2, int N2, bf16* y2, int K, int gs,
                             const XlBatch& x, int M, hipStream_t st);
-bool moe_gemm_ok(const MoeArgs& a);
+bool moe_gemm_gate_up_ok(const MoeArgs& a);
+bool moe_gemm_down_ok(const MoeArgs& a);
 hipError_t launch_moe_gemm_gate_up(const MoeArgs& m, const XlBatch& x, hipStream_t st);  // x per token
 hipError_t launch_moe_gemm_down(const MoeArgs& m, const XlBatch& x, hipStream_t st);     // x per slot
 

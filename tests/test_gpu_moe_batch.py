@@ -54,3 +54,32 @@ def test_moe_batch_matches_windows(ctx, H, E, K, n, q4):
     if used is not head:
         used.close()
     head.close()
+
+
+# row blocks of 128 rows of H: whole ones and a last one of 32 rows
+@pytest.mark.parametrize("H,E,K,n,gs", [(1024, 32, 4, 70, 64), (544, 16, 3, 33, 32), (512, 9, 9, 17, 64)])
+def test_expert_down_chunks_at_other_hidden_sizes(ctx, H, E, K, n, gs):
+    """The expert down GEMM at expert width 640 takes any hidden size (the only launch here that reads activations in
+    limb form), bit-equal to windows of 8."""
+    import mtpx
+    lc = mtpx.LayerConfig(H, E, K, 640, gs, 4, 2, 64, 16, 32, 1e7, 1e-6, 256)
+    head = mtpx.MTPHead(ctx, mtpx.HeadConfig(lc, 4, 64, 1000, 500, 980), seed=41 + n)
+    W = 4 * H
+    r = np.random.default_rng(H + n)
+    ids, multi = dev(r.integers(0, 1000, n).astype(np.int32)), dev(rand_bf16(r, (n, W)))
+    kva, kvb = (mtpx.KVCache(ctx, 2, 64, 256) for _ in range(2))
+    print("case expert down", H, E, K, n, gs, flush=True)
+    got, want = empty_bf16(n, W), empty_bf16(n, W)
+    ctx.profile(True)
+    ctx.profile_reset()
+    head.forward(kva, ids, multi, got)
+    launched = ctx.profile_stats()
+    ctx.profile(False)
+    assert launched["moe_route_batch"][0] == 1 and launched["xlimb"][0] == 1, launched
+    for w0 in range(0, n, 8):
+        w1 = min(n, w0 + 8)
+        head.forward(kvb, ids[w0:w1], multi[w0:w1], want[w0:w1])
+    assert np.array_equal(host(got), host(want))
+    kva.close()
+    kvb.close()
+    head.close()
