@@ -103,10 +103,11 @@ __global__ __launch_bounds__(256) void k_hc_norm(const bf16* __restrict__ residu
   if (xp && d < H) xprep_lanes_direct(n, t & 31, xp + (base + d) / 32 * XP_DW);
 }
 
-// The same over a batch: grid (hc, S), a workgroup its whole row of a stream (the launch above loads and
+// The same over many rows: grid (hc, S), a workgroup its whole row of a stream (the launch above loads and
 // folds the row once per 256 elements of it: with thousands of rows that is ten times the work, 85 us at
 // 1003 x 4 rows of 2560, here 47 us with the limb form), and the normed row in limb form instead of xp where xl.xl is set
-// (a pass of 28 us over it saved; 126 MB).
+// (a pass of 28 us over it saved; 126 MB).  What bounds it at few rows: a thread's elements one after the other, about
+// 0.85 us each beyond a base of 3 us (norm_by_row).
 template <int IT, bool EXACT, int MODE>
 __global__ __launch_bounds__(256) void k_hc_norm_batch(const bf16* __restrict__ residual, const bf16* __restrict__ out,
                                                        const bf16* __restrict__ inject, int hc, int H, int tile,
@@ -228,11 +229,21 @@ static void hc_norm_mode(const dim3& grid, const bf16* residual, const bf16* out
                        eps, stream, normed, xp);
 }
 
+// Whether a row per workgroup is faster than a workgroup per 256 elements.  The first takes the chain of a row's
+// elements whatever the number of rows, the second 0.18 ns per row, 256 elements and element a thread loads (10, 16 or
+// 48: the instance's), so the line is a number of rows.  us by row / by 256, 36 .. 1024 rows: 2560 wide 11.2 / 4.2 at 36,
+// 12.6 / 10.6 at 320, 13.4 / 14.0 at 512, 15.7 / 20.4 at 1024; 4096 wide 18.2 / 10.2 at 128, 18.9 / 27.5 at 512;
+// 10240 wide 29.0 / 14.5 at 64, 29.3 / 32.4 at 192.  The limb form by 256 elements is a launch more (4 us), so half the rows.
+static bool norm_by_row(int64_t rows, int H, bool limbs) {
+  const int few = H == 2560 ? 448 : H <= 256 * 16 ? 288 : 176;
+  return rows > (limbs ? few / 2 : few);
+}
+
 hipError_t launch_hc_norm(const bf16* residual, const bf16* out, const bf16* inject, int S, int hc, int H,
                           int tile, const bf16* scale, float eps, bf16* stream, bf16* normed, uint32_t* xp,
                           hipStream_t st, const XlBatch* xl) {
-  if (S > MAX_TOKENS) {
-    if (xl && hc > XL_FLAGS) return hipErrorInvalidValue;
+  if (xl && (S <= MAX_TOKENS || hc > XL_FLAGS || !normed)) return hipErrorInvalidValue;
+  if (S > MAX_TOKENS && norm_by_row((int64_t)S * hc, H, xl != nullptr)) {
     const XlBatch x = xl ? *xl : XlBatch{};
     const dim3 grid(hc, S);
     if (H == 2560)
@@ -243,7 +254,7 @@ hipError_t launch_hc_norm(const bf16* residual, const bf16* out, const bf16* inj
       hc_norm_batch_mode<48, false>(grid, residual, out, inject, hc, H, tile, scale, eps, stream, normed, xp, x, st);
     return hipGetLastError();
   }
-  if (xl) return hipErrorInvalidValue;
+  if (xl) xp = nullptr;
   const dim3 grid(hc, S, (H + 255) / 256);
   if (H == 2560)
     hc_norm_mode<10, true>(grid, residual, out, inject, hc, H, tile, scale, eps, stream, normed, xp, st);
@@ -251,7 +262,8 @@ hipError_t launch_hc_norm(const bf16* residual, const bf16* out, const bf16* inj
     hc_norm_mode<16, false>(grid, residual, out, inject, hc, H, tile, scale, eps, stream, normed, xp, st);
   else
     hc_norm_mode<48, false>(grid, residual, out, inject, hc, H, tile, scale, eps, stream, normed, xp, st);
-  return hipGetLastError();
+  const hipError_t e = hipGetLastError();
+  return e != hipSuccess || !xl ? e : launch_xlimb(normed, S, hc * H, *xl, st);
 }
 
 hipError_t launch_silu_xprep(const bf16* lo, int S, int LW, bf16* act, uint32_t* xp, hipStream_t st) {

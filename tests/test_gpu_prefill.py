@@ -344,6 +344,31 @@ def test_head_batch_large_last_stream_matches_windows(ctx, hc, H):
     head.close()
 
 
+# Both sides of the line between the two norm launches: 448 rows (positions x streams) at hidden 2560, 288 up to 4096, 176
+# above (the hidden norm's, hc * hidden wide, one per position), half as many where a mixer takes the limb form (6144, 10240).
+@pytest.mark.parametrize("hc,H,n", [(4, 2560, 56), (4, 2560, 57), (4, 2560, 112), (4, 2560, 113), (4, 1024, 72),
+                                    (4, 1024, 73), (4, 1536, 36), (4, 1536, 37), (4, 1536, 176), (4, 1536, 177)])
+def test_head_batch_norm_launches_match_windows(ctx, hc, H, n):
+    import mtpx
+    layer = dict(LAYER, hidden=H, max_positions=200)
+    head = mtpx.MTPHead(ctx, mtpx.HeadConfig(mtpx.LayerConfig(**layer), hc, 64, 1000, 500, 980), seed=43)
+    W = hc * H
+    r = np.random.default_rng(H + n)
+    ids, multi = dev(r.integers(0, 1000, n).astype(np.int32)), dev(rand_bf16(r, (n, W)))
+    kva, kvb = (mtpx.KVCache(ctx, layer["kv_heads"], layer["head_dim"], 200) for _ in range(2))
+    print("case head batch norms", hc, H, n, flush=True)
+    na, sa, nb, sb = empty_bf16(n, W), empty_bf16(n, H), empty_bf16(n, W), empty_bf16(n, H)
+    head.forward(kva, ids, multi, na, sa)
+    for w0 in range(0, n, 8):
+        w1 = min(n, w0 + 8)
+        head.forward(kvb, ids[w0:w1], multi[w0:w1], nb[w0:w1], sb[w0:w1])
+    assert np.array_equal(host(na), host(nb))
+    assert np.array_equal(host(sa), host(sb))
+    kva.close()
+    kvb.close()
+    head.close()
+
+
 @pytest.mark.parametrize("n", [1, 8, 9, 30])
 def test_prefill_outputs_are_optional(ctx, n):
     """Without logits, without streams, without both: what is asked for has the same bits, and so has the state."""
