@@ -494,13 +494,33 @@ static int gemm_shape(int K) {
 }
 
 // Scales are loaded by the dword: an odd count of them (K = 320 at group size 64 with an odd N) is not taken.
-bool gemm_ok(const uint32_t* w, const bf16* s, const bf16* b, int64_t N, int K, int gs, int M) {
+bool gemm_takes(const uint32_t* w, const bf16* s, const bf16* b, int64_t N, int K, int gs, int M) {
   if (M <= MAX_TOKENS || !mat_ok(w, s, b) || N * (K / gs) % 2 != 0 || N * K / 2 >= ((int64_t)1 << 31) || (int64_t)M * K * 6 >= ((int64_t)1 << 31))
     return false;
   switch (gemm_shape(K)) {
     case 16 * 16 + 5: case 32 * 16 + 6: case 64 * 16 + 5: case 64 * 16 + 4: case 2 * 16 + 5: return true;
     default: return false;
   }
+}
+
+// A launch takes the walk of one unit over K (23 us at K = 2560, 30 at 10240), whatever it holds, until the units
+// fill the chip; the GEMV's windows take about 10 us and grow with the tokens and with tokens times rows.  So windows up
+// to a number of each per depth, read off both sides at 8 .. 5120 rows and 9 .. 1024 tokens (us by windows / by the
+// GEMM: 324 x 10240, 9 tokens 10 / 30, 64: 26 / 36, 96: 44 / 39; 640 x 6144, 64: 24 / 28, 96: 34 / 30; 160 x 8192, 48:
+// 27 / 28, 64: 33 / 30; 8 x 2560, 256: 22 / 24, 512: 36 / 27; 640 x 2560, 128: 20 / 25, 192: 27 / 26; 2560 x 2560, 48:
+// 19 / 24, 64: 25 / 24), with and without packed scale rows alike.  Above 5120 rows the GEMM (16480 x 2560, 9 tokens: 24).
+// K = 320: equal (10 us) where both prepare x; on blocks that are there the windows save a launch (10240 rows: 9
+// tokens 7 / 10, 24: 10 / 10).
+bool gemm_faster(int64_t N, int K, int M, bool xp_ready) {
+  int tokens, product;
+  switch (gemm_shape(K)) {
+    case 16 * 16 + 5: tokens = 300, product = 125000; break;
+    case 32 * 16 + 6: tokens = 256, product = 41000; break;
+    case 64 * 16 + 4: tokens = 128, product = 10200; break;
+    case 64 * 16 + 5: tokens = 256, product = 26000; break;
+    default: return !xp_ready || M * N >= 250000;
+  }
+  return N > 5120 || M > tokens || M * N > product;
 }
 
 hipError_t launch_gemm_pair(const uint32_t* w1, const bf16* s1, const bf16* b1, int N1, bf16* y1, float* yf1,

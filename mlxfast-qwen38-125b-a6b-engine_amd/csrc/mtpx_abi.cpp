@@ -181,11 +181,11 @@ size_t xl_ws(int M, int K) { return M > MAX_TOKENS ? al(xl_bytes(M, K)) : 0; }
 
 XlBatch xl_take(Ctx* c, int M, int K) { return xl_carve(ws_take<char>(c, xl_bytes(M, K)), M, K); }
 
-// y [M, N] = x [M, K] . W^T: the batch GEMM on x where it takes the matrix, else the GEMV paths on the
-// prepared blocks xp.  Workspace: xl_ws(M, K), free again on return.
+// y [M, N] = x [M, K] . W^T: the batch GEMM on x where it takes the matrix and is faster, else the GEMV paths on the
+// prepared blocks xp (null: they are not made where the GEMM runs).  Workspace: xl_ws(M, K), free again on return.
 int dense_enqueue(Ctx* c, const char* name, const mtpx_q4& w, int N, int K, int gs, const uint16_t* x,
                   const uint32_t* xp, int M, uint16_t* y, float* yf = nullptr) {
-  if (gemm_ok(w.w, w.s, w.b, N, K, gs, M)) {
+  if (gemm_ok(w.w, w.s, w.b, N, K, gs, M, xp != nullptr)) {
     const size_t mark = c->ws_used;
     const XlBatch xl = xl_take(c, M, K);
     LAUNCH(c, "xlimb", launch_xlimb(x, M, K, xl, c->stream));
@@ -572,7 +572,7 @@ int attn_enqueue(Ctx* c, const Layer* L, Kv* kv, const uint16_t* x, uint32_t* xp
                                             L->w.rope_cos, L->w.rope_sin, (int)kv->offset, q, kv->k, kv->v,
                                             kv->tmax, st));
     if (batch) {
-      const bool gemm = gemm_ok(L->w.o_w, L->w.o_s, L->w.o_b, H, HQ * D, gs, M);
+      const bool gemm = gemm_ok(L->w.o_w, L->w.o_s, L->w.o_b, H, HQ * D, gs, M, true);
       LAUNCH(c, "attn_batch", launch_attn_batch(q, M, HQ, HK, kv->k, kv->v, kv->tmax, T, 1.0f / std::sqrt((float)D), part,
                                                 qkv, QW, HQ * D, att, gemm ? nullptr : xp, st));
       return dense_enqueue(c, "qmv_o", {L->w.o_w, L->w.o_s, L->w.o_b, L->w.o_sb}, H, HQ * D, gs, att, xp, M, o);
@@ -648,11 +648,12 @@ struct HcGeom {
   int H, hc, LW, gs;  // hidden, streams, low rank, group size
 };
 
-// Whether a batch's down and inject rows run as the batch GEMM, on the normed rows in limb form.
+// Whether a batch's down and inject rows run as one batch GEMM, on the normed rows in limb form.
 bool mix_batch_ok(const HcGeom& g, const mtpx_hc_weights* hw, int S) {
   const int W = g.hc * g.H;
-  return gemm_ok(hw->down.w, hw->down.s, hw->down.b, g.LW, W, g.gs, S) &&
-         (!hw->inject.w || gemm_ok(hw->inject.w, hw->inject.s, hw->inject.b, g.hc, W, g.gs, S));
+  return gemm_takes(hw->down.w, hw->down.s, hw->down.b, g.LW, W, g.gs, S) &&
+         (!hw->inject.w || gemm_takes(hw->inject.w, hw->inject.s, hw->inject.b, g.hc, W, g.gs, S)) &&
+         gemm_faster(g.LW + (hw->inject.w ? g.hc : 0), W, S, true);
 }
 
 int hc_mix_enqueue(Ctx* c, const HcGeom& g, const mtpx_hc_weights* hw, const uint16_t* normed, const uint32_t* xpW,
@@ -690,8 +691,10 @@ int hc_mix_enqueue(Ctx* c, const HcGeom& g, const mtpx_hc_weights* hw, const uin
            launch_gemm_pair(hw->down.w, hw->down.s, hw->down.b, LW, reinterpret_cast<bf16*>(lo), nullptr, hw->inject.w,
                             hw->inject.s, hw->inject.b, inj_on ? g.hc : 0, reinterpret_cast<bf16*>(inj), W, gs, xlW, S, st));
   } else {
-    if ((rc = dense_enqueue(c, "hc_down", hw->down, LW, W, gs, normed, xpW, S, lo))) return rc;
-    if (inj_on && (rc = dense_enqueue(c, "hc_inject", hw->inject, g.hc, W, gs, normed, xpW, S, inj))) return rc;
+    LAUNCH(c, "hc_down", launch_qmv(hw->down.w, hw->down.s, hw->down.b, hw->down.sb, LW, W, gs, xpW, S, lo, nullptr, st));
+    if (inj_on)
+      LAUNCH(c, "hc_inject", launch_qmv(hw->inject.w, hw->inject.s, hw->inject.b, hw->inject.sb, g.hc, W, gs, xpW, S, inj,
+                                        nullptr, st));
   }
   LAUNCH(c, "hc_silu", launch_silu_xprep(lo, S, LW, act, xpL, st));
   if ((rc = dense_enqueue(c, "hc_up", hw->up, W, LW, gs, act, xpL, S, wm))) return rc;
@@ -1590,7 +1593,7 @@ int mtpx_qmv(mtpx_ctx h, const uint32_t* wq, const uint16_t* s, const uint16_t* 
   ARG(gs_ok(gs) && k_ok(K, gs), "K=%d gs=%d unsupported", K, gs);
   if (set_device(c)) return MTPX_ERR_HIP;
   const size_t xpn = (size_t)M * (K / 32) * XP_DW;
-  const bool batch = gemm_ok(wq, s, b, N, K, gs, M);
+  const bool batch = gemm_ok(wq, s, b, N, K, gs, M, false);
   int rc = ws_reserve(c, (batch ? xl_ws(M, K) : al(xpn * 4)) + 256);
   if (rc) return rc;
   ws_begin(c);
@@ -2822,7 +2825,7 @@ int target_verify_enqueue(Ctx* c, Target* t, TargetState* s, const int32_t* ids,
       if ((rc = dense_enqueue(c, "qmv_gdn_in", ip, gg.pw, H, gs, x, xpH, S, proj))) return rc;
       if (prefill) {  // the batch in one launch, committed
         const size_t mark3 = c->ws_used;
-        if ((rc = gdn_enqueue_batch(c, L.gdn, s->gdn[i], proj, S, gated, gemm_ok(op.w, op.s, op.b, H, VD, gs, S) ? nullptr : xpG))) return rc;
+        if ((rc = gdn_enqueue_batch(c, L.gdn, s->gdn[i], proj, S, gated, gemm_ok(op.w, op.s, op.b, H, VD, gs, S, true) ? nullptr : xpG))) return rc;
         c->ws_used = mark3;
       } else if ((rc = gdn_enqueue(c, L.gdn, s->gdn[i], proj, S, nullptr, xpG))) {
         return rc;

@@ -171,8 +171,13 @@ __device__ __forceinline__ void xl_flag(uint8_t* big, size_t t, int who, int of,
 size_t xl_bytes(int M, int K);                // workspace of one batch
 XlBatch xl_carve(void* ws, int M, int K);     // its arrays in that workspace (256-byte aligned)
 hipError_t launch_xlimb(const bf16* x, int M, int K, const XlBatch& b, hipStream_t st);
-bool gemm_ok(const uint32_t* w, const bf16* s, const bf16* b, int64_t N, int K, int gs, int M);
-// y1 [M, N1] (and y2 [M, N2] where w2 is set) from x; every matrix passes gemm_ok
+bool gemm_takes(const uint32_t* w, const bf16* s, const bf16* b, int64_t N, int K, int gs, int M);
+// Whether one launch over N rows in all is faster than the GEMV's windows on prepared blocks (xp_ready: they are there).
+bool gemm_faster(int64_t N, int K, int M, bool xp_ready);
+inline bool gemm_ok(const uint32_t* w, const bf16* s, const bf16* b, int64_t N, int K, int gs, int M, bool xp_ready) {
+  return gemm_takes(w, s, b, N, K, gs, M) && gemm_faster(N, K, M, xp_ready);
+}
+// y1 [M, N1] (and y2 [M, N2] where w2 is set) from x; gemm_takes every matrix
 hipError_t launch_gemm_pair(const uint32_t* w1, const bf16* s1, const bf16* b1, int N1, bf16* y1, float* yf1,
                             const uint32_t* w2, const bf16* s2, const bf16* b2, int N2, bf16* y2, int K, int gs,
                             const XlBatch& x, int M, hipStream_t st);

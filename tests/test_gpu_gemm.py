@@ -21,28 +21,50 @@ def ctx():
     c.close()
 
 
-def _check(ctx, wq, s, b, gs, x, ds=None, db=None):
+def _check(ctx, wq, s, b, gs, x, ds=None, db=None, gemm=True, packed=False):
+    """gemm: whether the batch GEMM (which prepares x in limb form) is what runs."""
     M, N = x.shape[0], wq.shape[0]
     y_o, yf_o = O.qmv(wq, s, b, gs, x)
     ds, db = dev(s) if ds is None else ds, dev(b) if db is None else db
     y, yf = empty_bf16(M, N), torch.zeros(M, N, dtype=torch.float32, device="cuda")
-    ctx.qmv(dev(wq), ds, db, gs, dev(x), y, yf)
-    ctx.synchronize()
+    sb = ctx.pack_sb(ds, db, x.shape[1], gs) if packed else None
+    ctx.profile(True)
+    ctx.profile_reset()
+    ctx.qmv(dev(wq), ds, db, gs, dev(x), y, yf, sb=sb)
+    launched = ctx.profile_stats()
+    ctx.profile(False)
+    assert ("xlimb" in launched) == gemm, launched
     assert np.array_equal(host(yf).view(np.uint32), yf_o.view(np.uint32))
     assert np.array_equal(host(y), y_o)
 
 
-# row blocks of 128 (K 2560), 64 (6144), 32 (8192, 10240) and 256 (320) rows; tiles of 16 tokens
+# row blocks of 128 (K 2560), 64 (6144), 32 (8192, 10240) and 256 (320) rows; tiles of 16 tokens; the fewest tokens or
+# rows that it takes at each depth
 @pytest.mark.parametrize("N,K,gs,M", [
-    (1, 2560, 64, 9), (127, 2560, 32, 16), (128, 2560, 64, 17), (385, 2560, 64, 33), (17, 2560, 32, 80),
-    (64, 6144, 64, 16), (65, 6144, 32, 15), (1, 10240, 32, 9), (33, 10240, 64, 31), (31, 8192, 64, 17),
-    (255, 320, 64, 9), (513, 320, 32, 47), (16, 320, 64, 16),
+    (1, 2560, 64, 301), (127, 2560, 32, 304), (128, 2560, 64, 305), (385, 2560, 64, 325), (17, 2560, 32, 319),
+    (5121, 2560, 64, 9), (5247, 2560, 32, 16), (5120, 2560, 64, 25),
+    (64, 6144, 64, 257), (641, 6144, 32, 64), (5121, 6144, 32, 9), (1, 10240, 32, 257), (325, 10240, 64, 81),
+    (5150, 10240, 64, 17), (31, 8192, 64, 129), (200, 8192, 32, 52), (254, 320, 64, 9), (513, 320, 32, 47),
+    (16, 320, 64, 16),
 ])
 def test_gemm_edges_bit_exact(ctx, N, K, gs, M):
     print("case", N, K, gs, M, flush=True)
     r = np.random.default_rng(N * 7 + K + M)
     wq, s, b = qweights(r, N, K, gs)
     _check(ctx, wq, s, b, gs, rand_bf16(r, (M, K)))
+
+
+@pytest.mark.parametrize("packed", [False, True])
+@pytest.mark.parametrize("N,K,gs,M", [
+    (385, 2560, 64, 300), (5120, 2560, 32, 24), (65, 6144, 32, 256), (640, 6144, 64, 64), (33, 10240, 64, 256),
+    (325, 10240, 64, 80), (31, 8192, 64, 128), (200, 8192, 32, 51), (324, 10240, 64, 9), (255, 320, 64, 9)])
+def test_batch_by_windows_below_the_gemms_line(ctx, N, K, gs, M, packed):
+    """The most tokens that the windows take, a mixer's rows at nine tokens, and an odd count of scales, which its loads do
+    not take: the GEMV's windows."""
+    print("case windows", N, K, gs, M, packed, flush=True)
+    r = np.random.default_rng(N + K + M)
+    wq, s, b = qweights(r, N, K, gs)
+    _check(ctx, wq, s, b, gs, rand_bf16(r, (M, K)), gemm=False, packed=packed)
 
 
 @pytest.mark.parametrize("K,gs", [(2560, 64), (6144, 32), (10240, 64), (320, 32)])
@@ -52,7 +74,7 @@ def test_gemm_extreme_blocks_bit_exact(ctx, K, gs):
     print("case", K, gs, flush=True)
     r = np.random.default_rng(K)
     wq, s, b = qweights(r, 70, K, gs)
-    x = r.standard_normal((40, K)).astype(np.float32)
+    x = r.standard_normal((310, K)).astype(np.float32)
     x[5, 32:64] *= 3e4                                            # the first tile walks with the factor
     x[17] *= np.float32(2.0) ** np.repeat(np.linspace(-118, -2, K // 32).astype(int), 32)
     x[18] = 0
@@ -70,7 +92,7 @@ def test_gemm_two_byte_aligned_scales(ctx):
     pad = [torch.zeros(s.size + 1, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
     for p, a in zip(pad, (s, b)):
         p[1:] = dev(a).reshape(-1)
-    _check(ctx, wq, s, b, 64, rand_bf16(r, (21, 2560)), *[p[1:].view(48, 40) for p in pad])
+    _check(ctx, wq, s, b, 64, rand_bf16(r, (310, 2560)), *[p[1:].view(48, 40) for p in pad], gemm=False)
 
 
 @pytest.mark.parametrize("large", [False, True])

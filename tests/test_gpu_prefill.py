@@ -288,21 +288,26 @@ def test_head_batch_matches_windows(ctx, n):
     head.close()
 
 
-@pytest.mark.parametrize("n", [9, 41])
+@pytest.mark.parametrize("n", [9, 41, 80, 81, 121])
 def test_head_batch_at_width_matches_windows(ctx, n):
-    """The head's batch at hidden 2560 (the batch norm's limb form, the mixers' batch GEMMs) against windows of 8:
-    one position more than a window, and a ragged token tile."""
+    """The head's batch at hidden 2560 against windows of 8: one position more than a window, a ragged token tile, and both
+    sides of the line from which the norms write the limb form for the mixers' batch GEMM (81 positions)."""
     import mtpx
-    layer = dict(LAYER, hidden=2560, group_size=64, max_positions=64)
+    layer = dict(LAYER, hidden=2560, group_size=64, max_positions=128)
     hc, vocab = 4, 1000
     head = mtpx.MTPHead(ctx, mtpx.HeadConfig(mtpx.LayerConfig(**layer), hc, 320, vocab, 500, 980), seed=29)
     W = hc * 2560
     r = np.random.default_rng(n)
     ids, multi = dev(r.integers(0, vocab, n).astype(np.int32)), dev(rand_bf16(r, (n, W)))
-    kva, kvb = (mtpx.KVCache(ctx, layer["kv_heads"], layer["head_dim"], 64) for _ in range(2))
+    kva, kvb = (mtpx.KVCache(ctx, layer["kv_heads"], layer["head_dim"], 128) for _ in range(2))
     print("case head batch at width", n, flush=True)
     na, sa, nb, sb = empty_bf16(n, W), empty_bf16(n, 2560), empty_bf16(n, W), empty_bf16(n, 2560)
+    ctx.profile(True)
+    ctx.profile_reset()
     head.forward(kva, ids, multi, na, sa)
+    launched = ctx.profile_stats()
+    ctx.profile(False)
+    assert ("hc_down_inject" in launched) == (n > 80), launched
     for w0 in range(0, n, 8):
         w1 = min(n, w0 + 8)
         head.forward(kvb, ids[w0:w1], multi[w0:w1], nb[w0:w1], sb[w0:w1])
@@ -320,38 +325,45 @@ def test_head_batch_large_last_stream_matches_windows(ctx, hc, H):
     """Normed rows above 4096 in the last stream alone (its norm scales 1e5 in every mixer): the batch's mixers
     walk with the blocks' factors whichever stream holds them, bit-equal to windows of 8."""
     import mtpx
-    layer = dict(LAYER, hidden=H, max_positions=64)
-    head = mtpx.MTPHead(ctx, mtpx.HeadConfig(mtpx.LayerConfig(**layer), hc, 64, 1000, 500, 980), seed=37)
+    layer = dict(LAYER, hidden=H, max_positions=256)
+    head = mtpx.MTPHead(ctx, mtpx.HeadConfig(mtpx.LayerConfig(**layer), hc, 512, 1000, 500, 980), seed=37)
     w = head.weights()
     for m in (w.attn_hc, w.mlp_hc, w.final_hc):
         sc = O.f32_to_bf16(np.ones((hc, H), np.float32))
         sc[hc - 1] = O.f32_to_bf16(np.full(H, 1e5, np.float32))
         write_device(m.norm_scale, sc)
-    n, W = 21, hc * H
+    n, W = 250, hc * H  # enough positions for the mixers' batch GEMM at every depth
     r = np.random.default_rng(H + hc)
     ids, multi = dev(r.integers(0, 1000, n).astype(np.int32)), dev(rand_bf16(r, (n, W)))
-    kva, kvb = (mtpx.KVCache(ctx, layer["kv_heads"], layer["head_dim"], 64) for _ in range(2))
+    kva, kvb = (mtpx.KVCache(ctx, layer["kv_heads"], layer["head_dim"], 256) for _ in range(2))
     print("case head batch, large last stream", hc, H, flush=True)
     na, sa, nb, sb = empty_bf16(n, W), empty_bf16(n, H), empty_bf16(n, W), empty_bf16(n, H)
+    ctx.profile(True)
+    ctx.profile_reset()
     head.forward(kva, ids, multi, na, sa)
+    launched = ctx.profile_stats()
+    ctx.profile(False)
     for w0 in range(0, n, 8):
         w1 = min(n, w0 + 8)
         head.forward(kvb, ids[w0:w1], multi[w0:w1], nb[w0:w1], sb[w0:w1])
     assert np.array_equal(host(na), host(nb))
     assert np.array_equal(host(sa), host(sb))
+    assert launched["hc_down_inject"][0] == 3, launched
     kva.close()
     kvb.close()
     head.close()
 
 
 # Both sides of the line between the two norm launches: 448 rows (positions x streams) at hidden 2560, 288 up to 4096, 176
-# above (the hidden norm's, hc * hidden wide, one per position), half as many where a mixer takes the limb form (6144, 10240).
-@pytest.mark.parametrize("hc,H,n", [(4, 2560, 56), (4, 2560, 57), (4, 2560, 112), (4, 2560, 113), (4, 1024, 72),
-                                    (4, 1024, 73), (4, 1536, 36), (4, 1536, 37), (4, 1536, 176), (4, 1536, 177)])
-def test_head_batch_norm_launches_match_windows(ctx, hc, H, n):
+# above (the hidden norm's, hc * hidden wide, one per position), half as many where a mixer takes the limb form: two
+# streams of 4096, against smaller batches, which it takes in blocks (windows of that width are refused).
+@pytest.mark.parametrize("hc,H,n,lowrank,win", [
+    (4, 2560, 112, 64, 8), (4, 2560, 113, 64, 8), (4, 1024, 72, 64, 8), (4, 1024, 73, 64, 8), (4, 1536, 72, 64, 8),
+    (4, 1536, 73, 64, 8), (4, 1536, 176, 64, 8), (4, 1536, 177, 64, 8), (2, 4096, 72, 320, 24), (2, 4096, 75, 320, 25)])
+def test_head_batch_norm_launches_match_windows(ctx, hc, H, n, lowrank, win):
     import mtpx
     layer = dict(LAYER, hidden=H, max_positions=200)
-    head = mtpx.MTPHead(ctx, mtpx.HeadConfig(mtpx.LayerConfig(**layer), hc, 64, 1000, 500, 980), seed=43)
+    head = mtpx.MTPHead(ctx, mtpx.HeadConfig(mtpx.LayerConfig(**layer), hc, lowrank, 1000, 500, 980), seed=43)
     W = hc * H
     r = np.random.default_rng(H + n)
     ids, multi = dev(r.integers(0, 1000, n).astype(np.int32)), dev(rand_bf16(r, (n, W)))
@@ -359,8 +371,8 @@ def test_head_batch_norm_launches_match_windows(ctx, hc, H, n):
     print("case head batch norms", hc, H, n, flush=True)
     na, sa, nb, sb = empty_bf16(n, W), empty_bf16(n, H), empty_bf16(n, W), empty_bf16(n, H)
     head.forward(kva, ids, multi, na, sa)
-    for w0 in range(0, n, 8):
-        w1 = min(n, w0 + 8)
+    for w0 in range(0, n, win):
+        w1 = min(n, w0 + win)
         head.forward(kvb, ids[w0:w1], multi[w0:w1], nb[w0:w1], sb[w0:w1])
     assert np.array_equal(host(na), host(nb))
     assert np.array_equal(host(sa), host(sb))
