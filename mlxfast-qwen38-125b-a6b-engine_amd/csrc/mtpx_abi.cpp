@@ -317,12 +317,16 @@ int moe_enqueue(Ctx* c, const mtpx_moe_weights* w, const uint16_t* x, int M, uin
       a.chunk_n = ws_take<int32_t>(c, 1);
       a.max_chunks = moe_max_chunks((int)T, a.E, a.K);
       LAUNCH(c, "moe_sort", launch_moe_sort(a, c->stream));
-      if (moe_gemm_down_ok(a)) {  // the experts over their chunks on the matrix cores
-        // gate|up: a chunk costs 16 tokens whatever it holds, so below about 2.7 slots per expert the walk of
-        // one slot per workgroup is faster (whole prefill of four layers, 128 / 160 tokens of 512 experts
-        // top-10: 3515 / 3804 us by chunks, 3487 / 3959 by slots; 75 tokens: 2900 / 2650; 512: 7000 / 9700)
-        const XlBatch xt = xl_take(c, (int)T, a.H), xs = xl_take(c, (int)slots, a.F);
+      // The experts over their chunks on the matrix cores.  A chunk costs 16 tokens whatever it holds, so with few slots
+      // per expert the walk of one slot per workgroup is faster.  Down: below 1.25 (launches by slots / by chunks and their
+      // limb pass, us: 512 experts, hidden 1024, top-10, 64 tokens (1.25 slots) 46 / 55; hidden 2560, top-16, 24 (0.75) 68 /
+      // 88, 64 (2.0) 158 / 126; 64 experts top-8, 24 (3.0) 20 / 22, 64 (8.0) 38 / 22).  Gate|up: below 2.7 (whole prefill of
+      // four layers, 128 / 160 tokens of 512 experts top-10: 3515 / 3804 by chunks, 3487 / 3959 by slots; 75 tokens: 2900 /
+      // 2650; 512: 7000 / 9700).
+      if (moe_gemm_down_ok(a) && T * a.K * 4 >= (size_t)a.E * 5) {
+        const XlBatch xs = xl_take(c, (int)slots, a.F);
         if (moe_gemm_gate_up_ok(a) && T * a.K * 3 >= (size_t)a.E * 8) {
+          const XlBatch xt = xl_take(c, (int)T, a.H);
           LAUNCH(c, "xlimb", launch_xlimb(a.x, (int)T, a.H, xt, c->stream));
           LAUNCH(c, "moe_gate_up", launch_moe_gemm_gate_up(a, xt, c->stream));
         } else {

@@ -56,11 +56,12 @@ def test_moe_batch_matches_windows(ctx, H, E, K, n, q4):
     head.close()
 
 
-# row blocks of 128 rows of H: whole ones and a last one of 32 rows
-@pytest.mark.parametrize("H,E,K,n,gs", [(1024, 32, 4, 70, 64), (544, 16, 3, 33, 32), (512, 9, 9, 17, 64)])
-def test_expert_down_chunks_at_other_hidden_sizes(ctx, H, E, K, n, gs):
-    """The expert down GEMM at expert width 640 takes any hidden size (the only launch here that reads activations in
-    limb form), bit-equal to windows of 8."""
+# row blocks of 128 rows of H: whole ones and a last one of 32 rows; slots per expert on both sides of 1.25
+@pytest.mark.parametrize("H,E,K,n,gs,chunks", [(1024, 32, 4, 70, 64, 1), (544, 16, 3, 33, 32, 1), (512, 9, 9, 17, 64, 1),
+                                               (1024, 32, 4, 10, 32, 1), (1024, 32, 4, 9, 32, 0), (2560, 96, 6, 19, 64, 0)])
+def test_expert_down_chunks_at_other_hidden_sizes(ctx, H, E, K, n, gs, chunks):
+    """The expert down GEMM at expert width 640 takes any hidden size, from 1.25 slots per expert on (it reads the experts'
+    activations in limb form: its number of passes tells), bit-equal to windows of 8."""
     import mtpx
     lc = mtpx.LayerConfig(H, E, K, 640, gs, 4, 2, 64, 16, 32, 1e7, 1e-6, 256)
     head = mtpx.MTPHead(ctx, mtpx.HeadConfig(lc, 4, 64, 1000, 500, 980), seed=41 + n)
@@ -75,7 +76,9 @@ def test_expert_down_chunks_at_other_hidden_sizes(ctx, H, E, K, n, gs):
     head.forward(kva, ids, multi, got)
     launched = ctx.profile_stats()
     ctx.profile(False)
-    assert launched["moe_route_batch"][0] == 1 and launched["xlimb"][0] == 1, launched
+    assert launched["moe_route_batch"][0] == 1, launched
+    if H != 2560:  # no projection here is of a depth that the dense GEMM takes
+        assert launched.get("xlimb", (0,))[0] == chunks, launched
     for w0 in range(0, n, 8):
         w1 = min(n, w0 + 8)
         head.forward(kvb, ids[w0:w1], multi[w0:w1], want[w0:w1])
