@@ -410,7 +410,7 @@ __global__ __launch_bounds__(RR_THREADS) void k_moe_router_route(MoeArgs a0, int
 // the four rows' values together (a permlane swap puts one row's lower lanes beside the other's), so every
 // quarter of the wave goes on with one row.  What bounds it: 220 vector instructions per token and wave at
 // H = 2560 (160 fmaf, 40 to widen x) where the window launch spends 140 per token and row: 1003 tokens of
-// 513 rows BEFORE -> AFTER us.
+// 513 rows: 187 us in the windows' launches, 69 here (and 8 in k_moe_route_batch).
 constexpr int RB_TOK = 4;
 
 template <int NIT, bool EXACT, int RW>
@@ -1017,7 +1017,19 @@ static hipError_t router_batch_go(const MoeArgs& a, hipStream_t st) {
 
 hipError_t launch_moe_route_batch(const MoeArgs& a, hipStream_t st) {
   if (a.M <= MAX_TOKENS || a.H % 8 != 0 || a.H / 8 > ROUTER_IT * 64 || !a.xp_ready) return hipErrorInvalidValue;
-  hipError_t e = a.H / 8 == 5 * 64 ? router_batch_go<5, true, 4>(a, st) : router_batch_go<ROUTER_IT, false, 1>(a, st);
+  // four rows per wave while their weights fit its registers; the chunk count of the width, so that no lane walks past it
+  // (512 experts, hidden 1024, 256 tokens, router and route: one row per wave and eight chunks 55 us, four rows and two
+  // chunks 23; the windows' launch 48)
+  const int nc = a.H / 8;
+  hipError_t e;
+  if (nc == 5 * 64)
+    e = router_batch_go<5, true, 4>(a, st);
+  else if (nc <= 2 * 64)
+    e = router_batch_go<2, false, 4>(a, st);
+  else if (nc <= 4 * 64)
+    e = router_batch_go<4, false, 4>(a, st);
+  else
+    e = router_batch_go<ROUTER_IT, false, 1>(a, st);
   if (e != hipSuccess) return e;
   const dim3 grid((a.M + MAX_TOKENS - 1) / MAX_TOKENS);
   if (a.E <= 512)

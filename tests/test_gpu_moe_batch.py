@@ -1,7 +1,7 @@
 """The MoE block of a prefill batch (its own router launch, one expert order for all its tokens), bit-exact against the
 same positions in windows of 8: one position more than a window, a tail that is no window, expert counts that do not
-fill a wave's or a workgroup's rows, the largest counts, both widths of the router launch, and the shared expert's gate
-as a bf16 row and as a q4 row."""
+fill a wave's or a workgroup's rows, the largest counts, every instance of the router launch (by the 16-byte chunks of a
+row: up to 128, up to 256, 320, more; whole and ragged), and the shared expert's gate as a bf16 row and as a q4 row."""
 import numpy as np
 import pytest
 
@@ -20,13 +20,14 @@ def ctx():
 
 
 @pytest.mark.parametrize("H,E,K,n,q4", [
-    (256, 16, 4, 9, False), (256, 1024, 16, 37, True), (256, 31, 1, 255, False), (2560, 33, 3, 13, True),
+    (512, 16, 4, 9, False), (544, 1024, 16, 37, True), (1024, 31, 1, 255, False), (2048, 33, 3, 13, True),
+    (1056, 40, 7, 20, False), (2080, 70, 5, 21, False), (4096, 16, 2, 33, False), (2560, 33, 3, 13, True),
     (2560, 520, 10, 30, False), (2560, 16, 10, 70, False)])
 def test_moe_batch_matches_windows(ctx, H, E, K, n, q4):
     import mtpx
     layer = dict(hidden=H, experts=E, top_k=K, expert_width=128, group_size=32, heads=4, kv_heads=2, head_dim=64,
                  rot_dims=16, index_dim=32, rope_theta=1e7, eps=1e-6, max_positions=256)
-    hc, V = 4, 1000
+    hc, V = 4 if H < 2048 or H == 2560 else 1, 1000
     cfg = mtpx.HeadConfig(mtpx.LayerConfig(**layer), hc, 64, V, 500, 980)
     head = mtpx.MTPHead(ctx, cfg, seed=31 + n)
     r = np.random.default_rng(E + n)
@@ -44,7 +45,12 @@ def test_moe_batch_matches_windows(ctx, H, E, K, n, q4):
     kva, kvb = (mtpx.KVCache(ctx, 2, 64, 256) for _ in range(2))
     print("case MoE batch", H, E, K, n, q4, flush=True)
     got, want = empty_bf16(n, W), empty_bf16(n, W)
+    ctx.profile(True)
+    ctx.profile_reset()
     used.forward(kva, ids, multi, got)
+    launched = ctx.profile_stats()
+    ctx.profile(False)
+    assert launched["moe_route_batch"][0] == 1, launched
     for w0 in range(0, n, 8):
         w1 = min(n, w0 + 8)
         used.forward(kvb, ids[w0:w1], multi[w0:w1], want[w0:w1])
