@@ -546,9 +546,14 @@ int layer_create(Ctx* c, const mtpx_layer_config* cfg, uint64_t seed, Layer** ou
   return MTPX_OK;
 }
 
+// Queries per launch of the chunk partials, whose workspace is (D + 2) / 32 floats per query, head and key (24 heads of
+// 128, 512 queries over 2048 keys: 0.41 GB).
+constexpr int PARTIAL_QUERIES = 512;
+
 // A batch's scores, or the chunks' partials.
 size_t attn_ws_floats(int M, int HQ, int HK, int D, int T) {
-  return attn_batch_ok(M, HQ, HK, D, T) ? attn_batch_floats(M, HQ, T) : attn_partial_floats(M, HQ, D, T);
+  return attn_batch_ok(M, HQ, HK, D, T) ? attn_batch_floats(M, HQ, T)
+                                        : attn_partial_floats(std::min(M, PARTIAL_QUERIES), HQ, D, T);
 }
 
 // Attention sublayer for M tokens x whose prepared input blocks are in xp:
@@ -567,24 +572,29 @@ int attn_enqueue(Ctx* c, const Layer* L, Kv* kv, const uint16_t* x, uint32_t* xp
   hipStream_t st = c->stream;
   int rc = dense_enqueue(c, "qmv_qkv", {L->w.qkv_w, L->w.qkv_s, L->w.qkv_b, L->w.qkv_sb}, QW, H, gs, x, xp, M, qkv);
   if (rc) return rc;
+  const float scale = 1.0f / std::sqrt((float)D);
   if (attn_prep_fused_ok(M, HQ, HK, D, QW)) {  // a verify window: the prep inside the partial launch
     LAUNCH(c, "attn_partial", launch_attn_partial_prep(qkv, QW, M, HQ, HK, D, g.rot_dims, L->w.q_norm, L->w.k_norm,
                                                        g.eps, L->w.rope_cos, L->w.rope_sin, kv->k, kv->v, kv->tmax, T,
-                                                       1.0f / std::sqrt((float)D), part, st));
+                                                       scale, part, st));
+    LAUNCH(c, "attn_combine", launch_attn_combine(M, HQ, HK, D, T, part, qkv, QW, HQ * D, nullptr, att, xp, st));
   } else {  // a batch: the prep over all positions, then its own attention where the geometry allows
     LAUNCH(c, "attn_prep", launch_attn_prep(qkv, M, QW, HQ, HK, D, g.rot_dims, L->w.q_norm, L->w.k_norm, g.eps,
                                             L->w.rope_cos, L->w.rope_sin, (int)kv->offset, q, kv->k, kv->v,
                                             kv->tmax, st));
     if (batch) {
       const bool gemm = gemm_ok(L->w.o_w, L->w.o_s, L->w.o_b, H, HQ * D, gs, M, true);
-      LAUNCH(c, "attn_batch", launch_attn_batch(q, M, HQ, HK, kv->k, kv->v, kv->tmax, T, 1.0f / std::sqrt((float)D), part,
-                                                qkv, QW, HQ * D, att, gemm ? nullptr : xp, st));
-      return dense_enqueue(c, "qmv_o", {L->w.o_w, L->w.o_s, L->w.o_b, L->w.o_sb}, H, HQ * D, gs, att, xp, M, o);
+      LAUNCH(c, "attn_batch", launch_attn_batch(q, M, HQ, HK, kv->k, kv->v, kv->tmax, T, scale, part, qkv, QW, HQ * D, att,
+                                                gemm ? nullptr : xp, st));
     }
-    LAUNCH(c, "attn_partial", launch_attn_partial(q, M, HQ, HK, D, kv->k, kv->v, kv->tmax, T,
-                                                  1.0f / std::sqrt((float)D), part, st));
+    for (int m0 = 0; !batch && m0 < M; m0 += PARTIAL_QUERIES) {  // each query sees the keys up to its own position
+      const int n = std::min(M - m0, PARTIAL_QUERIES), Tn = T - (M - m0 - n);
+      const size_t q0 = (size_t)m0 * HQ * D;
+      LAUNCH(c, "attn_partial", launch_attn_partial(q + q0, n, HQ, HK, D, kv->k, kv->v, kv->tmax, Tn, scale, part, st));
+      LAUNCH(c, "attn_combine", launch_attn_combine(n, HQ, HK, D, Tn, part, qkv + (size_t)m0 * QW, QW, HQ * D, nullptr,
+                                                    att + q0, xp + q0 / 32 * XP_DW, st));
+    }
   }
-  LAUNCH(c, "attn_combine", launch_attn_combine(M, HQ, HK, D, T, part, qkv, QW, HQ * D, nullptr, att, xp, st));
   return dense_enqueue(c, "qmv_o", {L->w.o_w, L->w.o_s, L->w.o_b, L->w.o_sb}, H, HQ * D, gs, att, xp, M, o);
 }
 

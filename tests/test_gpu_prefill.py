@@ -196,6 +196,36 @@ def test_prefill_past_one_batch_matches_windows(ctx, monkeypatch):
     t.close()
 
 
+def test_prefill_workspace_at_head_dim_128():
+    """Where attention goes by chunk partials (head dim 128) a batch of 1024 queries takes them 512 at a time: 0.41 GB of
+    them over 2048 keys at 24 heads, not 0.82."""
+    need_gpu()
+    import mtpx
+    own = mtpx.Context(0)
+    lc = mtpx.LayerConfig(256, 16, 4, 128, 32, 24, 2, 128, 32, 32, 1e7, 1e-6, 2048)
+    cfg = mtpx.TargetConfig(lc, 1, 2, 4, 1, 1, 4, 64, 1000)
+    cfg.ple_layer = -1
+    t = mtpx.Target(own, cfg, seed=3)
+    st = mtpx.TargetState(own, t)
+    ids = dev(np.arange(1024, dtype=np.int32) % 1000)
+    print("case prefill workspace", flush=True)
+    t.prefill(st, ids[:8].contiguous())
+    st.set_offset(1024)
+    own.synchronize()
+    before = torch.cuda.mem_get_info()[0]
+    own.profile(True)
+    own.profile_reset()
+    t.prefill(st, ids)
+    launched = own.profile_stats()
+    own.profile(False)
+    grown = before - torch.cuda.mem_get_info()[0]
+    st.close()
+    t.close()
+    own.close()
+    assert launched["attn_partial"][0] == launched["attn_combine"][0] == 2, launched
+    assert grown < 800e6, grown  # the workspace, with a quarter above the need
+
+
 @pytest.mark.timeout(600)
 @pytest.mark.parametrize("pre,n,partial", [(1024, 45, False), (400, 600, False), (300, 70, True)],
                          ids=["45-after-1024", "600-after-400", "70-after-partial-window"])
