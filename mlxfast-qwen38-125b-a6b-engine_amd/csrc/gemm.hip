@@ -239,8 +239,16 @@ __global__ __launch_bounds__(GT_THREADS, MINW) void k_gemm(std::conditional_t<MO
   }
   auto xrow_at = [&](int t) -> uint32_t { return __shfl((int)xrow_n, t, 64); };
   const uint32_t xrow_l = xrow_at(lane >> 2), xoff = (xrow_l * NB + ((lane & 3) ^ g) * 4) * 4;
-  // row of row-in-block r, clamped: rows past the end repeat the last one (computed, not stored)
-  auto lrow = [&](int r) { return min(row0 + (MODE == GT_GATE_UP && r >= R / 2 ? r - R / 2 : r), rows_w - 1); };
+  // The weight and scale resources start at the unit's first row, so that offsets are of 32 bits whatever the matrix holds.
+  const int rows_u = min(rows_w - row0, MODE == GT_GATE_UP ? R / 2 : R);
+  w0 += (size_t)row0 * (ROWB / 4);
+  w1 += (size_t)row0 * (ROWB / 4);
+  s0 += (size_t)row0 * ng;
+  b0 += (size_t)row0 * ng;
+  s1 += (size_t)row0 * ng;
+  b1 += (size_t)row0 * ng;
+  // unit row of row-in-block r, clamped: rows past the end repeat the last one (computed, not stored)
+  auto lrow = [&](int r) { return min(MODE == GT_GATE_UP && r >= R / 2 ? r - R / 2 : r, rows_u - 1); };
   auto my_tile = [&](int rt) {  // row tile of this wave's tile rt
     return MODE == GT_GATE_UP ? (rt / (RT / 2)) * (NT / 2) + rg * (RT / 2) + rt % (RT / 2) : rg * RT + rt;
   };
@@ -252,10 +260,10 @@ __global__ __launch_bounds__(GT_THREADS, MINW) void k_gemm(std::conditional_t<MO
   // One weight and one scale resource per wave.  gate|up: the stage loads are 12 of limbs and 8 of weights, so
   // waves 4-7 load the gate's row tiles and waves 0-3 the up's; scale load i (s: i < SI, then b) is wave i's.
   static_assert(MODE != GT_GATE_UP || (AI == 12 && WI == 8), "the waves' weight loads");
-  const auto rW = make_rsrc(sel(MODE == GT_GATE_UP && wave < 4, w1, w0), (size_t)rows_w * ROWB);
+  const auto rW = make_rsrc(sel(MODE == GT_GATE_UP && wave < 4, w1, w0), (size_t)rows_u * ROWB);
   static_assert(WHOLE || 2 * SI <= 8, "a scale load per wave and granule");
   const bool cup = MODE == GT_GATE_UP && wave % SI >= SI / 2;
-  const auto rC = make_rsrc(sel(wave < SI, sel(cup, s1, s0), sel(cup, b1, b0)), (size_t)rows_w * ng * 2);
+  const auto rC = make_rsrc(sel(wave < SI, sel(cup, s1, s0), sel(cup, b1, b0)), (size_t)rows_u * ng * 2);
 
   // ---- staging: this wave's loads i = wave, wave + 8, ..: limbs i < AI, then weights ----
   uint32_t off[PER_W];
@@ -294,9 +302,9 @@ __global__ __launch_bounds__(GT_THREADS, MINW) void k_gemm(std::conditional_t<MO
       for (int k = 0; k < (2 * SI + XI + 7) / 8; ++k) {
         const int i = wave + 8 * k;
         if (i < 2 * SI) {
-          const auto r = make_rsrc(sel(i < SI, s0, b0), (size_t)rows_w * ng * 2);  // past the end: zeros
+          const auto r = make_rsrc(sel(i < SI, s0, b0), (size_t)rows_u * ng * 2);  // past the end: zeros
           __builtin_amdgcn_raw_ptr_buffer_load_lds(r, (lds_void_t*)(d + i * 64), 16,
-                                                   (uint32_t)row0 * (ng * 2) + ((i % SI) * 64 + lane) * 16, 0, 0, 0);
+                                                   (uint32_t)((i % SI) * 64 + lane) * 16, 0, 0, 0);
         } else if (i < 2 * SI + XI) {
           const int j = i - 2 * SI, u = j * 64 + lane;
           const uint32_t o = (xrow_at(min(u / GB, 15)) * NB + u % GB) * 4;
@@ -476,7 +484,7 @@ static bool mat_ok(const uint32_t* w, const bf16* s, const bf16* b) {
 // ---- dense ----
 template <int L, int IT, int C, int RT, int NST, int MINW>
 static hipError_t dense_li(GemmArgs a, bool gs32, hipStream_t st) {
-  constexpr int R = 8 / C * RT * 16;
+  constexpr int R = 8 / C * RT * 16;  // gemm_rows
   a.rblocks1 = (a.mat[0].N + R - 1) / R;
   a.rblocks = a.rblocks1 + (a.mat[1].w ? (a.mat[1].N + R - 1) / R : 0);
   a.tiles = (a.M + 15) / 16;
@@ -493,14 +501,23 @@ static int gemm_shape(int K) {
   return nb % L == 0 ? L * 16 + nb / L : 0;
 }
 
-// Scales are loaded by the dword: an odd count of them (K = 320 at group size 64 with an odd N) is not taken.
-bool gemm_takes(const uint32_t* w, const bf16* s, const bf16* b, int64_t N, int K, int gs, int M) {
-  if (M <= MAX_TOKENS || !mat_ok(w, s, b) || N * (K / gs) % 2 != 0 || N * K / 2 >= ((int64_t)1 << 31) || (int64_t)M * K * 6 >= ((int64_t)1 << 31))
-    return false;
+// Rows of a unit of the dense launch, 0 where it has no instance.
+static int gemm_rows(int K) {
   switch (gemm_shape(K)) {
-    case 16 * 16 + 5: case 32 * 16 + 6: case 64 * 16 + 5: case 64 * 16 + 4: case 2 * 16 + 5: return true;
-    default: return false;
+    case 16 * 16 + 5: return 128;
+    case 32 * 16 + 6: return 64;
+    case 64 * 16 + 5: case 64 * 16 + 4: return 32;
+    case 2 * 16 + 5: return 256;
+    default: return 0;
   }
+}
+
+// Scales are loaded by the dword: an odd count of them (K = 320 at group size 64 with an odd N) is not taken.  A grid has
+// less than 2^32 threads, the limb form less than 2^31 bytes.
+bool gemm_takes(const uint32_t* w, const bf16* s, const bf16* b, int64_t N, int K, int gs, int M) {
+  const int R = gemm_rows(K);
+  if (!R || M <= MAX_TOKENS || !mat_ok(w, s, b) || N * (K / gs) % 2 != 0 || (int64_t)M * K * 6 >= ((int64_t)1 << 31)) return false;
+  return ((N + R - 1) / R * ((M + 15) / 16) + 8) * GT_THREADS < ((int64_t)1 << 32);
 }
 
 // A launch takes the walk of one unit over K (23 us at K = 2560, 30 at 10240), whatever it holds, until the units

@@ -85,6 +85,27 @@ def test_gemm_extreme_blocks_bit_exact(ctx, K, gs):
     _check(ctx, wq, s, b, gs, xb)
 
 
+def test_gemm_past_two_gib_of_weights(ctx):
+    """A matrix of more than 2^31 bytes, bit-equal to a window of 8 and a token more, rows of both ends included."""
+    N, K, gs, M = 1677760 + 5, 2560, 64, 9
+    g = torch.Generator(device="cuda").manual_seed(7)
+    wq = torch.randint(-2 ** 31, 2 ** 31 - 1, (N, K // 8), generator=g, device="cuda", dtype=torch.int32)
+    s, b = ((torch.rand(N, K // gs, generator=g, device="cuda") * f).bfloat16() for f in (0.01, -0.08))
+    x = dev(rand_bf16(np.random.default_rng(3), (M, K)))
+    y, want = empty_bf16(M, N), empty_bf16(M, N)
+    print("case two GiB", N, K, flush=True)
+    ctx.profile(True)
+    ctx.profile_reset()
+    ctx.qmv(wq, s, b, gs, x, y)
+    launched = ctx.profile_stats()
+    ctx.profile(False)
+    ctx.qmv(wq, s, b, gs, x[:8], want[:8])
+    ctx.qmv(wq, s, b, gs, x[8:], want[8:])
+    ctx.synchronize()
+    assert "xlimb" in launched, launched
+    assert torch.equal(y.view(torch.int16), want.view(torch.int16))
+
+
 def test_gemm_two_byte_aligned_scales(ctx):
     """Scales and biases at an odd bf16 offset: the GEMV paths take the batch."""
     r = np.random.default_rng(2)
