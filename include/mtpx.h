@@ -95,7 +95,7 @@ int mtpx_q4_pack_sb(mtpx_ctx ctx, const uint16_t* scales, const uint16_t* biases
  * y[M, N] = x[M, K] . W[N, K]^T, M <= 4096, bf16 out (yf: optional f32 before
  * rounding); sb: packed scale/bias rows or NULL.  Every token's row is the
  * same whatever M (above 8 tokens: a prefill batch's GEMM on the matrix cores
- * where sb is given and the shape allows).  Replaces MLX quantizedMM's
+ * where the shape allows and enough tokens or rows make it faster).  Replaces MLX quantizedMM's
  * qmv_fast / qmv / qmv_wide (MLX/backend/metal/kernels/quantized.h:758,825,989)
  * and the track's TrackQuantWeight.apply / TrackLUTGemv
  * (Runner/FastModel/TrackFastWeights.swift:40-49, Runner/FastModel/TrackAffineLUT.swift:121-368). */
@@ -567,7 +567,9 @@ int mtpx_target_new_random(mtpx_ctx ctx, const mtpx_target_config* cfg, uint64_t
  * every q4 matrix and vector is used in place and must outlive the target.  layers [num_layers]
  * in the config's schedule (a GDN layer's MoE in attn.moe, the PLE layer's block in ple; attention
  * norms attn_norm/post_norm unused).  The library adds only: packed scale/bias rows when pack_sb != 0
- * and the caller gave none (else the kernels read the checkpoint's scales/biases), RoPE tables when
+ * and the caller gave none (else the kernels read the checkpoint's scales/biases), copies of scales or
+ * biases that start at an odd element (of matrices with packed rows: the batch GEMM reads them by the
+ * word), RoPE tables when
  * rope_cos/rope_sin are NULL (rows max_positions), and the n-gram table's head sizes and offsets,
  * which follow from the config (the table must hold at least their sum of rows -- a checkpoint pads it to
  * whole shards, and rows past the sum are never read; the multipliers are the

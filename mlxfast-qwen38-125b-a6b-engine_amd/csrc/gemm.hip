@@ -476,9 +476,8 @@ __global__ __launch_bounds__(GT_THREADS, MINW) void k_gemm(std::conditional_t<MO
 #endif
 }
 
-static bool al4(const void* p) { return ((uintptr_t)p & 3) == 0; }
 static bool mat_ok(const uint32_t* w, const bf16* s, const bf16* b) {
-  return w && s && b && ((uintptr_t)w & 15) == 0 && al4(s) && al4(b);
+  return w && s && b && ((uintptr_t)w & 15) == 0 && word_aligned(s) && word_aligned(b);
 }
 
 // ---- dense ----

@@ -1606,12 +1606,24 @@ int mtpx_qmv(mtpx_ctx h, const uint32_t* wq, const uint16_t* s, const uint16_t* 
   ARG(N >= 1 && M >= 1 && M <= QMV_MAX_TOKENS, "N=%d M=%d", N, M);
   ARG(gs_ok(gs) && k_ok(K, gs), "K=%d gs=%d unsupported", K, gs);
   if (set_device(c)) return MTPX_ERR_HIP;
-  const size_t xpn = (size_t)M * (K / 32) * XP_DW;
-  const bool batch = gemm_ok(wq, s, b, N, K, gs, M, false);
-  int rc = ws_reserve(c, (batch ? xl_ws(M, K) : al(xpn * 4)) + 256);
+  const size_t xpn = (size_t)M * (K / 32) * XP_DW, nsb = (size_t)N * (K / gs);
+  // The batch GEMM reads scales and biases by the word: arrays that start at an odd element are copied first (the rule
+  // is asked with a pointer that does not).
+  const bool odd = !word_aligned(s) || !word_aligned(b);
+  const uint16_t* any = reinterpret_cast<const uint16_t*>(wq);
+  const bool batch = gemm_ok(wq, odd ? any : s, odd ? any : b, N, K, gs, M, false);
+  int rc = ws_reserve(c, (batch ? xl_ws(M, K) : al(xpn * 4)) + (batch && odd ? 2 * al(2 * nsb) : 0) + 256);
   if (rc) return rc;
   ws_begin(c);
   uint32_t* xp = nullptr;
+  if (batch && odd) {
+    uint16_t* sc = ws_take<uint16_t>(c, nsb);
+    uint16_t* bc = ws_take<uint16_t>(c, nsb);
+    LAUNCH(c, "copy_sb", launch_copy_bf16(s, (int64_t)nsb, sc, c->stream));
+    LAUNCH(c, "copy_sb", launch_copy_bf16(b, (int64_t)nsb, bc, c->stream));
+    s = sc;
+    b = bc;
+  }
   if (!batch) {
     xp = ws_take<uint32_t>(c, xpn);
     LAUNCH(c, "xprep", launch_xprep(x, M, K, xp, c->stream));
@@ -2345,9 +2357,27 @@ struct Adopt {
       ok = false;
     *sb = static_cast<uint32_t*>(p);
   }
-  void q4(mtpx_q4* q, int64_t rows, int K, const char* what, bool optional = false) {
-    if (optional && !q->w) return;
-    if (need(q->w, what) & need(q->s, what) & need(q->b, what)) sb_rows(rows, K, q->s, q->b, &q->sb);
+  // A matrix that batches run over: the batch GEMM reads scales and biases by the word, so those that start at an odd
+  // element are copied (where the matrix has packed rows: without them nothing is added).
+  void words(int64_t rows, int K, const uint16_t** p, const uint32_t* sb) {
+    if (word_aligned(*p) || !sb) return;
+    const int64_t n = rows * (K / gs);
+    void* q = nullptr;
+    if (hipMalloc(&q, (size_t)n * 2) != hipSuccess) {
+      ok = false;
+      return;
+    }
+    allocs->push_back(q);
+    (void)hipGetLastError();  // only this launch's error counts
+    if (launch_copy_bf16(*p, n, static_cast<uint16_t*>(q), c->stream) != hipSuccess) ok = false;
+    *p = static_cast<uint16_t*>(q);
+  }
+  void q4(mtpx_q4* q, int64_t rows, int K, const char* what, bool batch = true) {
+    if (!(need(q->w, what) & need(q->s, what) & need(q->b, what))) return;
+    sb_rows(rows, K, q->s, q->b, &q->sb);
+    if (!batch) return;  // (the embedding, and what runs over windows only)
+    words(rows, K, &q->s, q->sb);
+    words(rows, K, &q->b, q->sb);
   }
   void moe(mtpx_moe_weights* m, const mtpx_layer_config& lc) {
     const int H = lc.hidden, E = lc.experts, F = lc.expert_width;
@@ -2366,17 +2396,19 @@ struct Adopt {
     const int nsb = !!m->gate_sb + !!m->up_sb + !!m->down_sb + !!m->sh_gate_sb + !!m->sh_up_sb + !!m->sh_down_sb;
     if (nsb != 0 && nsb != 6 && missing.empty()) missing = "moe packed scale/bias rows (all six or none)";
     struct {
-      const uint32_t* w; const uint16_t* s; const uint16_t* b; const uint32_t** sb; int64_t rows; int K;
-    } mats[6] = {{m->gate_w, m->gate_s, m->gate_b, &m->gate_sb, (int64_t)E * F, H},
-                 {m->up_w, m->up_s, m->up_b, &m->up_sb, (int64_t)E * F, H},
-                 {m->down_w, m->down_s, m->down_b, &m->down_sb, (int64_t)E * H, F},
-                 {m->sh_gate_w, m->sh_gate_s, m->sh_gate_b, &m->sh_gate_sb, F, H},
-                 {m->sh_up_w, m->sh_up_s, m->sh_up_b, &m->sh_up_sb, F, H},
-                 {m->sh_down_w, m->sh_down_s, m->sh_down_b, &m->sh_down_sb, H, F}};
+      const uint32_t* w; const uint16_t **s, **b; const uint32_t** sb; int64_t rows; int K;
+    } mats[6] = {{m->gate_w, &m->gate_s, &m->gate_b, &m->gate_sb, (int64_t)E * F, H},
+                 {m->up_w, &m->up_s, &m->up_b, &m->up_sb, (int64_t)E * F, H},
+                 {m->down_w, &m->down_s, &m->down_b, &m->down_sb, (int64_t)E * H, F},
+                 {m->sh_gate_w, &m->sh_gate_s, &m->sh_gate_b, &m->sh_gate_sb, F, H},
+                 {m->sh_up_w, &m->sh_up_s, &m->sh_up_b, &m->sh_up_sb, F, H},
+                 {m->sh_down_w, &m->sh_down_s, &m->sh_down_b, &m->sh_down_sb, H, F}};
     for (auto& x : mats)
-      if (need(x.w, "moe expert matrix") & need(x.s, "moe expert scales") & need(x.b, "moe expert biases") &&
-          nsb == 0)
-        sb_rows(x.rows, x.K, x.s, x.b, x.sb);
+      if (need(x.w, "moe expert matrix") & need(*x.s, "moe expert scales") & need(*x.b, "moe expert biases")) {
+        if (nsb == 0) sb_rows(x.rows, x.K, *x.s, *x.b, x.sb);
+        words(x.rows, x.K, x.s, *x.sb);
+        words(x.rows, x.K, x.b, *x.sb);
+      }
   }
   void hc(mtpx_hc_weights* m, int H, int hc_, int LW, bool inject) {
     const int W = hc_ * H;
@@ -2414,8 +2446,8 @@ int mtpx_target_adopt(mtpx_ctx h, const mtpx_target_config* cfg, const mtpx_targ
   t->embed = tw->embed;
   t->lm_head = tw->lm_head;
   t->final_hc = tw->final_hc;
-  ad.q4(&t->embed, cfg->vocab, H, "embed");
-  ad.q4(&t->lm_head, cfg->vocab, H, "lm_head");
+  ad.q4(&t->embed, cfg->vocab, H, "embed", false);
+  ad.q4(&t->lm_head, cfg->vocab, H, "lm_head", false);
   ad.hc(&t->final_hc, H, cfg->hc, cfg->lowrank, false);
   const mtpx_gdn_config gc = target_gdn_cfg(*cfg);
   const GdnGeom gg = gdn_geom(gc);
@@ -2440,8 +2472,8 @@ int mtpx_target_adopt(mtpx_ctx h, const mtpx_target_config* cfg, const mtpx_targ
       mtpx_q4 qkv{w.qkv_w, w.qkv_s, w.qkv_b, w.qkv_sb}, o{w.o_w, w.o_s, w.o_b, w.o_sb};
       la.q4(&qkv, L.attn->QW, H, "attention qkv");
       la.q4(&o, H, lc.heads * lc.head_dim, "attention o_proj");
-      w.qkv_sb = qkv.sb;
-      w.o_sb = o.sb;
+      w.qkv_s = qkv.s, w.qkv_b = qkv.b, w.qkv_sb = qkv.sb;
+      w.o_s = o.s, w.o_b = o.b, w.o_sb = o.sb;
       la.moe(&w.moe, lc);
       if ((!w.rope_cos || !w.rope_sin) && !rope_tables(c, &lc, &L.attn->allocs, &w.rope_cos, &w.rope_sin))
         la.ok = false;
@@ -2471,8 +2503,8 @@ int mtpx_target_adopt(mtpx_ctx h, const mtpx_target_config* cfg, const mtpx_targ
     mtpx_ple_weights& w = t->ple->w;
     Adopt la{c, cfg->ple.group_size, pack_sb != 0, &t->ple->allocs};
     const PleGeom pg = ple_geom(cfg->ple);
-    la.q4(&w.key_proj, pg.W, cfg->ple.embed_dim, "ple key_proj");
-    la.q4(&w.value_proj, H, cfg->ple.embed_dim, "ple value_proj");
+    la.q4(&w.key_proj, pg.W, cfg->ple.embed_dim, "ple key_proj", false);
+    la.q4(&w.value_proj, H, cfg->ple.embed_dim, "ple value_proj", false);
     la.need(w.norm_key, "ple norm_key");
     la.need(w.norm_query, "ple norm_query");
     la.need(w.norm_conv, "ple norm_conv");
@@ -2987,15 +3019,15 @@ int mtpx_head_adopt(mtpx_ctx h, const mtpx_head_config* cfg, const mtpx_head_wei
   mtpx_q4 qkv{lw.qkv_w, lw.qkv_s, lw.qkv_b, lw.qkv_sb}, o{lw.o_w, lw.o_s, lw.o_b, lw.o_sb};
   la.q4(&qkv, hd->layer->QW, H, "head qkv");
   la.q4(&o, H, lc.heads * lc.head_dim, "head o_proj");
-  lw.qkv_sb = qkv.sb;
-  lw.o_sb = o.sb;
+  lw.qkv_s = qkv.s, lw.qkv_b = qkv.b, lw.qkv_sb = qkv.sb;
+  lw.o_s = o.s, lw.o_b = o.b, lw.o_sb = o.sb;
   la.need(lw.q_norm, "head q_norm");
   la.need(lw.k_norm, "head k_norm");
   la.moe(&lw.moe, lc);
   if ((!lw.rope_cos || !lw.rope_sin) && !rope_tables(c, &lc, &hd->layer->allocs, &lw.rope_cos, &lw.rope_sin))
     la.ok = false;
   mtpx_head_weights& w = hd->w;
-  ad.q4(&w.embed, cfg->vocab, H, "head embed (the target's embed_tokens)");
+  ad.q4(&w.embed, cfg->vocab, H, "head embed (the target's embed_tokens)", false);
   ad.need(w.pre_norm_embedding, "pre_norm_embedding");
   ad.need(w.pre_norm_hidden, "pre_norm_hidden");
   ad.q4(&w.fc_embedding, H, H, "fc_embedding");
@@ -3003,7 +3035,7 @@ int mtpx_head_adopt(mtpx_ctx h, const mtpx_head_config* cfg, const mtpx_head_wei
   ad.hc(&w.attn_hc, H, cfg->hc, cfg->lowrank, true);
   ad.hc(&w.mlp_hc, H, cfg->hc, cfg->lowrank, true);
   ad.hc(&w.final_hc, H, cfg->hc, cfg->lowrank, false);
-  ad.q4(&w.shortlist, w.shortlist_rows, H, "shortlist rows");
+  ad.q4(&w.shortlist, w.shortlist_rows, H, "shortlist rows", false);
   ad.need(w.shortlist_ids, "shortlist ids");
   (void)W;
   rc = la.finish("head layer");

@@ -75,6 +75,7 @@ hipError_t launch_quantize(const bf16* w, int64_t rows, int K, int gs, uint32_t*
 hipError_t launch_randn_bf16(bf16* out, int64_t n, uint64_t seed, uint32_t tensor, float sigma,
                              hipStream_t st);
 hipError_t launch_fill_bf16(bf16* out, int64_t n, bf16 v, hipStream_t st);
+hipError_t launch_copy_bf16(const bf16* in, int64_t n, bf16* out, hipStream_t st);  // any alignment
 
 // --- scratch of the allocation-free MoE entry point (noalloc.hip)
 size_t moe_scratch_bytes();
@@ -171,6 +172,7 @@ __device__ __forceinline__ void xl_flag(uint8_t* big, size_t t, int who, int of,
 size_t xl_bytes(int M, int K);                // workspace of one batch
 XlBatch xl_carve(void* ws, int M, int K);     // its arrays in that workspace (256-byte aligned)
 hipError_t launch_xlimb(const bf16* x, int M, int K, const XlBatch& b, hipStream_t st);
+inline bool word_aligned(const void* p) { return ((uintptr_t)p & 3) == 0; }
 bool gemm_takes(const uint32_t* w, const bf16* s, const bf16* b, int64_t N, int K, int gs, int M);
 // Whether one launch over N rows in all is faster than the GEMV's windows on prepared blocks (xp_ready: they are there).
 bool gemm_faster(int64_t N, int K, int M, bool xp_ready);

@@ -655,6 +655,11 @@ __global__ void k_fill_bf16(bf16* __restrict__ out, int64_t n, bf16 v) {
   if (i < n) out[i] = v;
 }
 
+__global__ void k_copy_bf16(const bf16* __restrict__ in, int64_t n, bf16* __restrict__ out) {
+  const int64_t i = (int64_t)blockIdx.x * blockDim.x + threadIdx.x;
+  if (i < n) out[i] = in[i];
+}
+
 // Packed (scale, bias) pairs of a q4 matrix in the walker's lane order: one
 // thread per entry [row][q][it] = pair of the group of block q*r + L*it.
 __global__ void k_pack_sb(const bf16* __restrict__ s, const bf16* __restrict__ b, int64_t N, int K, int gs,
@@ -996,6 +1001,12 @@ hipError_t launch_randn_bf16(bf16* out, int64_t n, uint64_t seed, uint32_t tenso
 hipError_t launch_fill_bf16(bf16* out, int64_t n, bf16 v, hipStream_t st) {
   if (n == 0) return hipSuccess;
   hipLaunchKernelGGL(k_fill_bf16, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, out, n, v);
+  return hipGetLastError();
+}
+
+hipError_t launch_copy_bf16(const bf16* in, int64_t n, bf16* out, hipStream_t st) {
+  if (n == 0) return hipSuccess;
+  hipLaunchKernelGGL(k_copy_bf16, dim3((unsigned)((n + 255) / 256)), dim3(256), 0, st, in, n, out);
   return hipGetLastError();
 }
 

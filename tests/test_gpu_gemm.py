@@ -8,7 +8,7 @@ import torch
 
 pytestmark = pytest.mark.gpu
 
-from gpu_util import dev, empty_bf16, host, need_gpu, qweights, rand_bf16, write_device  # noqa: E402
+from gpu_util import dev, empty_bf16, host, need_gpu, qweights, rand_bf16, read_device, write_device  # noqa: E402
 from oracle import oracle as O  # noqa: E402
 
 
@@ -106,14 +106,70 @@ def test_gemm_past_two_gib_of_weights(ctx):
     assert torch.equal(y.view(torch.int16), want.view(torch.int16))
 
 
+def _odd(a):
+    """The bf16 bits a on the device, from an odd element on."""
+    p = torch.zeros(a.size + 1, dtype=torch.bfloat16, device="cuda")
+    p[1:] = dev(a).reshape(-1)
+    return p[1:].view(*a.shape)
+
+
 def test_gemm_two_byte_aligned_scales(ctx):
-    """Scales and biases at an odd bf16 offset: the GEMV paths take the batch."""
+    """Scales and biases at an odd bf16 offset, or one of them: copied for the call."""
     r = np.random.default_rng(2)
     wq, s, b = qweights(r, 48, 2560, 64)
-    pad = [torch.zeros(s.size + 1, dtype=torch.bfloat16, device="cuda") for _ in range(2)]
-    for p, a in zip(pad, (s, b)):
-        p[1:] = dev(a).reshape(-1)
-    _check(ctx, wq, s, b, 64, rand_bf16(r, (310, 2560)), *[p[1:].view(48, 40) for p in pad], gemm=False)
+    x = rand_bf16(r, (310, 2560))
+    _check(ctx, wq, s, b, 64, x, _odd(s), _odd(b))
+    _check(ctx, wq, s, b, 64, x, dev(s), _odd(b))
+    _check(ctx, wq, s, b, 64, x[:21], _odd(s), _odd(b), gemm=False)
+
+
+def test_adopted_two_byte_aligned_scales(ctx):
+    """A head adopted with every scale and bias array of its batch matrices at an odd bf16 offset takes the same launches as
+    one with aligned arrays, and gives the same bits."""
+    import mtpx
+    lc = mtpx.LayerConfig(2560, 24, 4, 640, 64, 24, 2, 256, 64, 128, 1e7, 1e-6, 256)
+    cfg = mtpx.HeadConfig(lc, 4, 320, 1000, 500, 980)
+    base = mtpx.MTPHead(ctx, cfg, seed=51)
+    w, keep = base.weights(), []
+
+    def odd(obj, prefix, rows, k):
+        for part in "sb":
+            a = read_device(getattr(obj, prefix + part), rows * (k // 64) * 2, np.uint16)
+            keep.append(_odd(a))
+            setattr(obj, prefix + part, keep[-1].data_ptr())
+
+    H, W, E, F = 2560, 4 * 2560, 24, 640
+    odd(w.layer, "qkv_", w.layer.qkv_rows, H)
+    odd(w.layer, "o_", H, 24 * 256)
+    for name, rows, k in (("gate_", E * F, H), ("up_", E * F, H), ("down_", E * H, F), ("sh_gate_", F, H),
+                          ("sh_up_", F, H), ("sh_down_", H, F)):
+        odd(w.layer.moe, name, rows, k)
+    for q, rows, k in ((w.fc_embedding, H, H), (w.fc_hidden, H, H)):
+        odd(q, "", rows, k)
+    for m in (w.attn_hc, w.mlp_hc, w.final_hc):
+        odd(m.down, "", 320, W)
+        odd(m.up, "", W, 320)
+        if m.inject.w:
+            odd(m.inject, "", 4, W)
+    head = mtpx.MTPHead.adopt(ctx, cfg, w)
+    n = 90
+    r = np.random.default_rng(n)
+    ids, multi = dev(r.integers(0, 1000, n).astype(np.int32)), dev(rand_bf16(r, (n, W)))
+    print("case adopted odd scales", flush=True)
+    got = []
+    for h in (base, head):
+        kv = mtpx.KVCache(ctx, 2, 256, 256)
+        out = empty_bf16(n, W)
+        ctx.profile(True)
+        ctx.profile_reset()
+        h.forward(kv, ids, multi, out)
+        got.append((host(out), {k: v[0] for k, v in ctx.profile_stats().items()}))
+        ctx.profile(False)
+        kv.close()
+    head.close()
+    base.close()
+    assert got[0][1] == got[1][1]
+    assert np.array_equal(got[0][0], got[1][0])
 
 
 @pytest.mark.parametrize("large", [False, True])
