@@ -526,17 +526,18 @@ bool gemm_takes(const uint32_t* w, const bf16* s, const bf16* b, int64_t N, int 
 // 27 / 28, 64: 33 / 30; 8 x 2560, 256: 22 / 24, 512: 36 / 27; 640 x 2560, 128: 20 / 25, 192: 27 / 26; 2560 x 2560, 48:
 // 19 / 24, 64: 25 / 24), with and without packed scale rows alike.  Above 5120 rows the GEMM (16480 x 2560, 9 tokens: 24).
 // K = 320: equal (10 us) where both prepare x; on blocks that are there the windows save a launch (10240 rows: 9
-// tokens 7 / 10, 24: 10 / 10).
-bool gemm_faster(int64_t N, int K, int M, bool xp_ready) {
+// tokens 7 / 10, 24: 10 / 10).  The windows of two matrices pay their tokens twice: half as many, and none at K = 2560
+// (a mixer's 64 + 4 rows: 9 tokens 18 + 16 / 21, 300 24 + 23 / 22).
+bool gemm_faster(int64_t N, int K, int M, bool xp_ready, int mats) {
   int tokens, product;
   switch (gemm_shape(K)) {
-    case 16 * 16 + 5: tokens = 300, product = 125000; break;
+    case 16 * 16 + 5: tokens = mats > 1 ? 0 : 300, product = 125000; break;
     case 32 * 16 + 6: tokens = 256, product = 41000; break;
     case 64 * 16 + 4: tokens = 128, product = 10200; break;
     case 64 * 16 + 5: tokens = 256, product = 26000; break;
     default: return !xp_ready || M * N >= 250000;
   }
-  return N > 5120 || M > tokens || M * N > product;
+  return N > 5120 || M * mats > tokens || M * N > product;
 }
 
 hipError_t launch_gemm_pair(const uint32_t* w1, const bf16* s1, const bf16* b1, int N1, bf16* y1, float* yf1,

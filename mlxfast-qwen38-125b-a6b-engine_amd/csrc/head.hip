@@ -233,10 +233,11 @@ static void hc_norm_mode(const dim3& grid, const bf16* residual, const bf16* out
 // elements whatever the number of rows, the second 0.18 ns per row, 256 elements and element a thread loads (10, 16 or
 // 48: the instance's), so the line is a number of rows.  us by row / by 256, 36 .. 1024 rows: 2560 wide 11.2 / 4.2 at 36,
 // 12.6 / 10.6 at 320, 13.4 / 14.0 at 512, 15.7 / 20.4 at 1024; 4096 wide 18.2 / 10.2 at 128, 18.9 / 27.5 at 512;
-// 10240 wide 29.0 / 14.5 at 64, 29.3 / 32.4 at 192.  The limb form by 256 elements is a launch more (4 us), so half the rows.
+// 10240 wide 29.0 / 14.5 at 64, 29.3 / 32.4 at 192.  The limb form by 256 elements is a launch more (4 us): half the
+// rows, and by row whatever their number up to 1536 wide (640 wide, 36 rows: 6.4 / 4.6 + 4).
 static bool norm_by_row(int64_t rows, int H, bool limbs) {
   const int few = H == 2560 ? 448 : H <= 256 * 16 ? 288 : 176;
-  return rows > (limbs ? few / 2 : few);
+  return limbs ? H <= 1536 || rows > few / 2 : rows > few;
 }
 
 hipError_t launch_hc_norm(const bf16* residual, const bf16* out, const bf16* inject, int S, int hc, int H,

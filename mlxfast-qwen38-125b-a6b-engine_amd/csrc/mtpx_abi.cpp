@@ -320,10 +320,11 @@ int moe_enqueue(Ctx* c, const mtpx_moe_weights* w, const uint16_t* x, int M, uin
       // The experts over their chunks on the matrix cores.  A chunk costs 16 tokens whatever it holds, so with few slots
       // per expert the walk of one slot per workgroup is faster.  Down: below 1.25 (launches by slots / by chunks and their
       // limb pass, us: 512 experts, hidden 1024, top-10, 64 tokens (1.25 slots) 46 / 55; hidden 2560, top-16, 24 (0.75) 68 /
-      // 88, 64 (2.0) 158 / 126; 64 experts top-8, 24 (3.0) 20 / 22, 64 (8.0) 38 / 22).  Gate|up: below 2.7 (whole prefill of
-      // four layers, 128 / 160 tokens of 512 experts top-10: 3515 / 3804 by chunks, 3487 / 3959 by slots; 75 tokens: 2900 /
+      // 88, 64 (2.0) 158 / 126; 64 experts, hidden 1024, top-8, 64 (8.0) 38 / 22), or below 200000 output elements in all (there
+      // 24 tokens, 221000: 20 / 22; 16 experts, hidden 640, top-4, nine, 29000: 10 / 16).  Gate|up: below 2.7 (whole prefill
+      // of four layers, 128 / 160 tokens of 512 experts top-10: 3515 / 3804 by chunks, 3487 / 3959 by slots; 75 tokens: 2900 /
       // 2650; 512: 7000 / 9700).
-      if (moe_gemm_down_ok(a) && T * a.K * 4 >= (size_t)a.E * 5) {
+      if (moe_gemm_down_ok(a) && T * a.K * 4 >= (size_t)a.E * 5 && slots * a.H >= 200000) {
         const XlBatch xs = xl_take(c, (int)slots, a.F);
         if (moe_gemm_gate_up_ok(a) && T * a.K * 3 >= (size_t)a.E * 8) {
           const XlBatch xt = xl_take(c, (int)T, a.H);
@@ -667,7 +668,7 @@ bool mix_batch_ok(const HcGeom& g, const mtpx_hc_weights* hw, int S) {
   const int W = g.hc * g.H;
   return gemm_takes(hw->down.w, hw->down.s, hw->down.b, g.LW, W, g.gs, S) &&
          (!hw->inject.w || gemm_takes(hw->inject.w, hw->inject.s, hw->inject.b, g.hc, W, g.gs, S)) &&
-         gemm_faster(g.LW + (hw->inject.w ? g.hc : 0), W, S, true);
+         gemm_faster(g.LW + (hw->inject.w ? g.hc : 0), W, S, true, hw->inject.w ? 2 : 1);
 }
 
 int hc_mix_enqueue(Ctx* c, const HcGeom& g, const mtpx_hc_weights* hw, const uint16_t* normed, const uint32_t* xpW,

@@ -174,8 +174,9 @@ XlBatch xl_carve(void* ws, int M, int K);     // its arrays in that workspace (2
 hipError_t launch_xlimb(const bf16* x, int M, int K, const XlBatch& b, hipStream_t st);
 inline bool word_aligned(const void* p) { return ((uintptr_t)p & 3) == 0; }
 bool gemm_takes(const uint32_t* w, const bf16* s, const bf16* b, int64_t N, int K, int gs, int M);
-// Whether one launch over N rows in all is faster than the GEMV's windows on prepared blocks (xp_ready: they are there).
-bool gemm_faster(int64_t N, int K, int M, bool xp_ready);
+// Whether one launch over the N rows of one or two matrices is faster than the GEMV's windows of each on prepared blocks
+// (xp_ready: they are there).
+bool gemm_faster(int64_t N, int K, int M, bool xp_ready, int mats = 1);
 inline bool gemm_ok(const uint32_t* w, const bf16* s, const bf16* b, int64_t N, int K, int gs, int M, bool xp_ready) {
   return gemm_takes(w, s, b, N, K, gs, M) && gemm_faster(N, K, M, xp_ready);
 }

@@ -62,12 +62,14 @@ def test_moe_batch_matches_windows(ctx, H, E, K, n, q4):
     head.close()
 
 
-# row blocks of 128 rows of H: whole ones and a last one of 32 rows; slots per expert on both sides of 1.25
-@pytest.mark.parametrize("H,E,K,n,gs,chunks", [(1024, 32, 4, 70, 64, 1), (544, 16, 3, 33, 32, 1), (512, 9, 9, 17, 64, 1),
-                                               (1024, 32, 4, 10, 32, 1), (1024, 32, 4, 9, 32, 0), (2560, 96, 6, 19, 64, 0)])
+# row blocks of 128 rows of H: whole ones and a last one of 32 rows; both sides of 1.25 slots per expert and of 200000
+# output elements in all
+@pytest.mark.parametrize("H,E,K,n,gs,chunks", [
+    (1024, 32, 4, 70, 64, 1), (544, 16, 3, 100, 32, 1), (512, 9, 9, 45, 64, 1), (1024, 256, 8, 40, 32, 1),
+    (1024, 256, 8, 39, 32, 0), (1024, 32, 4, 40, 64, 1), (1024, 32, 4, 39, 64, 0), (2560, 96, 6, 19, 64, 0)])
 def test_expert_down_chunks_at_other_hidden_sizes(ctx, H, E, K, n, gs, chunks):
-    """The expert down GEMM at expert width 640 takes any hidden size, from 1.25 slots per expert on (it reads the experts'
-    activations in limb form: its number of passes tells), bit-equal to windows of 8."""
+    """The expert down GEMM at expert width 640 takes any hidden size, where experts hold enough slots (it reads the
+    experts' activations in limb form: its number of passes tells), bit-equal to windows of 8."""
     import mtpx
     lc = mtpx.LayerConfig(H, E, K, 640, gs, 4, 2, 64, 16, 32, 1e7, 1e-6, 256)
     head = mtpx.MTPHead(ctx, mtpx.HeadConfig(lc, 4, 64, 1000, 500, 980), seed=41 + n)
