@@ -784,11 +784,12 @@ hipError_t launch_attn_batch(const bf16* q, int S, int HQ, int HK, const bf16* k
                              uint32_t* xp_gated, hipStream_t st) {
   if (!attn_batch_ok(S, HQ, HK, PP_D, T) || T < S) return hipErrorInvalidValue;
   const int R = S * (HQ / HK), TP = (T + 31) & ~31;
-  // tiles of 64 rows x 64 keys where those of 128 would not give each CU one (75 queries of 24 heads, 16 tiles
-  // of 128: 44 us with the large tile, 17 us with the small)
+  // tiles of 64 rows x 64 keys until those of 128 are three per CU (24 heads, us by 64 / by 128: 96 queries over 96 keys,
+  // 18 tiles of 128, 17 / 42; 96 over 1796, 270: 37 / 54; 160 over 1860, 450: 54 / 56; 256 over 1456, 576: 63 / 77; 256
+  // over 1956, 768: 80 / 79)
   const auto tiles = [&](int t) { return dim3((R + t - 1) / t, (T + t - 1) / t, HK); };
   const dim3 big = tiles(128);
-  if (big.x * big.y * big.z < 256)
+  if (big.x * big.y * big.z < 768)
     hipLaunchKernelGGL((k_attn_scores<64>), tiles(64), dim3(256), 0, st, q, S, HQ, HK, kc, tmax, T, scale, TP, scores);
   else
     hipLaunchKernelGGL((k_attn_scores<128>), big, dim3(256), 0, st, q, S, HQ, HK, kc, tmax, T, scale, TP, scores);

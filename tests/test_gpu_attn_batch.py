@@ -1,7 +1,8 @@
 """The attention of a prefill batch (head dim 256, more than a window of positions: scores in one launch,
 the chunks of 32 keys folded per row in another), bit-exact against the same positions in windows of 8:
 query counts around the least that takes it (96 at 24 heads), ragged row tiles, prefixes around a chunk's and
-a tile's edge, group sizes 1, 2, 8 and 12, the last keys that a cache of 2048 holds, and keys whose scores are
+a tile's edge, group sizes 1, 2, 8 and 12, both score tiles (64 wide, and 128 where those are 768 or more: 256
+queries of 24 heads over 2048 keys), the last keys that a cache of 2048 holds, and keys whose scores are
 infinite or NaN (such a chunk adds nothing to any query that sees it)."""
 import numpy as np
 import pytest
@@ -22,7 +23,8 @@ def ctx():
 
 @pytest.mark.parametrize("HQ,HK,pre,n,odd", [
     (24, 2, 0, 96, False), (24, 2, 31, 95, False), (24, 24, 33, 97, False), (12, 12, 127, 193, False),
-    (32, 4, 96, 73, False), (12, 1, 1792, 256, False), (24, 2, 1900, 148, False), (24, 2, 40, 101, True),
+    (32, 4, 96, 73, False), (12, 1, 1792, 256, False), (24, 2, 1663, 256, False), (24, 2, 1792, 256, False),
+    (24, 2, 1900, 148, False), (24, 2, 40, 101, True),
     (16, 8, 257, 200, True)])
 def test_attention_batch_matches_windows(ctx, HQ, HK, pre, n, odd):
     import mtpx
