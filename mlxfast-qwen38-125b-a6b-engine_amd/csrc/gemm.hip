@@ -26,7 +26,7 @@
 // waves per CU (128 registers), each with its next segments in flight (LDS-direct loads, the wait
 // counted so that the later ones stay in flight).  Measured against the i8 batch GEMM and the slot walk
 // it replaced, 512 tokens, group size 64: GDN in-projection 431 -> 190 us, K = 6144 projections 236 ->
-// 127 (before the split below), mixer down and inject 94 -> 43 (and their layout pass), mixer up 71 -> 22, expert gate|up 1000 ->
+// 127, mixer down and inject 94 -> 43 (and their layout pass), mixer up 71 -> 22, expert gate|up 1000 ->
 // 340 (HBM floor about 200), expert down 213 -> 160.  On the way (in-projection): segments through
 // registers 423 us, one segment ahead 313, a token's limbs in four 16-byte runs instead of one of 64
 // bytes 246, limb reads with bank conflicts 232, a register for every rotation of sx (spilled ones make

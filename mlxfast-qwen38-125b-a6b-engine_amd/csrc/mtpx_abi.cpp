@@ -2781,10 +2781,10 @@ int mtpx_target_prefill(mtpx_ctx h, mtpx_target th, mtpx_target_state sh, const 
 namespace {
 // One window of S <= MAX_TOKENS positions (verify), or a prefill batch of S positions: the same
 // kernels over all S tokens where every token's output is its own (GEMVs, norms, mixers,
-// attention -- each query sees the keys up to its own position --, the MoE as windows of
-// MAX_TOKENS), the recurrent cores (GDN, PLE) window by window of MAX_TOKENS with each window
-// committed before the next, and the logits of the last position only.  Every output equals that
-// of the windows of MAX_TOKENS verified and committed in turn.
+// attention -- each query sees the keys up to its own position --, the MoE in one expert order
+// where moe_batch_ok), the GDN recurrence over the batch, the PLE block window by window of MAX_TOKENS
+// with each committed before the next, and the mix and logits of the last position only.  Every output
+// equals that of the windows of MAX_TOKENS verified and committed in turn.
 int target_verify_enqueue(Ctx* c, Target* t, TargetState* s, const int32_t* ids, int S, uint16_t* logits,
                           uint16_t* multi, uint16_t* mixed, bool* launched, bool prefill) {
   const mtpx_target_config& g = t->cfg;
@@ -3127,7 +3127,7 @@ int mtpx_head_forward(mtpx_ctx h, mtpx_head hh, mtpx_kv kvh, const int32_t* ids,
   // MoE block
   if ((rc = hc_norm_enqueue(c, hg, &w.mlp_hc, st0, ao, j, S, 0, eps, st1, nrm, xpW, xlW))) return rc;
   if ((rc = hc_mix_enqueue(c, hg, &w.mlp_hc, nrm, xpW, xlW, S, x, j, xpH))) return rc;
-  if (S > MAX_TOKENS) {  // a batch of the drafter's backlog: the MoE as windows of MAX_TOKENS
+  if (S > MAX_TOKENS) {  // a batch of the drafter's backlog
     if ((rc = moe_enqueue_windows(c, &w.layer.moe, x, S, ao, xpH))) return rc;
   } else if ((rc = moe_enqueue(c, &w.layer.moe, x, S, ao, nullptr, nullptr, nullptr, nullptr, nullptr, xpH))) {
     return rc;

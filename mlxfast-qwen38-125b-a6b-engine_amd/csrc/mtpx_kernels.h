@@ -203,7 +203,7 @@ hipError_t launch_moe_down(const MoeArgs& a, hipStream_t st);
 // one workgroup per (slot, row block) in dispatch order (the slots of one expert side by side on
 // one XCD, so its weight rows are fetched from HBM once and served to the others by that L2)
 bool moe_dd_supported(int H, int F, int K);
-hipError_t launch_moe_sort(const MoeArgs& a, hipStream_t st);  // a.gorder from the windows' routes
+hipError_t launch_moe_sort(const MoeArgs& a, hipStream_t st);  // a.gorder and the chunks from a batch's routes
 hipError_t launch_moe_gate_up_dd(const MoeArgs& a, hipStream_t st);
 hipError_t launch_moe_down_dd(const MoeArgs& a, hipStream_t st);
 hipError_t launch_moe_combine(const MoeArgs& a, hipStream_t st);

@@ -172,13 +172,14 @@ def test_adopted_two_byte_aligned_scales(ctx):
     assert np.array_equal(got[0][0], got[1][0])
 
 
-@pytest.mark.parametrize("large", [False, True])
-@pytest.mark.parametrize("gs,n", [(64, 200), (32, 149)])
+@pytest.mark.parametrize("gs,n,large", [(64, 200, False), (64, 200, True), (32, 149, False), (32, 149, True),
+                                        (64, 1100, False)])
 def test_expert_chunks_match_windows(ctx, gs, n, large):
-    """A prompt whose experts run by chunks of 16 slots gives the verify windows' bits; large: the MoE's
-    input scaled so that its blocks and the experts' activations pass 4096."""
+    """A prompt whose experts run by chunks of 16 slots gives the verify windows' bits, and so does a window after it; large:
+    the MoE's input scaled so that its blocks and the experts' activations pass 4096; 1100: a batch of 1024 positions and
+    one of 76 behind it, every kernel of a long prompt at the model's widths."""
     import mtpx
-    lc = mtpx.LayerConfig(2560, 96, 6, 640, gs, 24, 2, 256, 64, 128, 1e7, 1e-6, 300)
+    lc = mtpx.LayerConfig(2560, 96, 6, 640, gs, 24, 2, 256, 64, 128, 1e7, 1e-6, n + 8)
     cfg = mtpx.TargetConfig(lc, 16, 48, 4, 2, 4, 4, 320, 4000)
     cfg.ple_layer = -1
     t = mtpx.Target(ctx, cfg, seed=77)
@@ -199,6 +200,10 @@ def test_expert_chunks_match_windows(ctx, gs, n, large):
         want.append(host(mw))
     assert np.array_equal(host(mt), np.concatenate(want))
     assert np.array_equal(host(lg), host(lw)[-1])
+    nxt, la, lb = dev(np.array([5, 6, 7, 8], np.int32)), empty_bf16(4, 4000), empty_bf16(4, 4000)
+    t.verify(a, nxt, la)
+    t.verify(b, nxt, lb)
+    assert np.array_equal(host(la), host(lb))
     a.close()
     b.close()
     t.close()

@@ -3,7 +3,7 @@ batch gives every position's multi stream and the last position's logits exactly
 committing it in windows of 8 does, and leaves the same state (the next verify is bit-equal).
 Against the oracle composition's windows at small dims (a prompt of two full windows and a tail,
 with the PLE block), against the GPU's own windowed verify path for a prompt of 600 positions
-(75 windows, the batched MoE launches) and of 1100 (two batches, 1024 + 76) and at full width (hidden 2560, 512
+(75 windows of the MoE in a launch) and of 1100 (two batches, 1024 + 76) and at full width (hidden 2560, 512
 experts, hyper-connections 4 x 2560, the full PLE table, 4 layers): 45 positions over a
 1024-position prefix, 600 positions, and a prompt after a
 partly committed verify window; and the MTP head over a batch of backlog positions (the drafter's
@@ -132,7 +132,7 @@ def test_prefill_matches_oracle_windows(ctx):
     t.close()
 
 
-def test_prefill_two_batches_matches_windows(ctx):
+def test_prefill_600_matches_windows(ctx):
     """600 positions: one batch, 75 full windows; then a prefill of 3 more positions
     (one short window) and a verify, each against the windowed path's state."""
     import mtpx
@@ -172,7 +172,8 @@ def test_prefill_two_batches_matches_windows(ctx):
 
 
 def test_prefill_past_one_batch_matches_windows(ctx, monkeypatch):
-    """1100 positions after 9: a batch of 1024 committed before one of 76 that attends to it, 128 windows routed in the first."""
+    """1100 positions after 9: a batch of 1024 committed before one of 76 that attends to it; the MoE (hidden 256) by windows, 128 of them
+    in the first batch's launch."""
     import mtpx
     from oracle.target_ref import download_target
     monkeypatch.setitem(LAYER, "max_positions", 1200)
